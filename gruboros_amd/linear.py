@@ -11,8 +11,8 @@ a bf16 copy next to its fp32 master:
   * the backward produces the weight gradient directly in fp32 (bf16 x bf16
     GEMM with fp32 output), so no cast of the gradient either.
 With fp32 activations and fp32 weights (the reference's own precision: an
-unchanged train.py, cfg1's single layer) every product runs on mg_gemm over
-three-limb bf16 splits, fp32-accurate on MFMA: F32Linear.
+unchanged train.py, cfg1's single layer) every product runs on mg_gemm_f32:
+three bf16 limbs per value, fp32-accurate on MFMA (F32Linear).
 
 Two products are computed to fp32 accuracy from bf16 hi/lo pairs (mg_gemm
 HILO: A_hi B_hi + A_lo B_hi + A_hi B_lo on MFMA): the hidden half of
@@ -242,21 +242,17 @@ def accurate_linear_f32(x, layer):
 class F32Linear(torch.autograd.Function):
     """y = x W^T (+ b) for fp32 x [N, K] and fp32 W [O, K] (reference nn.Linear in fp32:
     mingru/minGRU.py:40-41,45,71; minLM.py:17-23,75,138), all three products on MFMA to
-    fp32 accuracy: each fp32 operand is split into three bf16 limbs (h + m + l == x,
-    mg_split_limbs) and one plain bf16 product over the 6-fold reduction sums the six limb
-    products through 2^-16 (hh, mh, hm, mm, lh, hl; the dropped ones are below 2^-24).
-    Forward y = x W^T (+ b in the epilogue); backward dx = dy W (dy's limbs side by side,
-    W's stacked), dW = dy^T x (both stacked along the rows, so no transposes and no
-    padding), db = column sums of dy. The limbs are formed per call, so nothing cached can
-    go stale when W changes.
+    fp32 accuracy (mg_gemm_f32: three bf16 limbs per value, six limb products).
+    Forward y = x W^T + b; backward dx = dy W, dW = dy^T x, db = column sums of dy.
     (Two limbs, x = hi + lo to 2^-16, are not enough here: the reference's g(x) has a kink
     at 0, and at cfg1's size a 4e-6 product error moves ~10 hidden pre-activations across
     it, 8e-4 on dx and dW.)"""
 
     @staticmethod
     def forward(ctx, x, w, b):
-        y = gemm.linear_fwd(gemm.split_limbs(x, gemm.LIMBS_A, False), gemm.split_limbs(w.detach(), gemm.LIMBS_B, False),
-                            b.detach().contiguous() if b is not None else None, out_dtype=torch.float32)
+        (n, k), o = x.shape, w.shape[0]
+        y = gemm.gemm_f32(x, gemm.KCONTIG, w, gemm.KCONTIG, n, o, k,
+                          bias=b.detach().contiguous() if b is not None else None)
         ctx.save_for_backward(x, w)
         ctx.has_bias = b is not None
         return y
@@ -265,12 +261,12 @@ class F32Linear(torch.autograd.Function):
     def backward(ctx, dy):
         x, w = ctx.saved_tensors
         dy = dy.contiguous()
+        (n, k), o = x.shape, w.shape[0]
         dx = dw = db = None
         if ctx.needs_input_grad[0]:
-            dx = gemm.linear_dx(gemm.split_limbs(dy, gemm.LIMBS_A, False), gemm.split_limbs(w.detach(), gemm.LIMBS_B, True),
-                                out_dtype=torch.float32)
+            dx = gemm.gemm_f32(dy, gemm.KCONTIG, w, gemm.MNCONTIG, n, k, o)
         if ctx.needs_input_grad[1]:
-            dw = gemm.linear_dw(gemm.split_limbs(dy, gemm.LIMBS_A, True), gemm.split_limbs(x, gemm.LIMBS_B, True))
+            dw = gemm.gemm_f32(dy, gemm.MNCONTIG, x, gemm.MNCONTIG, o, k, n)
         if ctx.has_bias and ctx.needs_input_grad[2]:
             db = column_sum(dy)
         return dx, dw, db
@@ -315,8 +311,8 @@ class BF16Linear(torch.autograd.Function):
 
 
 def linear(x, layer):
-    """layer(x) in x's dtype: fp32 activations and weights on the GPU -> F32Linear (mg_gemm
-    hi/lo, fp32-accurate); other equal dtypes, or widths F32Linear does not take -> F.linear;
+    """layer(x) in x's dtype: fp32 activations and weights on the GPU -> F32Linear
+    (mg_gemm_f32, fp32-accurate); other equal dtypes, or widths F32Linear does not take -> F.linear;
     bf16 activations over fp32 masters -> BF16Linear over the cached bf16 weight; parameters
     in another dtype (a model cast to float16) -> the product in the parameters' dtype, the
     result back in x's."""

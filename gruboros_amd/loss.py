@@ -80,7 +80,7 @@ def logits_cross_entropy(embed, to_logits, labels):
     if embed.dtype == torch.bfloat16 and w.dtype == torch.float32:
         return LogitsCrossEntropy.apply(e2.contiguous(), w, bf16_copy(w), lab)
     if f32_linear_applies(e2, w):
-        logits = f32_linear(e2, w)  # the fp32 path: the logits product on mg_gemm over bf16 limbs
+        logits = f32_linear(e2, w)  # the fp32 path: the logits product on mg_gemm_f32
     else:
         logits = torch.nn.functional.linear(e2.to(w.dtype), w)  # (parameters cast to another dtype: product in it)
     return CrossEntropyFromLogits.apply(logits.float().contiguous(), lab)

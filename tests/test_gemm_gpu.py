@@ -702,3 +702,33 @@ def test_hilo_prefix_matches_the_two_products(M, N, K, hc):
     assert torch.equal(out, ref)
     exact = (x.double() @ w.double().t())[:, :hc]
     assert _rel(out[:, :hc], exact) <= 2 ** -8
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 4, 4), (37, 200, 64), (128, 128, 32), (132, 260, 36), (300, 136, 1000),
+                                   (1000, 520, 4096)])
+@pytest.mark.parametrize("a_layout,b_layout", [(0, 0), (0, 1), (1, 1), (1, 0)])
+def test_gemm_f32_edges_match_fp64(M, N, K, a_layout, b_layout):
+    """mg_gemm_f32 (three bf16 limbs split between memory and LDS) at the edges of its 128 x 128 x
+    32 tiles, whole (deterministic) and split along K, with a bias and accumulated, against float64.
+    Elementwise bound: fp32 accumulation's K 2^-24 sum |a b| (and the dropped limb products', below
+    2^-24 of it each), plus one rounding for the bias and one for the accumulation."""
+    from gruboros_amd.gemm import gemm_f32
+
+    if a_layout == 1:
+        M = (M + 3) // 4 * 4
+    g = torch.Generator().manual_seed(M + N + K)
+    A, B = torch.randn(M, K, generator=g), torch.randn(N, K, generator=g)
+    bias, old = torch.randn(N, generator=g), torch.randn(M, N, generator=g)
+    ref, mag = A.double() @ B.double().t(), A.double().abs() @ B.double().abs().t()
+    a = (A if a_layout == 0 else A.t().contiguous()).to(DEV)
+    b = (B if b_layout == 0 else B.t().contiguous()).to(DEV)
+    bound = (K + 8) * 2.0 ** -24 * mag
+    for det in (False, True):
+        y = gemm_f32(a, a_layout, b, b_layout, M, N, K, bias=bias.to(DEV), deterministic=det)
+        err = (y.double().cpu() - (ref + bias.double())).abs()
+        assert bool((err <= bound + 2.0 ** -23 * bias.double().abs()).all()), float(err.max())
+        z = gemm_f32(a, a_layout, b, b_layout, M, N, K, out=old.to(DEV), accumulate=True, deterministic=det)
+        err = (z.double().cpu() - (ref + old.double())).abs()
+        assert bool((err <= bound + 2.0 ** -23 * old.double().abs()).all()), float(err.max())
+        again = gemm_f32(a, a_layout, b, b_layout, M, N, K, out=old.to(DEV), accumulate=True, deterministic=det)
+        assert torch.equal(z, again)
