@@ -9,7 +9,7 @@ import os
 
 import torch  # noqa: F401  (loads the HIP runtime the library binds to)
 
-from .build import LIB_PATH
+from .build import LIB_PATH, NATIVE_PATH
 
 MG_F32 = 0
 MG_BF16 = 1
@@ -98,6 +98,7 @@ SIGNATURES = {
 }
 
 _LIB = None
+_NATIVE = None
 
 
 class MingruHipError(RuntimeError):
@@ -119,6 +120,20 @@ def lib():
             fn.argtypes = args
         _LIB = L
     return _LIB
+
+
+def native():
+    """The host-side extension (csrc/host/native.cpp: output allocation, checks and launches of
+    whole operations and block passes); raises if it has not been built."""
+    global _NATIVE
+    if _NATIVE is None:
+        lib()
+        if not os.path.exists(NATIVE_PATH):
+            raise MingruHipError(f"{NATIVE_PATH} is missing: build it with `python -m gruboros_amd.build`")
+        from . import _native
+        _native.set_error(MingruHipError)
+        _NATIVE = _native
+    return _NATIVE
 
 
 def check(rc: int, what: str = "") -> None:

@@ -27,18 +27,14 @@ gradients (measured on the fp64 restatement: 4-7% at the cfg3 row count
 against 0.5% with stochastic rounding). The gradients crossing block boundaries
 are the fp32 residual stream's, the fp32 minGRU output's, and the bf16
 FeedForward output's (stochastically rounded by the next block's norm).
+
+The launches of a block pass are issued by one call into csrc/host/native.cpp.
 """
 import torch
 
 from . import _lib
-from . import gemm
-from .linear import bf16_copy, bf16_pair, column_sum, gelu_backward, gelu_backward_bias_grads, grad_target
-from .norm import FP32_EPS  # noqa: F401  (the kernels' eps; norm._fwd passes it)
-from .norm import _bwd as _norm_bwd
-from .norm import _fwd as _norm_fwd
-from .scan import _launch_bwd as _scan_bwd
-from .scan import _launch_fwd as _scan_fwd
-from .scan import _launch_fwd_residual as _scan_fwd_res
+from .linear import bf16_copy, bf16_pair, grad_target
+from .scan import _workspace as _scan_workspace
 
 BF16 = torch.bfloat16
 
@@ -51,10 +47,6 @@ FF_DW_PAIR = True
 # (mg_scan_fwd_residual) and keeps h only as fp32 checkpoints for the backward;
 # False: the scan writes h and the FeedForward's norm adds it.
 SCAN_RESIDUAL = True
-
-# The FeedForward backward's GELU backward and both bias gradients in one launch
-# (mg_ff_bias_bwd); False: mg_gelu_bwd and mg_column_sum separately.
-FF_BIAS_BWD_FUSED = True
 
 # to_hidden_and_gate's forward as one launch (mg_gemm_hilo_prefix: the hidden
 # half's tiles hi/lo, the gate half's plain) instead of two.
@@ -82,95 +74,33 @@ class MinGRUBlock(torch.autograd.Function):
         B, T, D = x.shape
         N, Di = B * T, w_hg.shape[0] // 2
         ctx.w_hg, ctx.w_to = w_hg, w_to  # for their .grad (weight gradients added in place, grad_target)
+        _lib.require_cuda(x, pending, w_norm, w_hg, h0, w_to)
         x2 = x.reshape(N, D)
-        p2 = pending.reshape(N, D) if pending is not None else None
-        x_out, n, rstd, pair = _norm_fwd(x2, p2, w_norm, BF16, with_lo=True)
+        whp = bf16_pair(w_hg)
+        whb = bf16_copy(w_hg)
+        x_out, rstd, pair, hg, h, h_last, out, h_pair, ckpt = _lib.native().gru_forward(
+            x2, pending.reshape(N, D) if pending is not None else None, w_norm, whp, whb,
+            bf16_pair(w_to) if w_to is not None else None, h0, B, T, SCAN_RESIDUAL, HG_ONE_LAUNCH,
+            _scan_workspace(x.device, B, T, Di), _lib.stream_of(x))
         xn = x_out if x_out is not None else x2
-        whp, whb = bf16_pair(w_hg), bf16_copy(w_hg)
-        hg = torch.empty(N, 2 * Di, dtype=BF16, device=x.device)
-        if HG_ONE_LAUNCH and gemm.hilo_prefix_fits(pair, whp, D, Di):
-            gemm.linear_fwd_hilo_prefix(pair, whp, hg, D, Di)                   # minGRU.py:45, both halves
-        else:
-            gemm.linear_fwd_hilo(pair, whp[:Di], hg[:, :Di], D)                # minGRU.py:45, hidden half
-            gemm.gemm(n, gemm.KCONTIG, whb[Di:], gemm.KCONTIG, N, Di, D, hg[:, Di:])  # gate half
-        hg3 = hg.view(B, T, 2 * Di)
-        if w_to is None and SCAN_RESIDUAL:
-            # minGRU.py:47-69 and the residual add of minLM.py:125 in one pass; the
-            # backward rebuilds h from the fp32 checkpoints
-            x2, h_last, ckpt = _scan_fwd_res(hg3[..., :Di], hg3[..., Di:], h0, xn.view(B, T, D))
-            ctx.save_for_backward(xn, w_norm, rstd, pair, hg, None, h0, whb, ckpt)
-            ctx.dims = (B, T, D, Di)
-            ctx.has_pending, ctx.has_to, ctx.res = pending is not None, False, True
-            return x2, None, h_last
-        h, h_last, _ = _scan_fwd(hg3[..., :Di], hg3[..., Di:], h0, torch.float32)   # minGRU.py:47-69
-        saved = [xn, w_norm, rstd, pair, hg, h, h0, whb]
-        if w_to is not None:                                                   # minGRU.py:71
-            h_pair = gemm.split_hilo(h.view(N, Di))
-            out = torch.empty(N, D, dtype=torch.float32, device=x.device)
-            gemm.linear_fwd_hilo(h_pair, bf16_pair(w_to), out, Di)
-            out = out.view(B, T, D)
-            saved += [h_pair, bf16_copy(w_to)]
-        else:
-            out = h
-        ctx.save_for_backward(*saved)
+        ctx.save_for_backward(xn, w_norm, rstd, pair, hg, h, h0, whb, ckpt, h_pair,
+                              bf16_copy(w_to) if w_to is not None else None)
         ctx.dims = (B, T, D, Di)
-        ctx.has_pending, ctx.has_to, ctx.res = pending is not None, w_to is not None, False
+        ctx.has_pending = pending is not None
+        if ckpt is not None:  # expansion 1: x_next = x1 + h, h kept as checkpoints
+            return out, None, h_last
         x1 = x_out.view(B, T, D) if x_out is not None else x.view_as(x)
         return x1, out, h_last
 
     @staticmethod
     def backward(ctx, dx1, dout, dh_last):
         B, T, D, Di = ctx.dims
-        N = B * T
-        saved = ctx.saved_tensors
-        xn, w_norm, rstd, pair, hg, h, h0, whb = saved[:8]
-        ckpt = None
-        dev = xn.device
-        dW_to = None
-        if ctx.res:
-            # x_next = x1 + h: h and the residual get the same gradient
-            ckpt = saved[8]
-            dh = dx1
-        elif dout is None:
-            dh = None
-        elif ctx.has_to:
-            h_pair, wtb = saved[8:10]
-            dob = gemm.round_bf16_sr(dout.reshape(N, D).contiguous().float())
-            dh = gemm.linear_dx(dob, wtb, out_dtype=torch.float32).view(B, T, Di)
-            if ctx.needs_input_grad[5] and not (FF_DW_PAIR and ctx.needs_input_grad[3]):
-                g_to = grad_target(ctx.w_to)
-                if g_to is not None:
-                    gemm.linear_dw(dob, h_pair[:, :Di], out=g_to, accumulate=True)
-                else:
-                    dW_to = gemm.linear_dw(dob, h_pair[:, :Di])
-        else:
-            dh = dout.float()
-        dhg = torch.empty(N, 2 * Di, dtype=BF16, device=dev)
-        hg3, dhg3 = hg.view(B, T, 2 * Di), dhg.view(B, T, 2 * Di)
-        want_dh0 = h0 is not None and ctx.needs_input_grad[4]
-        if dh is None and dh_last is None:
-            dhg.zero_()
-            dh0 = torch.zeros_like(h0) if want_dh0 else None
-        else:
-            dh0 = _scan_bwd(hg3[..., :Di], hg3[..., Di:], h0, h, ckpt, dh, dh_last, dhg3[..., :Di], dhg3[..., Di:],
-                            want_dh0)
-        dn = gemm.linear_dx(dhg, whb, stochastic=True)             # bf16, stochastically rounded
-        dW_hg = None
-        if ctx.needs_input_grad[3]:
-            g_hg = grad_target(ctx.w_hg)
-            if ctx.has_to and dout is not None and ctx.needs_input_grad[5] and FF_DW_PAIR:
-                # to_out's and to_hidden_and_gate's weight gradients in one launch
-                g_to = grad_target(ctx.w_to)
-                if g_to is not None and g_hg is not None:
-                    gemm.linear_dw_pair(dob, h_pair[:, :Di], dhg, pair[:, :D], out0=g_to, out1=g_hg, accumulate=True)
-                else:
-                    dW_to, dW_hg = gemm.linear_dw_pair(dob, h_pair[:, :Di], dhg, pair[:, :D])
-            elif g_hg is not None:
-                gemm.linear_dw(dhg, pair[:, :D], out=g_hg, accumulate=True)
-            else:
-                dW_hg = gemm.linear_dw(dhg, pair[:, :D])
-        dres = dx1.reshape(N, D) if dx1 is not None else None
-        dx, dpend, dw_norm = _norm_bwd(xn, w_norm, rstd, dn, dres, True, BF16, ctx.has_pending)
+        xn, w_norm, rstd, pair, hg, h, h0, whb, ckpt, h_pair, wtb = ctx.saved_tensors
+        want_hg, want_to = ctx.needs_input_grad[3], ctx.needs_input_grad[5]
+        dx, dpend, dw_norm, dW_hg, dh0, dW_to = _lib.native().gru_backward(
+            xn, w_norm, rstd, pair, hg, h, h0, whb, ckpt, h_pair, wtb, dx1, dout, dh_last, B, T, ctx.has_pending, want_hg,
+            want_to, h0 is not None and ctx.needs_input_grad[4], FF_DW_PAIR, grad_target(ctx.w_hg) if want_hg else None,
+            grad_target(ctx.w_to) if want_to else None, _scan_workspace(xn.device, B, T, Di), _lib.stream_of(xn))
         return (dx.view(B, T, D), dpend.view(B, T, D) if dpend is not None else None,
                 dw_norm if ctx.needs_input_grad[2] else None, dW_hg,
                 dh0.reshape(h0.shape) if dh0 is not None else None, dW_to)
@@ -192,15 +122,13 @@ class FFBlock(torch.autograd.Function):
         B, T, D = x1.shape
         N = B * T
         ctx.w1, ctx.w2 = w1, w2  # for their .grad (weight gradients added in place, grad_target)
-        x2, n2, rstd, _ = _norm_fwd(x1.reshape(N, D), out.reshape(N, D) if out is not None else None, w_norm, BF16)
-        ctx.has_out = out is not None
-        if x2 is None:
-            x2 = x1.reshape(N, D)
+        _lib.require_cuda(x1, out, w_norm, w1, b1, w2, b2)
+        x1r = x1.reshape(N, D)
         w1b, w2b = bf16_copy(w1), bf16_copy(w2)
-        pre = torch.empty(N, w1.shape[0], dtype=BF16, device=x1.device)
-        act = gemm.linear_fwd(n2, w1b, _f32(b1), gelu_pre=pre)   # pre = n2 W1^T + b1, act = gelu(pre)
-        pend = gemm.linear_fwd(act, w2b, _f32(b2))                # act W2^T + b2
-        ctx.save_for_backward(x2, w_norm, rstd, n2, pre, act, w1b, w2b)
+        x2, n2, rstd, pre, act, pend = _lib.native().ff_forward(
+            x1r, out.reshape(N, D) if out is not None else None, w_norm, w1b, _f32(b1), w2b, _f32(b2), _lib.stream_of(x1))
+        ctx.has_out = out is not None
+        ctx.save_for_backward(x2 if x2 is not None else x1r, w_norm, rstd, n2, pre, act, w1b, w2b)
         ctx.dims = (B, T, D)
         return (x2.view(B, T, D) if ctx.has_out else x1), pend.view(B, T, D)
 
@@ -209,37 +137,19 @@ class FFBlock(torch.autograd.Function):
         B, T, D = ctx.dims
         N = B * T
         x2, w_norm, rstd, n2, pre, act, w1b, w2b = ctx.saved_tensors
-        dres = dx2.reshape(N, D) if dx2 is not None else None
+        nat, stream = _lib.native(), _lib.stream_of(x2)
         dW1 = db1 = dW2 = db2 = None
         if dpend is None:
-            dn2 = torch.zeros(N, D, dtype=torch.float32, device=x2.device)
+            dres = dx2.reshape(N, D) if dx2 is not None else None
+            dx1, _, dw_norm = nat.norm_bwd(x2, w_norm, rstd, None, dres, True, -1, None, stream)
         else:
             dp = dpend.reshape(N, D)
             if dp.dtype != BF16 or not dp.is_contiguous():
                 dp = dp.to(BF16).contiguous()
-            dact = gemm.linear_dx(dp, w2b, stochastic=True)            # bf16, stochastically rounded
-            if FF_BIAS_BWD_FUSED:
-                dpre, db1, db2 = gelu_backward_bias_grads(dact, pre, dp)  # dpre bf16, stochastically rounded
-            else:
-                (dpre, db1), db2 = gelu_backward(dact, pre), column_sum(dp)
-            dn2 = gemm.linear_dx(dpre, w1b, stochastic=True)           # bf16, stochastically rounded
-            g1, g2 = grad_target(ctx.w1), grad_target(ctx.w2)
-            if FF_DW_PAIR and g1 is not None and g2 is not None:
-                gemm.linear_dw_pair(dp, act, dpre, n2, out0=g2, out1=g1, accumulate=True)  # into .grad
-            elif FF_DW_PAIR:
-                dW2, dW1 = gemm.linear_dw_pair(dp, act, dpre, n2)     # one launch for both weight gradients
-            else:
-                if g2 is not None:
-                    gemm.linear_dw(dp, act, out=g2, accumulate=True)
-                else:
-                    dW2 = gemm.linear_dw(dp, act)
-                if g1 is not None:
-                    gemm.linear_dw(dpre, n2, out=g1, accumulate=True)
-                else:
-                    dW1 = gemm.linear_dw(dpre, n2)
+            dx1, dw_norm, dW1, db1, dW2, db2 = nat.ff_backward(x2, w_norm, rstd, n2, pre, act, w1b, w2b, dx2, dp, FF_DW_PAIR,
+                                                               grad_target(ctx.w1), grad_target(ctx.w2), stream)
         # x2 = x1 + out: both inputs get the same gradient, written once and returned for both
         # (the consumer, MinGRUBlock.backward, only reads them)
-        dx1, _, dw_norm = _norm_bwd(x2, w_norm, rstd, dn2, dres, True, torch.float32, False)
         return dx1.view(B, T, D), (dx1.view(B, T, D) if ctx.has_out else None), dw_norm, dW1, db1, dW2, db2
 
 
@@ -252,33 +162,24 @@ class FinalNormCE(torch.autograd.Function):
     def forward(ctx, x, pending, w_norm, w_out, labels):
         B, T, D = x.shape
         N = B * T
-        V = w_out.shape[0]
+        _lib.require_cuda(x, pending, w_norm, w_out, labels)
         x2 = x.reshape(N, D)
-        x_out, embed, rstd, _ = _norm_fwd(x2, pending.reshape(N, D) if pending is not None else None, w_norm, BF16)
-        xn = x_out if x_out is not None else x2
         wob = bf16_copy(w_out)
-        L = _lib.lib()
-        dl = torch.empty(N, V, dtype=BF16, device=x.device)
-        part = torch.empty(L.mg_logits_cross_entropy_partials(N), dtype=torch.float32, device=x.device)
-        lab = labels.reshape(-1).contiguous()
-        _lib.check(L.mg_logits_cross_entropy(_lib.ptr(embed), embed.stride(0), _lib.ptr(wob), wob.stride(0),
-                                             _lib.ptr(lab), _lib.ptr(dl), V, _lib.ptr(part), None, N, D, V, 1.0 / N,
-                                             _lib.stream_of(embed)), "mg_logits_cross_entropy")
-        ctx.save_for_backward(xn, w_norm, rstd, embed, dl, wob)
+        loss, x_out, embed, rstd, dl = _lib.native().head_forward(
+            x2, pending.reshape(N, D) if pending is not None else None, w_norm, wob, labels.reshape(-1).contiguous(),
+            _lib.stream_of(x))
+        ctx.save_for_backward(x_out if x_out is not None else x2, w_norm, rstd, embed, dl, wob)
         ctx.dims = (B, T, D)
         ctx.has_pending = pending is not None
-        return part.sum() / N
+        return loss
 
     @staticmethod
     def backward(ctx, g):
         B, T, D = ctx.dims
         xn, w_norm, rstd, embed, dl, wob = ctx.saved_tensors
-        de = gemm.linear_dx(dl, wob, out_dtype=torch.float32)         # fp32, unscaled
-        dW = gemm.linear_dw(dl, embed) if ctx.needs_input_grad[3] else None
-        if dW is not None:
-            dW.mul_(g)  # upstream scale (1 / grad_accum in the reference loop), in fp32; no host sync
-        # de's scale by g is the norm backward's, as it loads de (the same fp32 products)
-        dx, dpend, dw_norm = _norm_bwd(xn, w_norm, rstd, de, None, True, BF16, ctx.has_pending, dy_scale=g)
+        # the logits gradient's product stays unscaled: the norm backward applies g as it loads it
+        dx, dpend, dw_norm, dW = _lib.native().head_backward(xn, w_norm, rstd, embed, dl, wob, g, ctx.has_pending,
+                                                             ctx.needs_input_grad[3], _lib.stream_of(xn))
         return (dx.view(B, T, D), dpend.view(B, T, D) if dpend is not None else None,
                 dw_norm if ctx.needs_input_grad[2] else None, dW, None)
 

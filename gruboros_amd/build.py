@@ -1,4 +1,5 @@
-"""Build libmingru_hip.so (all HIP kernels + the C ABI) for gfx950 with hipcc.
+"""Build libmingru_hip.so (all HIP kernels + the C ABI) for gfx950 with hipcc, and
+_native.so (the host side of the training path on torch tensors) with g++.
 
 The library is written next to this file so that it travels with the source
 tree; it links the HIP runtime by SONAME only, so inside a process that has
@@ -16,6 +17,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 LIB_NAME = "libmingru_hip.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
+NATIVE_PATH = os.path.join(HERE, "_native.so")
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
@@ -69,15 +71,48 @@ def _spilled_kernels(remarks):
     return bad
 
 
+def _native_cmds(objdir):
+    """(compile, link) commands of _native.so: torch's C++ API and the C ABI only, no GPU code."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    obj = os.path.join(objdir, "native.o")
+    inc = [a for d in [*cpp_extension.include_paths(), sysconfig.get_paths()["include"]] for a in ("-isystem", d)]
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        raise RuntimeError("g++ not found")
+    compile_cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-Wall", "-DTORCH_EXTENSION_NAME=_native",
+                   f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I", os.path.join(ROOT, "include"),
+                   *inc, "-c", os.path.join(HERE, "csrc", "host", "native.cpp"), "-o", obj]
+    link_cmd = [cxx, "-shared", obj, "-L", HERE, "-lmingru_hip", "-L", lib, "-ltorch", "-ltorch_cpu", "-lc10",
+                "-ltorch_python", "-Wl,-rpath,$ORIGIN"]
+    return compile_cmd, link_cmd
+
+
+def _link(cmd, path, verbose):
+    fd, tmp = tempfile.mkstemp(prefix=os.path.basename(path) + ".tmp", dir=HERE)
+    os.close(fd)
+    rc, out = _run([*cmd, "-o", tmp], verbose)
+    if rc != 0:
+        os.unlink(tmp)
+        raise RuntimeError(f"linking {os.path.basename(path)} failed ({rc}):\n{out}")
+    os.replace(tmp, path)
+
+
 def build(verbose: bool = False) -> str:
     """Compile every csrc/*.hip (one hipcc process per file, in parallel) and link them into one
-    shared library; returns its path."""
+    shared library, then link _native.so against it; returns the library's path."""
     srcs = sources()
     inc = ["-I", os.path.join(ROOT, "include"), "-I", os.path.join(HERE, "csrc")]
     with tempfile.TemporaryDirectory(prefix="mg_build_") as objdir:
         objs = [os.path.join(objdir, os.path.basename(s) + ".o") for s in srcs]
-        jobs = max(1, min(len(srcs), os.cpu_count() or 1, 16))
+        jobs = max(1, min(len(srcs) + 1, os.cpu_count() or 1, 16))
+        native_compile, native_link = _native_cmds(objdir)
         with ThreadPoolExecutor(jobs) as pool:
+            native_done = pool.submit(_run, native_compile, verbose)
             def compile_one(so):
                 extra = ["-Rpass-analysis=kernel-resource-usage"] if os.path.basename(so[0]) == "gemm.hip" else []
                 return _run([hipcc(), *HIPCC_FLAGS, *extra, *inc, "-c", so[0], "-o", so[1]], verbose and not extra)
@@ -93,13 +128,11 @@ def build(verbose: bool = False) -> str:
                                        "be trustworthy): " + ", ".join(f"{k} ({n})" for k, n in bad))
             elif verbose and out.strip():
                 print(out, flush=True)
-        fd, tmp = tempfile.mkstemp(prefix=LIB_NAME + ".tmp", dir=HERE)
-        os.close(fd)
-        rc, out = _run([hipcc(), "--offload-arch=gfx950", "-fPIC", "-shared", *objs, "-o", tmp], verbose)
+        rc, out = native_done.result()
         if rc != 0:
-            os.unlink(tmp)
-            raise RuntimeError(f"hipcc link failed ({rc}):\n{out}")
-    os.replace(tmp, LIB_PATH)
+            raise RuntimeError(f"g++ failed on native.cpp ({rc}):\n{out}")
+        _link([hipcc(), "--offload-arch=gfx950", "-fPIC", "-shared", *objs], LIB_PATH, verbose)
+        _link(native_link, NATIVE_PATH, verbose)
     return LIB_PATH
 
 

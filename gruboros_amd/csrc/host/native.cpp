@@ -1,0 +1,522 @@
+// The host side of the training path: output allocation, argument checks and
+// launches of libmingru_hip's entry points on torch tensors, one Python call
+// per operation or per block pass.
+//
+// Why: a block of the bf16 training path issues 9 to 16 launches forward and
+// backward. Issued one by one from Python (ctypes call, torch.empty, stride
+// and pointer reads, about 9 us each) they took 180 to 340 us of host time,
+// more than the GPU time of every block up to about 2000 rows and half of a
+// training step's; from here a launch costs 2 to 3 us. The maths stays in the
+// kernels and autograd stays in Python (blocks.py, linear.py, norm.py,
+// scan.py): these functions are the bodies of its Functions.
+//
+// Every function takes the handle of the current HIP stream and launches on
+// it; outputs and workspaces come from torch's caching allocator, so nothing
+// outlives a call here. The GIL is released while a call runs.
+
+#include <torch/extension.h>
+
+#include <optional>
+#include <stdexcept>
+#include <string>
+#include <tuple>
+#include <vector>
+
+#include "mingru_hip.h"
+
+namespace {
+
+using at::Tensor;
+typedef std::optional<Tensor> Opt;
+
+struct MgError : std::runtime_error {
+  using std::runtime_error::runtime_error;
+};
+py::object* g_error = nullptr;  // gruboros_amd._lib.MingruHipError
+
+[[noreturn]] void fail(const std::string& m) { throw MgError(m); }
+void check(int rc, const char* what) {
+  if (rc) fail(std::string(what) + " failed (code " + std::to_string(rc) + "): " + mg_last_error());
+}
+
+constexpr float kEps = 1.1920928955078125e-07f;  // torch.finfo(float32).eps, nn.RMSNorm's for fp32
+
+int code(const Tensor& t) {
+  if (t.scalar_type() == at::kFloat) return MG_F32;
+  if (t.scalar_type() == at::kBFloat16) return MG_BF16;
+  fail(std::string("unsupported dtype ") + c10::toString(t.scalar_type()) +
+       ": the MI355X kernels take float32 and bfloat16 (cast a float16 model with .to(torch.bfloat16) instead)");
+}
+void need_cuda(const Tensor& t) {
+  if (!t.is_cuda())
+    fail("libmingru_hip kernels run on the GPU only; got a tensor on " + t.device().str() +
+         ". There is no CPU path in the product; the CPU restatement of the reference lives in oracle/ for tests.");
+}
+Tensor make(at::IntArrayRef size, at::ScalarType type, const Tensor& like) {
+  return at::empty(size, like.options().dtype(type).requires_grad(false));
+}
+Tensor bytes(size_t n, const Tensor& like) { return make({static_cast<int64_t>(n)}, at::kByte, like); }
+void* ptr(const Tensor& t) { return t.data_ptr(); }
+void* ptr(const Opt& t) { return t ? t->data_ptr() : nullptr; }
+float* fp(const Tensor& t) { return static_cast<float*>(t.data_ptr()); }
+float* fp(const Opt& t) { return t ? static_cast<float*>(t->data_ptr()) : nullptr; }
+int16_t* h16(const Tensor& t) { return static_cast<int16_t*>(t.data_ptr()); }
+void* st(int64_t stream) { return reinterpret_cast<void*>(stream); }
+bool deterministic() { return at::globalContext().deterministicAlgorithms(); }
+
+int64_t row_stride(const Tensor& t, const char* name) {
+  if (t.dim() != 2 || t.stride(1) != 1) {
+    std::string s = std::string(name) + ": expected a 2-D tensor with unit inner stride, got shape ";
+    for (int64_t i = 0; i < t.dim(); ++i) s += std::to_string(t.size(i)) + (i + 1 < t.dim() ? "x" : "");
+    fail(s);
+  }
+  return t.stride(0);
+}
+
+// Rows per launch of a row-parallel product over n rows whose operands take
+// `row_bytes` per row at most: each operand then spans under 2 GiB, mg_gemm's
+// buffer range with 256 rows of slack; a multiple of 256.
+int64_t row_step(int64_t n, int64_t row_bytes) {
+  int64_t r = ((int64_t(1) << 31) - 1) / std::max<int64_t>(row_bytes, 1) - 257;
+  r = std::max<int64_t>(256, r / 256 * 256);
+  return n <= r ? n : r;
+}
+
+// A 2-D bf16 operand or output as the entry points take it.
+struct Mat {
+  void* p;
+  int64_t ld;
+  int64_t esize;
+  Mat rows(int64_t r0) const { return {static_cast<char*>(p) + r0 * ld * esize, ld, esize}; }
+  Mat cols(int64_t c0) const { return {static_cast<char*>(p) + c0 * esize, ld, esize}; }
+};
+Mat mat(const Tensor& t, const char* name) { return {t.data_ptr(), row_stride(t, name), int64_t(t.element_size())}; }
+
+// ------------------------------------------------------------------ products
+
+void gemm(int al, Mat a, int bl, Mat b, int64_t M, int64_t N, int64_t K, int epi, const float* bias, void* aux,
+          int64_t ldaux, int c_dtype, Mat c, int flags, const Tensor& like, int64_t stream) {
+  if (deterministic()) flags |= MG_GEMM_DETERMINISTIC;
+  const size_t wsb = mg_gemm_workspace_bytes(al, bl, M, N, K, epi, c_dtype, flags);
+  Tensor ws;
+  if (wsb) ws = bytes(wsb, like);
+  check(mg_gemm(al, a.p, a.ld, bl, b.p, b.ld, M, N, K, epi, bias, aux, ldaux, c_dtype, c.p, c.ld, flags,
+                wsb ? ptr(ws) : nullptr, wsb, st(stream)),
+        "mg_gemm");
+}
+
+// x w^T (+ bias, + GELU with the pre-activation kept) [N, O], bf16; x [N, K], w [O, K]
+Tensor linear_fwd(const Tensor& x, const Tensor& w, const float* bias, const Tensor* pre, int64_t stream) {
+  const int64_t n = x.size(0), k = x.size(1), o = w.size(0);
+  Tensor y = make({n, o}, at::kBFloat16, x);
+  const Mat xm = mat(x, "x"), wm = mat(w, "w"), ym = mat(y, "y");
+  const int epi = pre ? MG_EPI_BIAS_GELU : bias ? MG_EPI_BIAS : MG_EPI_NONE;
+  const int64_t step = row_step(n, 2 * std::max(xm.ld, o));
+  for (int64_t r = 0; r < n; r += step)
+    gemm(MG_KCONTIG, xm.rows(r), MG_KCONTIG, wm, std::min(n - r, step), o, k, epi, bias, pre ? h16(*pre) + r * o : nullptr,
+         pre ? o : 0, MG_BF16, ym.rows(r), 0, x, stream);
+  return y;
+}
+
+// out[N, O] = x w^T to fp32 accuracy from hi/lo pairs x [N, 2K], w [O, 2K]
+void linear_fwd_hilo(Mat x, Mat w, int64_t n, int64_t o, int64_t k, int c_dtype, Mat out, const Tensor& like,
+                     int64_t stream) {
+  const int64_t step = row_step(n, std::max(2 * x.ld, out.ld * out.esize));
+  for (int64_t r = 0; r < n; r += step)
+    gemm(MG_KCONTIG, x.rows(r), MG_KCONTIG, w, std::min(n - r, step), o, k, MG_EPI_NONE, nullptr, nullptr, 0, c_dtype,
+         out.rows(r), MG_GEMM_HILO, like, stream);
+}
+
+// dy w [N, K] for dy [N, O] bf16, w [O, K] bf16: bf16 rounded stochastically, or fp32
+Tensor linear_dx(const Tensor& dy, const Tensor& w, bool f32, int64_t stream) {
+  const int64_t n = dy.size(0), o = dy.size(1), k = w.size(1);
+  Tensor dx = make({n, k}, f32 ? at::kFloat : at::kBFloat16, dy);
+  const Mat dm = mat(dy, "dy"), wm = mat(w, "w"), xm = mat(dx, "dx");
+  const int64_t step = row_step(n, std::max(2 * dm.ld, k * xm.esize));
+  for (int64_t r = 0; r < n; r += step)
+    gemm(MG_KCONTIG, dm.rows(r), MG_MNCONTIG, wm, std::min(n - r, step), k, o, MG_EPI_NONE, nullptr, nullptr, 0,
+         f32 ? MG_F32 : MG_BF16, xm.rows(r), f32 ? 0 : MG_GEMM_STOCHASTIC, dy, stream);
+  return dx;
+}
+
+// dy^T x [M, N] fp32 for dy [rows, M], x [rows, N] bf16: a new tensor, or added into `into`
+Tensor linear_dw(Mat dy, Mat x, int64_t n, int64_t m, int64_t k, const Opt& into, const Tensor& like, int64_t stream) {
+  Tensor out = into ? *into : make({m, k}, at::kFloat, like);
+  const Mat om = mat(out, "dW");
+  const int64_t step = row_step(n, 2 * std::max(dy.ld, x.ld));
+  for (int64_t r = 0; r < n; r += step)
+    gemm(MG_MNCONTIG, dy.rows(r), MG_MNCONTIG, x.rows(r), m, k, std::min(n - r, step), MG_EPI_NONE, nullptr, nullptr, 0,
+         MG_F32, om, into || r ? MG_GEMM_ACCUMULATE : 0, like, stream);
+  return out;
+}
+
+// Two weight gradients over the same rows in one launch (mg_gemm_wgrad_pair), each
+// a new tensor or (both) added into into0 and into1; over 2 GiB one at a time.
+std::pair<Tensor, Tensor> linear_dw_pair(Mat dy0, Mat x0, int64_t m0, int64_t k0, Mat dy1, Mat x1, int64_t m1, int64_t k1,
+                                         int64_t n, const Opt& into0, const Opt& into1, const Tensor& like,
+                                         int64_t stream) {
+  const bool acc = into0 && into1;
+  if (row_step(n, 2 * std::max(std::max(dy0.ld, x0.ld), std::max(dy1.ld, x1.ld))) < n)
+    return {linear_dw(dy0, x0, n, m0, k0, acc ? into0 : Opt(), like, stream),
+            linear_dw(dy1, x1, n, m1, k1, acc ? into1 : Opt(), like, stream)};
+  Tensor o0 = acc ? *into0 : make({m0, k0}, at::kFloat, like), o1 = acc ? *into1 : make({m1, k1}, at::kFloat, like);
+  const int flags = (acc ? MG_GEMM_ACCUMULATE : 0) | (deterministic() ? MG_GEMM_DETERMINISTIC : 0);
+  const size_t wsb = mg_gemm_wgrad_pair_workspace_bytes(m0, k0, m1, k1, n, flags);
+  Tensor ws;
+  if (wsb) ws = bytes(wsb, like);
+  check(mg_gemm_wgrad_pair(dy0.p, dy0.ld, x0.p, x0.ld, m0, k0, fp(o0), o0.stride(0), dy1.p, dy1.ld, x1.p, x1.ld, m1, k1,
+                           fp(o1), o1.stride(0), n, flags, wsb ? ptr(ws) : nullptr, wsb, st(stream)),
+        "mg_gemm_wgrad_pair");
+  return {o0, o1};
+}
+
+// sum_k A(m, k) B(k, n) (+ bias) in fp32 (mg_gemm_f32), into `out` or a new tensor
+Tensor gemm_f32(const Tensor& a, int al, const Tensor& b, int bl, int64_t M, int64_t N, int64_t K, const Opt& out_,
+                const Opt& bias, int flags, int64_t stream) {
+  need_cuda(a);
+  need_cuda(b);
+  if (a.scalar_type() != at::kFloat || b.scalar_type() != at::kFloat) fail("mg_gemm_f32 operands must be float32");
+  Tensor out = out_ ? *out_ : make({M, N}, at::kFloat, a);
+  const Mat am = mat(a, "A"), bm = mat(b, "B"), om = mat(out, "C");
+  const size_t wsb = mg_gemm_f32_workspace_bytes(M, N, K, flags);
+  Tensor ws;
+  if (wsb) ws = bytes(wsb, a);
+  check(mg_gemm_f32(al, static_cast<float*>(am.p), am.ld, bl, static_cast<float*>(bm.p), bm.ld, M, N, K, fp(bias),
+                    static_cast<float*>(om.p), om.ld, flags, wsb ? ptr(ws) : nullptr, wsb, st(stream)),
+        "mg_gemm_f32");
+  return out;
+}
+
+// ------------------------------------------------------------------ norm
+
+typedef std::tuple<Opt, Tensor, Tensor, Opt> NormOut;
+
+// (x + delta or none, y, rstd, pair or none) of rows x [..., D]; with_lo: y is the first half of pair
+NormOut norm_fwd(const Tensor& x, const Opt& delta, const Tensor& w, bool bf16, bool with_lo, int64_t stream) {
+  const int64_t D = x.size(-1), N = x.numel() / std::max<int64_t>(D, 1);
+  Opt pair, x_out;
+  Tensor y;
+  if (with_lo) {
+    std::vector<int64_t> s = x.sizes().vec();
+    s.back() = 2 * D;
+    pair = make(s, at::kBFloat16, x);
+    y = pair->narrow(-1, 0, D);
+  } else {
+    y = make(x.sizes(), bf16 ? at::kBFloat16 : at::kFloat, x);
+  }
+  Tensor rstd = make({N}, at::kFloat, x);
+  if (delta) x_out = make(x.sizes(), at::kFloat, x);
+  check(mg_add_rmsnorm_fwd(fp(x), delta ? code(*delta) : 0, ptr(delta), fp(w), fp(x_out), bf16 || with_lo ? MG_BF16 : MG_F32,
+                           ptr(y), with_lo ? h16(*pair) + D : nullptr, with_lo ? 2 * D : D, fp(rstd), N, D, kEps, st(stream)),
+        "mg_add_rmsnorm_fwd");
+  return {x_out, y, rstd, pair};
+}
+
+// (dx, ddelta or none, dw); dy contiguous or none (zero); dy_scale a device scalar or none
+std::tuple<Opt, Opt, Tensor> norm_bwd(const Tensor& xn, const Tensor& w, const Tensor& rstd, const Opt& dy_, const Opt& dres_,
+                                      bool want_dx, int delta_type, const Opt& dy_scale_, int64_t stream) {
+  const int64_t D = xn.size(-1), N = xn.numel() / std::max<int64_t>(D, 1);
+  Tensor dy = dy_ ? dy_->contiguous() : at::zeros(xn.sizes(), xn.options().dtype(at::kFloat));
+  Opt dres, dx, dd, scale;
+  if (dres_) dres = dres_->to(at::kFloat).contiguous();
+  if (dy_scale_) scale = dy_scale_->detach().to(xn.device(), at::kFloat).reshape({1});
+  if (want_dx) dx = make(xn.sizes(), at::kFloat, xn);
+  if (delta_type >= 0) dd = make(xn.sizes(), delta_type == MG_BF16 ? at::kBFloat16 : at::kFloat, xn);
+  Tensor dw = make({D}, at::kFloat, xn);
+  const size_t wsb = mg_add_rmsnorm_bwd_workspace_bytes(N, D);
+  Tensor ws = bytes(wsb, xn);
+  check(mg_add_rmsnorm_bwd_scaled(fp(xn), fp(w), fp(rstd), code(dy), ptr(dy), fp(scale), fp(dres), fp(dx),
+                                  std::max(delta_type, 0), ptr(dd), fp(dw), N, D, ptr(ws), wsb, st(stream)),
+        "mg_add_rmsnorm_bwd");
+  return {dx, dd, dw};
+}
+
+// ------------------------------------------------------------------ scan
+
+// hidden and gate [B, T, Di] with unit inner stride and shared strides, as raw pointers
+struct HG {
+  int dtype;
+  char *hidden, *gate;
+  int64_t sb, ld;
+  int64_t B, T, Di;
+};
+HG split(const Tensor& hg) {  // [B, T, 2 Di] (or [N, 2 Di] with B, T set by the caller), contiguous
+  const int64_t Di = hg.size(-1) / 2;
+  char* p = static_cast<char*>(hg.data_ptr());
+  return {code(hg), p, p + Di * hg.element_size(), hg.dim() == 3 ? hg.size(1) * 2 * Di : 0, 2 * Di,
+          hg.dim() == 3 ? hg.size(0) : 0, hg.dim() == 3 ? hg.size(1) : 0, Di};
+}
+HG two(const Tensor& hidden, const Tensor& gate) {
+  return {code(hidden), static_cast<char*>(hidden.data_ptr()), static_cast<char*>(gate.data_ptr()), hidden.stride(0),
+          hidden.stride(1), hidden.size(0), hidden.size(1), hidden.size(2)};
+}
+
+// (h, h_last, ckpt or none)
+std::tuple<Tensor, Tensor, Opt> scan_fwd_hg(const HG& s, const Opt& h0, at::ScalarType out, bool need_ckpt, const Tensor& ws,
+                                            const Tensor& like, int64_t stream) {
+  Tensor h = make({s.B, s.T, s.Di}, out, like), last = make({s.B, 1, s.Di}, at::kFloat, like);
+  Opt ckpt;
+  if (need_ckpt && out != at::kFloat)
+    ckpt = make({static_cast<int64_t>(mg_scan_ckpt_elems(s.B, s.T, s.Di))}, at::kFloat, like);
+  check(mg_scan_fwd(s.dtype, s.hidden, s.gate, s.sb, s.ld, fp(h0), code(h), ptr(h), h.stride(0), h.stride(1), fp(last),
+                    fp(ckpt), s.B, s.T, s.Di, ptr(ws), ws.numel(), st(stream)),
+        "mg_scan_fwd");
+  return {h, last, ckpt};
+}
+
+// dhidden and dgate into d (a layout like s), returns dh0 or none
+Opt scan_bwd_hg(const HG& s, const Opt& h0, const Opt& h, const Opt& ckpt, const Opt& dh_, const Opt& dlast_, const HG& d,
+                bool want_dh0, const Tensor& ws, const Tensor& like, int64_t stream) {
+  const at::ScalarType hd = h ? h->scalar_type() : at::kFloat;
+  Tensor dh;
+  if (!dh_)
+    dh = at::zeros({s.B, s.T, s.Di}, like.options().dtype(hd));
+  else if (dh_->scalar_type() != hd || dh_->stride(-1) != 1 || dh_->stride(0) % 4 || dh_->stride(1) % 4)
+    dh = dh_->to(hd).contiguous();
+  else
+    dh = *dh_;
+  Opt dlast, dh0;
+  if (dlast_) dlast = dlast_->reshape({s.B, s.Di}).to(at::kFloat).contiguous();
+  if (want_dh0) dh0 = make({s.B, 1, s.Di}, at::kFloat, like);
+  check(mg_scan_bwd(s.dtype, s.hidden, s.gate, s.sb, s.ld, fp(h0), hd == at::kFloat ? MG_F32 : MG_BF16, ptr(h),
+                    h ? h->stride(0) : 0, h ? h->stride(1) : 0, fp(ckpt), ptr(dh), dh.stride(0), dh.stride(1), fp(dlast),
+                    d.hidden, d.gate, d.sb, d.ld, fp(dh0), s.B, s.T, s.Di, ptr(ws), ws.numel(), st(stream)),
+        "mg_scan_bwd");
+  return dh0;
+}
+
+std::tuple<Tensor, Tensor, Opt> scan_fwd(const Tensor& hidden, const Tensor& gate, const Opt& h0, bool bf16_out, bool need_ckpt,
+                                         const Tensor& ws, int64_t stream) {
+  return scan_fwd_hg(two(hidden, gate), h0, bf16_out ? at::kBFloat16 : at::kFloat, need_ckpt, ws, hidden, stream);
+}
+Opt scan_bwd(const Tensor& hidden, const Tensor& gate, const Opt& h0, const Opt& h, const Opt& ckpt, const Opt& dh,
+             const Opt& dlast, const Tensor& dhidden, const Tensor& dgate, bool want_dh0, const Tensor& ws, int64_t stream) {
+  return scan_bwd_hg(two(hidden, gate), h0, h, ckpt, dh, dlast, two(dhidden, dgate), want_dh0, ws, hidden, stream);
+}
+// (x_out, h_last, ckpt): x_out = res + h
+std::tuple<Tensor, Tensor, Tensor> scan_fwd_residual_hg(const HG& s, const Opt& h0, const Tensor& res_, const Tensor& ws,
+                                                        int64_t stream) {
+  const Tensor res = res_.contiguous();
+  Tensor x = make({s.B, s.T, s.Di}, at::kFloat, res), last = make({s.B, 1, s.Di}, at::kFloat, res);
+  Tensor ckpt = make({static_cast<int64_t>(mg_scan_ckpt_elems(s.B, s.T, s.Di))}, at::kFloat, res);
+  check(mg_scan_fwd_residual(s.dtype, s.hidden, s.gate, s.sb, s.ld, fp(h0), fp(res), fp(x), x.stride(0), x.stride(1), fp(last),
+                             fp(ckpt), s.B, s.T, s.Di, ptr(ws), ws.numel(), st(stream)),
+        "mg_scan_fwd_residual");
+  return {x, last, ckpt};
+}
+
+std::tuple<Tensor, Tensor, Tensor> scan_fwd_residual(const Tensor& hidden, const Tensor& gate, const Opt& h0, const Tensor& res,
+                                                     const Tensor& ws, int64_t stream) {
+  return scan_fwd_residual_hg(two(hidden, gate), h0, res, ws, stream);
+}
+
+// ------------------------------------------------------------------ blocks
+
+// MinGRUBlock.forward (blocks.py). x, pending [N, D] rows of [B, T, D]; w_pair, w_bf16:
+// to_hidden_and_gate's hi/lo pair [2 Di, 2 D] and bf16 copy; to_pair: to_out's pair or none.
+// Returns (x1 or none, rstd, pair, hg, h or none, h_last, out or none, h_pair or none, ckpt or
+// none): without to_out, `out` is x1 + h (`residual`) or h; with it, to_out's fp32 output.
+typedef std::tuple<Opt, Tensor, Tensor, Tensor, Opt, Tensor, Tensor, Opt, Opt> GruOut;
+GruOut gru_forward(const Tensor& x, const Opt& pending, const Tensor& w_norm, const Tensor& w_pair, const Tensor& w_bf16,
+                   const Opt& to_pair, const Opt& h0, int64_t B, int64_t T, bool residual, bool one_launch, const Tensor& ws,
+                   int64_t stream) {
+  const int64_t N = x.size(0), D = x.size(1), Di = w_pair.size(0) / 2;
+  auto [x_out, n, rstd, pair] = norm_fwd(x, pending, w_norm, true, true, stream);
+  Tensor hg = make({N, 2 * Di}, at::kBFloat16, x);
+  const Mat pm = mat(*pair, "pair"), wm = mat(w_pair, "w_pair"), hm = mat(hg, "hg");
+  const auto span = [](int64_t rows, int64_t ld) { return (rows + 256) * ld * 2 < (int64_t(1) << 31); };
+  if (one_launch && D % 128 == 0 && Di % 256 == 0 && wm.ld % 8 == 0 && wm.ld >= 2 * D &&
+      reinterpret_cast<uintptr_t>(wm.p) % 16 == 0 && span(N, pm.ld) && span(2 * Di, wm.ld)) {
+    check(mg_gemm_hilo_prefix(pm.p, pm.ld, wm.p, wm.ld, N, 2 * Di, D, Di, hm.p, hm.ld, st(stream)), "mg_gemm_hilo_prefix");
+  } else {
+    linear_fwd_hilo(pm, wm, N, Di, D, MG_BF16, hm, x, stream);  // minGRU.py:45, hidden half
+    const Mat wb = mat(w_bf16, "w_hg");                          // gate half
+    const int64_t step = row_step(N, 2 * std::max(pm.ld, hm.ld));
+    for (int64_t r = 0; r < N; r += step)
+      gemm(MG_KCONTIG, pm.rows(r), MG_KCONTIG, wb.rows(Di), std::min(N - r, step), Di, D, MG_EPI_NONE, nullptr, nullptr, 0,
+           MG_BF16, hm.rows(r).cols(Di), 0, x, stream);
+  }
+  HG s = split(hg);
+  s.B = B, s.T = T, s.sb = T * 2 * Di;
+  const Tensor& x1 = x_out ? *x_out : x;
+  if (!to_pair && residual) {
+    auto [x2, last, ckpt] = scan_fwd_residual_hg(s, h0, x1.view({B, T, D}), ws, stream);
+    return {x_out, rstd, *pair, hg, std::nullopt, last, x2, std::nullopt, ckpt};
+  }
+  auto [h, last, none] = scan_fwd_hg(s, h0, at::kFloat, false, ws, x, stream);
+  if (!to_pair) return {x_out, rstd, *pair, hg, h, last, h, std::nullopt, std::nullopt};
+  Tensor h_pair = make({N, 2 * Di}, at::kBFloat16, x), out = make({N, D}, at::kFloat, x);
+  check(mg_split_hilo(fp(h), Di, N, Di, ptr(h_pair), 2 * Di, st(stream)), "mg_split_hilo");
+  linear_fwd_hilo(mat(h_pair, "h_pair"), mat(*to_pair, "to_pair"), N, D, Di, MG_F32, mat(out, "out"), x, stream);
+  return {x_out, rstd, *pair, hg, h, last, out.view({B, T, D}), h_pair, std::nullopt};
+}
+
+// MinGRUBlock.backward. dx1: the gradient of the residual stream [B, T, D] or none; dout: of
+// to_out's output (with h_pair) or of h. into_hg / into_to: .grad tensors that the weight
+// gradients are added into (then none is returned for them).
+// Returns (dx, dpending or none, dw_norm, dW_hg or none, dh0 or none, dW_to or none).
+typedef std::tuple<Tensor, Opt, Tensor, Opt, Opt, Opt> GruGrads;
+GruGrads gru_backward(const Tensor& xn, const Tensor& w_norm, const Tensor& rstd, const Tensor& pair, const Tensor& hg,
+                      const Opt& h, const Opt& h0, const Tensor& w_bf16, const Opt& ckpt, const Opt& h_pair, const Opt& to_bf16,
+                      const Opt& dx1, const Opt& dout, const Opt& dlast, int64_t B, int64_t T, bool has_pending, bool want_hg,
+                      bool want_to, bool want_dh0, bool pair_launch, const Opt& into_hg, const Opt& into_to, const Tensor& ws,
+                      int64_t stream) {
+  const int64_t N = xn.size(0), D = xn.size(1), Di = hg.size(1) / 2;
+  Opt dh, dW_to, dW_hg, dh0;
+  Tensor dob;
+  if (ckpt) {
+    dh = dx1;  // x_next = x1 + h: h and the residual get the same gradient
+  } else if (dout && h_pair) {
+    const Tensor d = dout->reshape({N, D}).to(at::kFloat).contiguous();
+    dob = make({N, D}, at::kBFloat16, xn);
+    check(mg_round_bf16_sr(fp(d), d.numel(), ptr(dob), 0x3c1d, st(stream)), "mg_round_bf16_sr");
+    dh = linear_dx(dob, *to_bf16, true, stream).view({B, T, Di});
+    if (want_to && !(pair_launch && want_hg)) {
+      Tensor g = linear_dw(mat(dob, "dout"), mat(*h_pair, "h_pair"), N, D, Di, into_to, xn, stream);
+      if (!into_to) dW_to = g;
+    }
+  } else if (dout) {
+    dh = dout->to(at::kFloat);
+  }
+  Tensor dhg = make({N, 2 * Di}, at::kBFloat16, xn);
+  if (!dh && !dlast) {
+    dhg.zero_();
+    if (want_dh0) dh0 = at::zeros_like(*h0);
+  } else {
+    HG s = split(hg), d = split(dhg);
+    s.B = B, s.T = T, s.sb = d.sb = T * 2 * Di;
+    dh0 = scan_bwd_hg(s, h0, h, ckpt, dh, dlast, d, want_dh0, ws, xn, stream);
+  }
+  Tensor dn = linear_dx(dhg, w_bf16, false, stream);
+  if (want_hg) {
+    const Mat dm = mat(dhg, "dhg"), nm = mat(pair, "pair");
+    if (h_pair && dout && want_to && pair_launch) {
+      // to_out's and to_hidden_and_gate's weight gradients in one launch
+      const bool into = into_to && into_hg;
+      auto [g_to, g_hg] = linear_dw_pair(mat(dob, "dout"), mat(*h_pair, "h_pair"), D, Di, dm, nm, 2 * Di, D, N,
+                                         into ? into_to : Opt(), into ? into_hg : Opt(), xn, stream);
+      if (!into) dW_to = g_to, dW_hg = g_hg;
+    } else {
+      Tensor g = linear_dw(dm, nm, N, 2 * Di, D, into_hg, xn, stream);
+      if (!into_hg) dW_hg = g;
+    }
+  }
+  Opt dres;
+  if (dx1) dres = dx1->reshape({N, D});
+  auto [dx, dpend, dw] = norm_bwd(xn, w_norm, rstd, dn, dres, true, has_pending ? MG_BF16 : -1, std::nullopt, stream);
+  return {*dx, dpend, dw, dW_hg, dh0, dW_to};
+}
+
+// FFBlock.forward: (x2 or none, n2, rstd, pre, act, pending) of rows x1 [N, D] (+ out).
+typedef std::tuple<Opt, Tensor, Tensor, Tensor, Tensor, Tensor> FFOut;
+FFOut ff_forward(const Tensor& x1, const Opt& out, const Tensor& w_norm, const Tensor& w1, const Tensor& b1, const Tensor& w2,
+                 const Tensor& b2, int64_t stream) {
+  auto [x2, n2, rstd, none] = norm_fwd(x1, out, w_norm, true, false, stream);
+  Tensor pre = make({x1.size(0), w1.size(0)}, at::kBFloat16, x1);
+  Tensor act = linear_fwd(n2, w1, fp(b1), &pre, stream);     // pre = n2 W1^T + b1, act = gelu(pre)
+  Tensor pend = linear_fwd(act, w2, fp(b2), nullptr, stream);  // act W2^T + b2
+  return {x2, n2, rstd, pre, act, pend};
+}
+
+// (dpre, db1, db2): the GELU backward and both bias gradients (mg_ff_bias_bwd)
+std::tuple<Tensor, Tensor, Tensor> ff_bias_bwd(const Tensor& dact, const Tensor& pre, const Tensor& dy, int64_t stream) {
+  const int64_t N = pre.size(0), C1 = pre.size(1), C2 = dy.size(1);
+  Tensor dpre = make({N, C1}, at::kBFloat16, pre), db1 = make({C1}, at::kFloat, pre), db2 = make({C2}, at::kFloat, pre);
+  const size_t wsb = mg_ff_bias_bwd_workspace_bytes(N, C1, C2);
+  Tensor ws = bytes(wsb, pre);
+  check(mg_ff_bias_bwd(code(dact), ptr(dact), row_stride(dact, "dact"), ptr(pre), row_stride(pre, "pre"), ptr(dpre), C1,
+                       fp(db1), N, C1, ptr(dy), row_stride(dy, "dy"), fp(db2), C2, ptr(ws), wsb, st(stream)),
+        "mg_ff_bias_bwd");
+  return {dpre, db1, db2};
+}
+
+// FFBlock.backward for a bf16 contiguous dpend [N, D]: (dx, dw_norm, dW1 or none, db1, dW2 or
+// none, db2), the weight gradients added into into1 / into2 where given.
+typedef std::tuple<Tensor, Tensor, Opt, Tensor, Opt, Tensor> FFGrads;
+FFGrads ff_backward(const Tensor& x2, const Tensor& w_norm, const Tensor& rstd, const Tensor& n2, const Tensor& pre,
+                    const Tensor& act, const Tensor& w1, const Tensor& w2, const Opt& dx2, const Tensor& dp, bool pair_launch,
+                    const Opt& into1, const Opt& into2, int64_t stream) {
+  const int64_t N = x2.size(0), D = x2.size(1), F = pre.size(1);
+  Tensor dact = linear_dx(dp, w2, false, stream);
+  auto [dpre, db1, db2] = ff_bias_bwd(dact, pre, dp, stream);
+  Tensor dn2 = linear_dx(dpre, w1, false, stream);
+  const Mat dpm = mat(dp, "dpend"), am = mat(act, "act"), dm = mat(dpre, "dpre"), nm = mat(n2, "n2");
+  Opt dW1, dW2;
+  if (pair_launch) {
+    const bool into = into1 && into2;
+    auto [g2, g1] = linear_dw_pair(dpm, am, D, F, dm, nm, F, D, N, into ? into2 : Opt(), into ? into1 : Opt(), x2, stream);
+    if (!into) dW1 = g1, dW2 = g2;
+  } else {
+    Tensor g2 = linear_dw(dpm, am, N, D, F, into2, x2, stream), g1 = linear_dw(dm, nm, N, F, D, into1, x2, stream);
+    if (!into1) dW1 = g1;
+    if (!into2) dW2 = g2;
+  }
+  Opt dres;
+  if (dx2) dres = dx2->reshape({N, D});
+  auto [dx, none, dw] = norm_bwd(x2, w_norm, rstd, dn2, dres, true, -1, std::nullopt, stream);
+  return {*dx, dw, dW1, db1, dW2, db2};
+}
+
+// FinalNormCE.forward: (loss, x + pending or none, embed, rstd, dlogits); w bf16 [V, D]
+std::tuple<Tensor, Opt, Tensor, Tensor, Tensor> head_forward(const Tensor& x, const Opt& pending, const Tensor& w_norm,
+                                                             const Tensor& w, const Tensor& labels, int64_t stream) {
+  const int64_t N = x.size(0), D = x.size(1), V = w.size(0);
+  auto [x_out, embed, rstd, none] = norm_fwd(x, pending, w_norm, true, false, stream);
+  Tensor dl = make({N, V}, at::kBFloat16, x), part = make({mg_logits_cross_entropy_partials(N)}, at::kFloat, x);
+  check(mg_logits_cross_entropy(ptr(embed), D, ptr(w), row_stride(w, "w"), static_cast<int64_t*>(labels.data_ptr()), ptr(dl), V,
+                                fp(part), nullptr, N, D, V, static_cast<float>(1.0 / N), st(stream)),
+        "mg_logits_cross_entropy");
+  return {part.sum() / N, x_out, embed, rstd, dl};
+}
+
+// FinalNormCE.backward: (dx, dpending or none, dw_norm, dW or none); g: the loss's gradient
+std::tuple<Tensor, Opt, Tensor, Opt> head_backward(const Tensor& xn, const Tensor& w_norm, const Tensor& rstd,
+                                                   const Tensor& embed, const Tensor& dl, const Tensor& w, const Tensor& g,
+                                                   bool has_pending, bool want_w, int64_t stream) {
+  Tensor de = linear_dx(dl, w, true, stream);  // fp32, unscaled
+  Opt dW;
+  if (want_w) {
+    dW = linear_dw(mat(dl, "dlogits"), mat(embed, "embed"), xn.size(0), dl.size(1), embed.size(1), std::nullopt, xn, stream);
+    dW->mul_(g);  // the loss's upstream scale, in fp32; no host sync
+  }
+  auto [dx, dpend, dw] = norm_bwd(xn, w_norm, rstd, de, std::nullopt, true, has_pending ? MG_BF16 : -1, g, stream);
+  return {*dx, dpend, dw, dW};
+}
+
+// Column sums of a 2-D fp32 or bf16 tensor with unit inner stride, fp32.
+Tensor column_sum(const Tensor& x, int64_t stream) {
+  const int64_t N = x.size(0), C = x.size(1);
+  Tensor out = make({C}, at::kFloat, x);
+  const size_t wsb = mg_column_sum_workspace_bytes(N, C);
+  Tensor ws = bytes(wsb, x);
+  check(mg_column_sum(code(x), ptr(x), x.stride(0), N, C, fp(out), ptr(ws), wsb, st(stream)), "mg_column_sum");
+  return out;
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_native, m) {
+  typedef py::call_guard<py::gil_scoped_release> nogil;
+  py::register_exception_translator([](std::exception_ptr p) {
+    try {
+      if (p) std::rethrow_exception(p);
+    } catch (const MgError& e) {
+      PyErr_SetString(g_error ? g_error->ptr() : PyExc_RuntimeError, e.what());
+    }
+  });
+  m.def("set_error", [](py::object e) { g_error = new py::object(std::move(e)); });
+  m.def("gemm_f32", &gemm_f32, nogil());
+  m.def("norm_fwd", &norm_fwd, nogil());
+  m.def("norm_bwd", &norm_bwd, nogil());
+  m.def("scan_fwd", &scan_fwd, nogil());
+  m.def("scan_fwd_residual", &scan_fwd_residual, nogil());
+  m.def("scan_bwd", &scan_bwd, nogil());
+  m.def("gru_forward", &gru_forward, nogil());
+  m.def("gru_backward", &gru_backward, nogil());
+  m.def("ff_forward", &ff_forward, nogil());
+  m.def("ff_backward", &ff_backward, nogil());
+  m.def("ff_bias_bwd", &ff_bias_bwd, nogil());
+  m.def("head_forward", &head_forward, nogil());
+  m.def("head_backward", &head_backward, nogil());
+  m.def("column_sum", &column_sum, nogil());
+}

@@ -188,24 +188,10 @@ def gemm_f32(a, a_layout, b, b_layout, M, N, K, out=None, *, bias=None, accumula
     """out[M, N] (=|+=) sum_k A(m, k) B(k, n) (+ bias) for fp32 2-D tensors with a unit inner stride, to
     fp32 accuracy on the bf16 matrix cores (mg_gemm_f32). Results repeat bit for bit; deterministic as in
     gemm()."""
-    _lib.require_cuda(a, b)
-    if a.dtype != torch.float32 or b.dtype != torch.float32:
-        raise _lib.MingruHipError(f"mg_gemm_f32 operands must be float32 (got {a.dtype}, {b.dtype})")
     if deterministic is None:
         deterministic = torch.are_deterministic_algorithms_enabled()
     flags = (FLAG_ACCUMULATE if accumulate else 0) | (FLAG_DETERMINISTIC if deterministic else 0)
-    if out is None:
-        out = torch.empty(M, N, dtype=torch.float32, device=a.device)
-    L = _lib.lib()
-    wkey = (M, N, K, flags)
-    wsb = _WS_BYTES.get(wkey)
-    if wsb is None:
-        wsb = _WS_BYTES[wkey] = L.mg_gemm_f32_workspace_bytes(M, N, K, flags)
-    ws = _workspace(out.device, wsb) if wsb else None
-    _lib.check(L.mg_gemm_f32(a_layout, a.data_ptr(), _rows(a, "A"), b_layout, b.data_ptr(), _rows(b, "B"), M, N, K,
-                             _lib.ptr(bias), out.data_ptr(), _rows(out, "C"), flags, _lib.ptr(ws),
-                             ws.numel() if ws is not None else 0, _lib.stream_of(out)), "mg_gemm_f32")
-    return out
+    return _lib.native().gemm_f32(a, a_layout, b, b_layout, M, N, K, out, bias, flags, _lib.stream_of(a))
 
 
 def linear_dx(dy, w, *, gelu_pre=None, out_dtype=torch.bfloat16, stochastic=False):

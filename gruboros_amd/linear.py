@@ -29,7 +29,7 @@ import torch
 import torch.nn.functional as F
 
 from . import gemm
-from ._lib import check, dtype_code, lib, ptr, stream_of
+from ._lib import check, dtype_code, lib, native, ptr, stream_of
 
 _MM_OUT_DTYPE = None  # whether torch.mm(..., out_dtype=float32) works for bf16 on this build
 
@@ -87,12 +87,7 @@ def column_sum(x2):
     N, C = x2.shape
     if C % 8 or x2.stride(1) != 1 or x2.stride(0) % 8 or x2.data_ptr() % 16:
         return x2.sum(0, dtype=torch.float32)
-    L = lib()
-    out = torch.empty(C, dtype=torch.float32, device=x2.device)
-    ws = torch.empty(L.mg_column_sum_workspace_bytes(N, C), dtype=torch.uint8, device=x2.device)
-    check(L.mg_column_sum(dtype_code(x2.dtype), ptr(x2), x2.stride(0), N, C, ptr(out), ptr(ws), ws.numel(),
-                          stream_of(x2)), "mg_column_sum")
-    return out
+    return native().column_sum(x2, stream_of(x2))
 
 
 def _gelu_grad_f32(pre):
@@ -338,16 +333,7 @@ def gelu_backward_bias_grads(dh, pre, dy):
             dy.stride(1) != 1 or pre.stride(0) % 8 or dh.stride(0) % 8 or dy.stride(0) % 8 or dy.data_ptr() % 16):
         dpre, db1 = gelu_backward(dh, pre)
         return dpre, db1, column_sum(dy)
-    L = lib()
-    dpre = torch.empty_like(pre)
-    db1 = torch.empty(C1, dtype=torch.float32, device=pre.device)
-    db2 = torch.empty(C2, dtype=torch.float32, device=pre.device)
-    wsb = L.mg_ff_bias_bwd_workspace_bytes(N, C1, C2)
-    ws = torch.empty(wsb, dtype=torch.uint8, device=pre.device)
-    check(L.mg_ff_bias_bwd(dtype_code(dh.dtype), ptr(dh), dh.stride(0), ptr(pre), pre.stride(0), ptr(dpre),
-                           dpre.stride(0), ptr(db1), N, C1, ptr(dy), dy.stride(0), ptr(db2), C2, ptr(ws), wsb,
-                           stream_of(pre)), "mg_ff_bias_bwd")
-    return dpre, db1, db2
+    return native().ff_bias_bwd(dh, pre, dy, stream_of(pre))
 
 
 # Where the GELU of the FeedForward runs (measured on MI355X, 16384 x 1024

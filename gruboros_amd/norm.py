@@ -11,63 +11,23 @@ Weights of any floating dtype are accepted (a model cast with
 .to(torch.bfloat16), as reference generate.py:140-142 does); the kernels read
 them as fp32.
 """
-import ctypes
-
 import torch
 
-from ._lib import check, dtype_code, lib, ptr, require_cuda, stream_of
+from ._lib import MG_BF16, dtype_code, native, require_cuda, stream_of
 
 FP32_EPS = float(torch.finfo(torch.float32).eps)
-
-
-def _rows(t):
-    D = t.shape[-1]
-    return t.numel() // D, D
 
 
 def _fwd(x, delta, w, out_dtype, with_lo=False):
     """Returns (x_out, y, rstd, pair): pair is the [..., 2D] hi/lo buffer
     (y is its first half) when with_lo, else None."""
-    N, D = _rows(x)
-    pair = None
-    if with_lo:
-        pair = torch.empty(*x.shape[:-1], 2 * D, dtype=torch.bfloat16, device=x.device)
-        y = pair[..., :D]
-    else:
-        y = torch.empty(x.shape, dtype=out_dtype, device=x.device)
-    rstd = torch.empty(N, dtype=torch.float32, device=x.device)
-    x_out = torch.empty_like(x) if delta is not None else None
-    rc = lib().mg_add_rmsnorm_fwd(ptr(x), dtype_code(delta.dtype) if delta is not None else 0, ptr(delta), ptr(w),
-                                  ptr(x_out), dtype_code(y.dtype), ptr(y),
-                                  ctypes.c_void_p(pair.data_ptr() + 2 * D) if with_lo else None,
-                                  2 * D if with_lo else D, ptr(rstd), N, D, FP32_EPS, stream_of(x))
-    check(rc, "mg_add_rmsnorm_fwd")
-    return x_out, y, rstd, pair
+    require_cuda(x, delta, w)
+    return native().norm_fwd(x, delta, w, dtype_code(out_dtype) == MG_BF16, with_lo, stream_of(x))
 
 
-def _bwd(xn, w, rstd, dy, dres, want_dx, delta_dtype, want_ddelta, dy_scale=None):
-    """dy_scale: an optional fp32 device scalar dy is multiplied by as it is loaded."""
-    N, D = _rows(xn)
-    dev = xn.device
-    if dy is None:
-        dy = torch.zeros(xn.shape, dtype=torch.float32, device=dev)
-    elif not dy.is_contiguous():
-        dy = dy.contiguous()
-    if dres is not None:
-        dres = dres.to(torch.float32).contiguous()
-    dx = torch.empty(xn.shape, dtype=torch.float32, device=dev) if want_dx else None
-    ddelta = torch.empty(xn.shape, dtype=delta_dtype, device=dev) if want_ddelta else None
-    dw = torch.empty(D, dtype=torch.float32, device=dev)
-    L = lib()
-    wsb = L.mg_add_rmsnorm_bwd_workspace_bytes(N, D)
-    ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
-    if dy_scale is not None:
-        dy_scale = dy_scale.detach().to(device=dev, dtype=torch.float32).reshape(1)
-    rc = L.mg_add_rmsnorm_bwd_scaled(ptr(xn), ptr(w), ptr(rstd), dtype_code(dy.dtype), ptr(dy), ptr(dy_scale),
-                                     ptr(dres), ptr(dx), dtype_code(delta_dtype) if want_ddelta else 0,
-                                     ptr(ddelta), ptr(dw), N, D, ptr(ws), wsb, stream_of(xn))
-    check(rc, "mg_add_rmsnorm_bwd")
-    return dx, ddelta, dw
+def _bwd(xn, w, rstd, dy, dres, want_dx, delta_dtype, want_ddelta):
+    return native().norm_bwd(xn, w, rstd, dy, dres, want_dx, dtype_code(delta_dtype) if want_ddelta else -1, None,
+                             stream_of(xn))
 
 
 class RMSNormResidualFn(torch.autograd.Function):

@@ -113,11 +113,6 @@ def surface_errors(device):
         poll_workspaces(device)
 
 
-def _vec_ok(t: torch.Tensor) -> bool:
-    """Last dim dense and the two outer strides multiples of 4 elements."""
-    return t.stride(-1) == 1 and t.stride(0) % 4 == 0 and t.stride(1) % 4 == 0
-
-
 def _prep_h0(h0, B, Di, device):
     if h0 is None:
         return None
@@ -131,61 +126,23 @@ def _launch_fwd(hidden, gate, h0, out_dtype, need_ckpt=False):
     steps) is produced when asked for and h is not fp32: the backward needs
     fp32 states."""
     B, T, Di = hidden.shape
-    L = lib()
-    h = torch.empty(B, T, Di, dtype=out_dtype, device=hidden.device)
-    h_last = torch.empty(B, 1, Di, dtype=torch.float32, device=hidden.device)
-    ckpt = None
-    if need_ckpt and out_dtype != torch.float32:
-        ckpt = torch.empty(L.mg_scan_ckpt_elems(B, T, Di), dtype=torch.float32, device=hidden.device)
-    ws = _workspace(hidden.device, B, T, Di)
-    rc = L.mg_scan_fwd(dtype_code(hidden.dtype), ptr(hidden), ptr(gate), hidden.stride(0), hidden.stride(1),
-                       ptr(h0), dtype_code(out_dtype), ptr(h), h.stride(0), h.stride(1), ptr(h_last), ptr(ckpt),
-                       B, T, Di, ptr(ws), ws.numel(), stream_of(hidden))
-    check(rc, "mg_scan_fwd")
-    return h, h_last, ckpt
+    return _lib.native().scan_fwd(hidden, gate, h0, dtype_code(out_dtype) == _lib.MG_BF16, need_ckpt,
+                                  _workspace(hidden.device, B, T, Di), stream_of(hidden))
 
 
 def _launch_fwd_residual(hidden, gate, h0, res):
     """x_out = res + scan(hidden, gate) (fp32, res's layout: [B, T, Di] with a unit inner stride),
     with the scan state kept as fp32 checkpoints for the backward. Returns (x_out, h_last, ckpt)."""
     B, T, Di = hidden.shape
-    L = lib()
-    x_out = torch.empty(B, T, Di, dtype=torch.float32, device=hidden.device)
-    h_last = torch.empty(B, 1, Di, dtype=torch.float32, device=hidden.device)
-    ckpt = torch.empty(L.mg_scan_ckpt_elems(B, T, Di), dtype=torch.float32, device=hidden.device)
-    if res.stride() != x_out.stride():
-        res = res.contiguous()
-    ws = _workspace(hidden.device, B, T, Di)
-    rc = L.mg_scan_fwd_residual(dtype_code(hidden.dtype), ptr(hidden), ptr(gate), hidden.stride(0), hidden.stride(1),
-                                ptr(h0), ptr(res), ptr(x_out), x_out.stride(0), x_out.stride(1), ptr(h_last),
-                                ptr(ckpt), B, T, Di, ptr(ws), ws.numel(), stream_of(hidden))
-    check(rc, "mg_scan_fwd_residual")
-    return x_out, h_last, ckpt
+    return _lib.native().scan_fwd_residual(hidden, gate, h0, res, _workspace(hidden.device, B, T, Di), stream_of(hidden))
 
 
 def _launch_bwd(hidden, gate, h0, h, ckpt, dh, dh_last, dhidden, dgate, want_dh0):
     """dhidden, dgate: outputs with a shared layout (their strides are passed). h may be None when
     ckpt holds the forward's fp32 state checkpoints (the states are rebuilt from them)."""
     B, T, Di = hidden.shape
-    L = lib()
-    dev = hidden.device
-    hd = h.dtype if h is not None else torch.float32
-    if dh is None:
-        dh = torch.zeros(B, T, Di, dtype=hd, device=dev)
-    elif dh.dtype != hd or not _vec_ok(dh):
-        dh = dh.to(hd).contiguous()
-    if dh_last is not None:
-        dh_last = dh_last.reshape(B, Di).to(torch.float32).contiguous()
-    dh0 = torch.empty(B, 1, Di, dtype=torch.float32, device=dev) if want_dh0 else None
-    ws = _workspace(dev, B, T, Di)
-    rc = L.mg_scan_bwd(dtype_code(hidden.dtype), ptr(hidden), ptr(gate), hidden.stride(0), hidden.stride(1),
-                       ptr(h0), dtype_code(hd), ptr(h), h.stride(0) if h is not None else 0,
-                       h.stride(1) if h is not None else 0, ptr(ckpt),
-                       ptr(dh), dh.stride(0), dh.stride(1), ptr(dh_last), ptr(dhidden), ptr(dgate),
-                       dhidden.stride(0), dhidden.stride(1), ptr(dh0), B, T, Di, ptr(ws), ws.numel(),
-                       stream_of(hidden))
-    check(rc, "mg_scan_bwd")
-    return dh0
+    return _lib.native().scan_bwd(hidden, gate, h0, h, ckpt, dh, dh_last, dhidden, dgate, want_dh0,
+                                  _workspace(hidden.device, B, T, Di), stream_of(hidden))
 
 
 class GateScanPacked(torch.autograd.Function):
