@@ -1129,15 +1129,26 @@ struct W4MPipe {
   }
 };
 
-template <bool AK, bool BKM>
+// kRagged: an MN-contiguous operand's row count need not be a multiple of 256.
+// Its tile origin then rides in the per-lane offset (with the k offset), so the
+// buffer's range check covers the whole address; columns past the operand read
+// the next k-row's (or zero) and reach only output rows or columns that the
+// caller does not store.
+template <bool AK, bool BKM, bool kRagged = false>
 __device__ __forceinline__ void mainloop_w4m(const Params& p, uint4* sa, uint4* sb, int m0, int n0, int kt0, int kt1,
                                              f32x4v (&acc)[8][8]) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   W4MPipe<AK, BKM> P;
   P.init(p, wave, lane);
-  const uint32_t ar = P.aorg(m0), br = P.borg(n0);
+  constexpr bool kFoldA = kRagged && !AK, kFoldB = kRagged && !BKM;
+  const uint32_t ar = kFoldA ? 0 : P.aorg(m0), br = kFoldB ? 0 : P.borg(n0);
+  const uint32_t af = kFoldA ? P.aorg(m0) : 0, bf = kFoldB ? P.borg(n0) : 0;
   // k offsets of k-tile t (relative to kt0); tiles past kt1 reload tile kt1 - 1
-  auto koffs = [&](int t, uint32_t& ao, uint32_t& bo) { P.koffs(min(kt0 + t, kt1 - 1), ao, bo); };
+  auto koffs = [&](int t, uint32_t& ao, uint32_t& bo) {
+    P.koffs(min(kt0 + t, kt1 - 1), ao, bo);
+    ao += af;
+    bo += bf;
+  };
   const int n = kt1 - kt0;
   // prologue: tiles 0 and 1 in flight, tile 0's k-step 0 multiplied, then the
   // mid-tile barrier of tile 0
@@ -1508,6 +1519,152 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_pair_kernel(Params p0, Para
   const int bx = blockIdx.x;
   if (bx < wgs0) gemm_tile<BM, BN, WM, WN, AK, BKM, EPI_NONE, float, C_SPLIT>(p0, bx, 0);
   else gemm_tile<BM, BN, WM, WN, AK, BKM, EPI_NONE, float, C_SPLIT>(p1, bx - wgs0, 0);
+}
+
+// The split-K reduction reads each partial once and writes a weight gradient
+// the optimizer reads at the end of the step: both carry the non-temporal hint
+// (cfg3 step 11.19 -> 11.14 ms).
+typedef float f32x4_nt __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ f4 load4_stream(const float* q) {
+  const f32x4_nt x = __builtin_nontemporal_load(reinterpret_cast<const f32x4_nt*>(q));
+  f4 r; r.v[0] = x[0]; r.v[1] = x[1]; r.v[2] = x[2]; r.v[3] = x[3];
+  return r;
+}
+__device__ __forceinline__ void store4_stream(float* q, const f4& r) {
+  const f32x4_nt x = {r.v[0], r.v[1], r.v[2], r.v[3]};
+  __builtin_nontemporal_store(x, reinterpret_cast<f32x4_nt*>(q));
+}
+
+// ---------------------------------------------------------------- grouped products
+//
+// The products of a block's backward that depend only on one finished gradient
+// (dX = dY W, rounded stochastically to bf16, and one or two weight gradients
+// dY^T X) in one launch of 256 x 256 tiles, each split along K so that all
+// workgroups do about the same number of k-tiles. At 2048 rows each of them
+// alone has 24 to 96 such tiles: on 128 x 128 tiles with their own splits they
+// ran at 0.5-0.7 PFLOP/s (a 128 x 128 tile needs 64 bytes of LDS fill per
+// cycle and CU, twice what the loads sustain) and wrote 4 partials each;
+// together they give every CU one tile's share of about the same length, and
+// only the products that must be split write partials. What bounds the launch
+// now: the k-tiles (1.25 us each against 0.85 at the matrix cores' full rate)
+// and the stores, which no MFMA overlaps.
+// A workgroup's tile is stored by output kind: fp32 partial slice (then
+// group_reduce_kernel), fp32 C written or added to, or bf16 C rounded
+// stochastically.
+struct GroupParams {
+  Params p0, p1, p2;     // p0: A K-contiguous, B MN-contiguous (dX); p1, p2: both MN-contiguous (dW)
+  int wg1, wg2;          // first workgroup of p1, p2 (multiples of 8, so a workgroup's XCD is its index % 8)
+  int splits0, splits1, splits2;
+};
+
+template <bool AK, bool BKM>
+__device__ __forceinline__ void group_tile(const Params& p, int L, int splits, bool bf16_out, uint4* sa, uint4* sb) {
+  // (split, tile) pairs in split order, a contiguous range of them per XCD: an
+  // XCD's workgroups share a split's k-slices in its L2
+  const int T = p.tiles_m * p.tiles_n, per_xcd = (T * splits + 7) >> 3;
+  const int g = (L & 7) * per_xcd + (L >> 3);
+  if ((L >> 3) >= per_xcd || g >= T * splits) return;  // padding (whole workgroups)
+  const int split = g / T, pid = g - split * T;
+  const int per_group = 8 * p.tiles_n, group = pid / per_group, first = group * 8;
+  const int gsize = min(p.tiles_m - first, 8), in_group = pid - group * per_group;
+  const int m0 = (first + in_group % gsize) * 256, n0 = (in_group / gsize) * 256;
+  const int kt0 = split * p.kt_per_split, kt1 = min((p.K + BK - 1) / BK, kt0 + p.kt_per_split);
+  f32x4v acc[8][8];
+  mainloop_w4m<AK, BKM, true>(p, sa, sb, m0, n0, kt0, kt1, acc);
+
+  // 32 rows of the wave's 128 x 128 at a time through a wave-private 16 KB of
+  // the first stage, read back as 16-byte chunks of rows (as gemm_tile)
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int row0 = m0 + (wave >> 1) * 128, col0 = n0 + (wave & 1) * 128;
+  unsigned char* stage = reinterpret_cast<unsigned char*>(sa) + wave * 16384;
+  const int hq = lane >> 4, rl = lane & 15, qc = lane & 31, n = col0 + 4 * qc;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      const int r = 16 * a + rl;
+#pragma unroll
+      for (int J = 0; J < 8; ++J) {
+        f4 x;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x.v[e] = acc[2 * i + a][J][e];
+        io4<float>::store(reinterpret_cast<float*>(stage + r * 512 + (((4 * J + hq) ^ r) * 16)), x);
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+      const int r = 2 * t + (lane >> 5);
+      const int m = row0 + 32 * i + r;
+      f4 x = io4<float>::load(reinterpret_cast<const float*>(stage + r * 512 + ((qc ^ r) * 16)));
+      if (m >= p.M || n >= p.N) continue;
+      if (splits > 1) {
+        io4<float>::store(p.part + (static_cast<int64_t>(split) * p.M + m) * p.N + n, x);
+      } else if (bf16_out) {
+        io4<bf16_t>::store_grad(static_cast<bf16_t*>(p.C) + static_cast<int64_t>(m) * p.ldc + n, x,
+                                static_cast<uint32_t>(static_cast<int64_t>(m) * p.N + n), 0x9e5bu);
+      } else {
+        float* cp = static_cast<float*>(p.C) + static_cast<int64_t>(m) * p.ldc + n;
+        if (p.accumulate) {
+          const f4 old = io4<float>::load(cp);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x.v[e] = old.v[e] + x.v[e];
+        }
+        io4<float>::store(cp, x);
+      }
+    }
+    __syncthreads();
+  }
+}
+
+__global__ __launch_bounds__(256) void gemm_group_kernel(GroupParams g) {
+  __shared__ uint4 sa[2 * kW4Rows * 8];
+  __shared__ uint4 sb[2 * kW4Rows * 8];
+  const int bx = blockIdx.x;
+  if (bx < g.wg1) {
+    group_tile<true, false>(g.p0, bx, g.splits0, true, sa, sb);
+  } else {
+    Params p = g.p1;
+    int L = bx - g.wg1, splits = g.splits1;
+    if (bx >= g.wg2) p = g.p2, L = bx - g.wg2, splits = g.splits2;
+    group_tile<false, false>(p, L, splits, false, sa, sb);
+  }
+}
+
+// The split products' partials, summed in split order: into bf16 C rounded
+// stochastically (p0), into fp32 C (p1, p2), C's old value added last. Blocks
+// [0, b1), [b1, b2), [b2, ...) serve p0, p1, p2.
+__global__ __launch_bounds__(256) void group_reduce_kernel(GroupParams g, int b1, int b2) {
+  const int q = static_cast<int>(blockIdx.x) < b1 ? 0 : static_cast<int>(blockIdx.x) < b2 ? 1 : 2;
+  const Params p = q == 0 ? g.p0 : q == 1 ? g.p1 : g.p2;
+  const int S = q == 0 ? g.splits0 : q == 1 ? g.splits1 : g.splits2;
+  const int first = q == 0 ? 0 : q == 1 ? b1 : b2;
+  const int nb = (q == 0 ? b1 : q == 1 ? b2 : static_cast<int>(gridDim.x)) - first;
+  const int n4 = p.M * (p.N / 4), N4 = p.N / 4;  // (below 2^29: the host checks)
+  const int64_t slice = static_cast<int64_t>(p.M) * p.N;
+  for (int i = (blockIdx.x - first) * 256 + threadIdx.x; i < n4; i += nb * 256) {
+    const int m = i / N4, n = (i - m * N4) * 4;
+    const float* pp = p.part + static_cast<int64_t>(m) * p.N + n;
+    f4 sum = io4<float>::load(pp);
+#pragma unroll 4
+    for (int s = 1; s < S; ++s) {
+      const f4 v = io4<float>::load(pp + s * slice);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum.v[e] += v.v[e];
+    }
+    if (q == 0) {
+      io4<bf16_t>::store_grad(static_cast<bf16_t*>(p.C) + static_cast<int64_t>(m) * p.ldc + n, sum,
+                              static_cast<uint32_t>(m) * static_cast<uint32_t>(p.N) + n, 0x9e5bu);
+    } else {
+      float* cp = static_cast<float*>(p.C) + static_cast<int64_t>(m) * p.ldc + n;
+      if (p.accumulate) {
+        const f4 old = io4<float>::load(cp);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum.v[e] = old.v[e] + sum.v[e];
+      }
+      store4_stream(cp, sum);
+    }
+  }
 }
 
 // ---------------------------------------------------------------- persistent products
@@ -2223,20 +2380,6 @@ __global__ __launch_bounds__(256) void logits_ce_kernel(Params p, const int64_t*
   if (threadIdx.x == 0) loss_part[blockIdx.x] = s_loss[0] + s_loss[1] + s_loss[2] + s_loss[3];
 }
 
-// The split-K reduction reads each partial once and writes a weight gradient
-// the optimizer reads at the end of the step: both carry the non-temporal hint
-// (cfg3 step 11.19 -> 11.14 ms).
-typedef float f32x4_nt __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ f4 load4_stream(const float* q) {
-  const f32x4_nt x = __builtin_nontemporal_load(reinterpret_cast<const f32x4_nt*>(q));
-  f4 r; r.v[0] = x[0]; r.v[1] = x[1]; r.v[2] = x[2]; r.v[3] = x[3];
-  return r;
-}
-__device__ __forceinline__ void store4_stream(float* q, const f4& r) {
-  const f32x4_nt x = {r.v[0], r.v[1], r.v[2], r.v[3]};
-  __builtin_nontemporal_store(x, reinterpret_cast<f32x4_nt*>(q));
-}
-
 // C[m, n] (+)= sum over the S split partials, added in split order.
 __global__ __launch_bounds__(256) void split_reduce_kernel(const float* __restrict__ part, int S, int M, int N,
                                                            float* __restrict__ C, int64_t ldc, int accumulate) {
@@ -2555,10 +2698,139 @@ inline int launch_pair(Params p0, Params p1, const PairPlan& pp, hipStream_t s) 
   return check_launch("mg_gemm_wgrad_pair");
 }
 
+// One launch for a dX product and one or two weight gradients (mg_gemm_group).
+struct GroupPlan {
+  bool ok;
+  int splits[3], kt[3], wgs[3];
+};
+
+// Splits for a group. L, the longest share of k-tiles a workgroup takes, is
+// chosen by estimated time: 1.25 us per k-tile (a 256 x 256 x 64 step), 8 us to
+// start, fill and store a workgroup, and split products' partials written and
+// read at about 7.4 TB/s plus 4 us for their reduction; all workgroups at once
+// (one per CU). The group applies while its tiles fit the CUs at one each.
+// Measured against the products alone (us): expansion-3 minGRU block of 2048
+// rows, d1024 108.1 -> 64.5; FeedForward of 2048 rows, 1024 x 1536: 62.1 -> 41.7,
+// 1024 x 4096: 84.5 -> 58.2; expansion 2, d768, 333 rows: 34.6 -> 24.3; with
+// more tiles than CUs (8192 rows, d1024, expansion 3) 284 -> 287 to 320.
+inline GroupPlan group_plan(const mg_gemm_desc* d, int count, bool deterministic) {
+  GroupPlan best{};
+  if (deterministic || count < 2 || count > 3) return best;
+  int64_t T[3];
+  int kt[3], longest = 0;
+  for (int i = 0; i < count; ++i) {
+    if (d[i].M < 1 || d[i].N < 1 || d[i].K < 1) return best;
+    T[i] = int64_t((d[i].M + 255) / 256) * ((d[i].N + 255) / 256);
+    kt[i] = (d[i].K + BK - 1) / BK;
+    longest = std::max(longest, kt[i]);
+    if (int64_t(d[i].M) * d[i].N >= (int64_t(1) << 31) || T[i] > 4096) return best;
+  }
+  if (d[0].K % BK || T[0] + T[1] + (count > 2 ? T[2] : 0) > kCUs) return best;
+  double least = 1e300;
+  for (int s = 1; s <= 64 && s <= longest; ++s) {
+    const int L = std::max((longest + s - 1) / s, 2);
+    GroupPlan pl{};
+    int64_t wgs = 0;
+    double part = 0;
+    int most = 0;
+    for (int i = 0; i < count; ++i) {
+      const int si = (kt[i] + L - 1) / L;
+      pl.kt[i] = (kt[i] + si - 1) / si;
+      pl.splits[i] = (kt[i] + pl.kt[i] - 1) / pl.kt[i];
+      pl.wgs[i] = static_cast<int>((T[i] * pl.splits[i] + 7) / 8 * 8);
+      wgs += T[i] * pl.splits[i];
+      most = std::max(most, pl.kt[i]);
+      if (pl.splits[i] > 1) part += double(pl.splits[i]) * d[i].M * d[i].N * 8.0;
+    }
+    if (wgs > kCUs) continue;
+    const double cost = 1.25 * most + 8.0 + (part > 0 ? 4.0 + part / 7.4e6 : 0.0);
+    if (cost < least) least = cost, best = pl, best.ok = true;
+  }
+  return best;
+}
+
+inline size_t group_ws(const mg_gemm_desc* d, int count, const GroupPlan& pl) {
+  size_t n = 0;
+  for (int i = 0; i < count; ++i)
+    if (pl.splits[i] > 1) n += static_cast<size_t>(pl.splits[i]) * d[i].M * d[i].N * sizeof(float);
+  return n;
+}
+
 }  // namespace gemm
 }  // namespace mg
 
 using namespace mg;
+
+extern "C" size_t mg_gemm_group_workspace_bytes(const mg_gemm_desc* d, int count, int flags) {
+  if (!d) return 0;
+  const gemm::GroupPlan pl = gemm::group_plan(d, count, flags & MG_GEMM_DETERMINISTIC);
+  return pl.ok ? gemm::group_ws(d, count, pl) : 0;
+}
+
+extern "C" int mg_gemm_group_fits(const mg_gemm_desc* d, int count, int flags) {
+  return d && gemm::group_plan(d, count, flags & MG_GEMM_DETERMINISTIC).ok ? 1 : 0;
+}
+
+extern "C" int mg_gemm_group(const mg_gemm_desc* d, int count, int flags, void* workspace, size_t workspace_bytes,
+                             void* stream) {
+  const char* fn = "mg_gemm_group";
+  if (!d || count < 2 || count > 3) return fail(MG_ERR_ARG, "%s: two or three products", fn);
+  if (flags & ~MG_GEMM_DETERMINISTIC) return fail(MG_ERR_ARG, "%s: unknown flags %d", fn, flags);
+  const gemm::GroupPlan pl = gemm::group_plan(d, count, flags & MG_GEMM_DETERMINISTIC);
+  if (!pl.ok) return fail(MG_ERR_ARG, "%s: these products do not share a launch (mg_gemm_group_fits)", fn);
+  const size_t need = gemm::group_ws(d, count, pl);
+  if (need && (!workspace || workspace_bytes < need))
+    return fail(MG_ERR_WORKSPACE, "%s: workspace %zu bytes < required %zu (mg_gemm_group_workspace_bytes)", fn,
+                workspace_bytes, need);
+  if (need && !aligned(workspace, 16)) return fail(MG_ERR_ARG, "%s: workspace not 16-byte aligned", fn);
+  gemm::GroupParams g{};
+  gemm::Params* ps[3] = {&g.p0, &g.p1, &g.p2};
+  float* part = static_cast<float*>(workspace);
+  for (int i = 0; i < count; ++i) {
+    const mg_gemm_desc& q = d[i];
+    const bool ak = i == 0;
+    if (!q.A || !q.B || !q.C) return fail(MG_ERR_ARG, "%s: null operand", fn);
+    if (q.N % 8 || (!ak && q.M % 8)) return fail(MG_ERR_ARG, "%s: M=%d N=%d (multiples of 8)", fn, q.M, q.N);
+    if (q.lda % 8 || q.ldb % 8 || q.ldc % 4 || q.lda < (ak ? q.K : q.M) || q.ldb < q.N || q.ldc < q.N)
+      return fail(MG_ERR_ARG, "%s: bad leading dimensions", fn);
+    if (!aligned(q.A, 16) || !aligned(q.B, 16) || !aligned(q.C, 16))
+      return fail(MG_ERR_ARG, "%s: operands must be 16-byte aligned", fn);
+    if (q.accumulate && i == 0) return fail(MG_ERR_ARG, "%s: the bf16 product is not accumulated", fn);
+    const int64_t a_span = ak ? (int64_t(q.M - 1) * q.lda + q.K) * 2 : (int64_t(q.K - 1) * q.lda + q.M) * 2;
+    const int64_t b_span = (int64_t(q.K - 1) * q.ldb + q.N) * 2;
+    if (a_span + 512 * q.lda * 2 >= (int64_t(1) << 31) || b_span + 512 * q.ldb * 2 >= (int64_t(1) << 31))
+      return fail(MG_ERR_ARG, "%s: operands must span less than 2 GiB", fn);
+    gemm::Params& p = *ps[i];
+    p.A = static_cast<const bf16_t*>(q.A);
+    p.B = static_cast<const bf16_t*>(q.B);
+    p.C = q.C;
+    p.lda = q.lda; p.ldb = q.ldb; p.ldc = q.ldc;
+    p.M = q.M; p.N = q.N; p.K = q.K;
+    p.a_span = static_cast<uint32_t>(a_span);
+    p.b_span = static_cast<uint32_t>(b_span);
+    p.nkt_seg = (q.K + gemm::BK - 1) / gemm::BK;
+    p.tiles_m = (q.M + 255) / 256;
+    p.tiles_n = (q.N + 255) / 256;
+    p.kt_per_split = pl.kt[i];
+    p.accumulate = q.accumulate ? 1 : 0;
+    if (pl.splits[i] > 1) {
+      p.part = part;
+      part += static_cast<size_t>(pl.splits[i]) * q.M * q.N;
+    }
+  }
+  g.splits0 = pl.splits[0]; g.splits1 = pl.splits[1]; g.splits2 = pl.splits[2];
+  g.wg1 = pl.wgs[0];
+  g.wg2 = pl.wgs[0] + pl.wgs[1];
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  hipLaunchKernelGGL(gemm::gemm_group_kernel, dim3(pl.wgs[0] + pl.wgs[1] + pl.wgs[2]), dim3(256), 0, s, g);
+  if (check_launch(fn)) return MG_ERR_HIP;
+  if (!need) return MG_OK;
+  int nb[3] = {0, 0, 0};
+  for (int i = 0; i < count; ++i)
+    if (pl.splits[i] > 1) nb[i] = static_cast<int>(std::min<int64_t>((int64_t(d[i].M) * (d[i].N / 4) + 255) / 256, 2048));
+  hipLaunchKernelGGL(gemm::group_reduce_kernel, dim3(nb[0] + nb[1] + nb[2]), dim3(256), 0, s, g, nb[0], nb[0] + nb[1]);
+  return check_launch(fn);
+}
 
 extern "C" int mg_gemm(int a_layout, const void* A, int64_t lda, int b_layout, const void* B, int64_t ldb, int M,
                        int N, int K, int epilogue, const float* bias, void* aux, int64_t ldaux, int c_dtype, void* C,

@@ -170,6 +170,41 @@ std::pair<Tensor, Tensor> linear_dw_pair(Mat dy0, Mat x0, int64_t m0, int64_t k0
   return {o0, o1};
 }
 
+// dX = dy w and the weight gradients of `dws` (dy_i [n, m_i], x_i [n, k_i] over the same n
+// rows; each a new tensor or added into `into`) in one launch where they share one
+// (mg_gemm_group); nullopt otherwise.
+struct DW {
+  Mat dy, x;
+  int64_t m, k;
+  Opt into;
+};
+std::optional<std::vector<Tensor>> group(const Tensor& dy, const Tensor& w, const std::vector<DW>& dws, int64_t stream) {
+  const int64_t n = dy.size(0), o = dy.size(1), k = w.size(1);
+  const Mat dm = mat(dy, "dy"), wm = mat(w, "w");
+  const auto span = [](int64_t rows, int64_t ld) { return (rows + 512) * ld * 2 < (int64_t(1) << 31); };
+  bool ok = span(n, dm.ld) && span(o, wm.ld) && (dws.size() == 1 || dws.size() == 2);
+  mg_gemm_desc d[3] = {{dm.p, wm.p, nullptr, dm.ld, wm.ld, k, int(n), int(k), int(o), 0}};
+  for (size_t i = 0; ok && i < dws.size(); ++i) {
+    const DW& q = dws[i];
+    ok = span(n, q.dy.ld) && span(n, q.x.ld);
+    d[i + 1] = {q.dy.p, q.x.p, nullptr, q.dy.ld, q.x.ld, q.k, int(q.m), int(q.k), int(n), q.into ? 1 : 0};
+  }
+  const int count = 1 + int(dws.size()), flags = deterministic() ? MG_GEMM_DETERMINISTIC : 0;
+  if (!ok || !mg_gemm_group_fits(d, count, flags)) return std::nullopt;
+  std::vector<Tensor> out{make({n, k}, at::kBFloat16, dy)};
+  d[0].C = ptr(out[0]);
+  for (size_t i = 0; i < dws.size(); ++i) {
+    out.push_back(dws[i].into ? *dws[i].into : make({dws[i].m, dws[i].k}, at::kFloat, dy));
+    d[i + 1].C = ptr(out.back());
+    d[i + 1].ldc = out.back().stride(0);
+  }
+  const size_t wsb = mg_gemm_group_workspace_bytes(d, count, flags);
+  Tensor ws;
+  if (wsb) ws = bytes(wsb, dy);
+  check(mg_gemm_group(d, count, flags, wsb ? ptr(ws) : nullptr, wsb, st(stream)), "mg_gemm_group");
+  return out;
+}
+
 // sum_k A(m, k) B(k, n) (+ bias) in fp32 (mg_gemm_f32), into `out` or a new tensor
 Tensor gemm_f32(const Tensor& a, int al, const Tensor& b, int bl, int64_t M, int64_t N, int64_t K, const Opt& out_,
                 const Opt& bias, int flags, int64_t stream) {
@@ -371,7 +406,7 @@ GruGrads gru_backward(const Tensor& xn, const Tensor& w_norm, const Tensor& rstd
     dob = make({N, D}, at::kBFloat16, xn);
     check(mg_round_bf16_sr(fp(d), d.numel(), ptr(dob), 0x3c1d, st(stream)), "mg_round_bf16_sr");
     dh = linear_dx(dob, *to_bf16, true, stream).view({B, T, Di});
-    if (want_to && !(pair_launch && want_hg)) {
+    if (want_to && !want_hg) {
       Tensor g = linear_dw(mat(dob, "dout"), mat(*h_pair, "h_pair"), N, D, Di, into_to, xn, stream);
       if (!into_to) dW_to = g;
     }
@@ -387,18 +422,35 @@ GruGrads gru_backward(const Tensor& xn, const Tensor& w_norm, const Tensor& rstd
     s.B = B, s.T = T, s.sb = d.sb = T * 2 * Di;
     dh0 = scan_bwd_hg(s, h0, h, ckpt, dh, dlast, d, want_dh0, ws, xn, stream);
   }
-  Tensor dn = linear_dx(dhg, w_bf16, false, stream);
+  Tensor dn;
+  const Mat dm = mat(dhg, "dhg"), nm = mat(pair, "pair");
+  const bool both = want_hg && want_to && h_pair && dout;
   if (want_hg) {
-    const Mat dm = mat(dhg, "dhg"), nm = mat(pair, "pair");
-    if (h_pair && dout && want_to && pair_launch) {
+    std::vector<DW> dws{{dm, nm, 2 * Di, D, into_hg}};
+    if (both) dws.push_back({mat(dob, "dout"), mat(*h_pair, "h_pair"), D, Di, into_to});
+    if (auto g = group(dhg, w_bf16, dws, stream)) {
+      dn = (*g)[0];
+      if (!into_hg) dW_hg = (*g)[1];
+      if (both && !into_to) dW_to = (*g)[2];
+    }
+  }
+  if (!dn.defined()) {
+    dn = linear_dx(dhg, w_bf16, false, stream);
+    if (both && pair_launch) {
       // to_out's and to_hidden_and_gate's weight gradients in one launch
       const bool into = into_to && into_hg;
       auto [g_to, g_hg] = linear_dw_pair(mat(dob, "dout"), mat(*h_pair, "h_pair"), D, Di, dm, nm, 2 * Di, D, N,
                                          into ? into_to : Opt(), into ? into_hg : Opt(), xn, stream);
       if (!into) dW_to = g_to, dW_hg = g_hg;
     } else {
-      Tensor g = linear_dw(dm, nm, N, 2 * Di, D, into_hg, xn, stream);
-      if (!into_hg) dW_hg = g;
+      if (both) {
+        Tensor g = linear_dw(mat(dob, "dout"), mat(*h_pair, "h_pair"), N, D, Di, into_to, xn, stream);
+        if (!into_to) dW_to = g;
+      }
+      if (want_hg) {
+        Tensor g = linear_dw(dm, nm, N, 2 * Di, D, into_hg, xn, stream);
+        if (!into_hg) dW_hg = g;
+      }
     }
   }
   Opt dres;
@@ -439,17 +491,24 @@ FFGrads ff_backward(const Tensor& x2, const Tensor& w_norm, const Tensor& rstd, 
   const int64_t N = x2.size(0), D = x2.size(1), F = pre.size(1);
   Tensor dact = linear_dx(dp, w2, false, stream);
   auto [dpre, db1, db2] = ff_bias_bwd(dact, pre, dp, stream);
-  Tensor dn2 = linear_dx(dpre, w1, false, stream);
   const Mat dpm = mat(dp, "dpend"), am = mat(act, "act"), dm = mat(dpre, "dpre"), nm = mat(n2, "n2");
+  Tensor dn2;
   Opt dW1, dW2;
-  if (pair_launch) {
-    const bool into = into1 && into2;
-    auto [g2, g1] = linear_dw_pair(dpm, am, D, F, dm, nm, F, D, N, into ? into2 : Opt(), into ? into1 : Opt(), x2, stream);
-    if (!into) dW1 = g1, dW2 = g2;
+  if (auto g = group(dpre, w1, {{dpm, am, D, F, into2}, {dm, nm, F, D, into1}}, stream)) {
+    dn2 = (*g)[0];
+    if (!into2) dW2 = (*g)[1];
+    if (!into1) dW1 = (*g)[2];
   } else {
-    Tensor g2 = linear_dw(dpm, am, N, D, F, into2, x2, stream), g1 = linear_dw(dm, nm, N, F, D, into1, x2, stream);
-    if (!into1) dW1 = g1;
-    if (!into2) dW2 = g2;
+    dn2 = linear_dx(dpre, w1, false, stream);
+    if (pair_launch) {
+      const bool into = into1 && into2;
+      auto [g2, g1] = linear_dw_pair(dpm, am, D, F, dm, nm, F, D, N, into ? into2 : Opt(), into ? into1 : Opt(), x2, stream);
+      if (!into) dW1 = g1, dW2 = g2;
+    } else {
+      Tensor g2 = linear_dw(dpm, am, N, D, F, into2, x2, stream), g1 = linear_dw(dm, nm, N, F, D, into1, x2, stream);
+      if (!into1) dW1 = g1;
+      if (!into2) dW2 = g2;
+    }
   }
   Opt dres;
   if (dx2) dres = dx2->reshape({N, D});

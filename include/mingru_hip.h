@@ -410,6 +410,35 @@ int mg_gemm_wgrad_pair(const void* dy0, int64_t ld_dy0, const void* x0, int64_t 
                        void* workspace, size_t workspace_bytes, void* stream);
 size_t mg_gemm_wgrad_pair_workspace_bytes(int M0, int N0, int M1, int N1, int K, int flags);
 
+/* A block backward's products over one finished gradient in one launch
+ * (autograd of reference mingru/minGRU.py:45,71 and mingru/minLM.py:17-23):
+ *   d[0]: dX = dY W, A = dY [M, K] K-contiguous, B = W [K, N] (MN-contiguous),
+ *         C bf16 [M, N], rounded stochastically as mg_gemm's MG_GEMM_STOCHASTIC;
+ *   d[1], d[2] (count 2 or 3): weight gradients dY^T X, A = dY [K, M] and
+ *         B = X [K, N] MN-contiguous, C fp32 [M, N], written, or with
+ *         `accumulate` added to (the product's sum first, then C's old value).
+ * 256 x 256 tiles, each product split along K so that the workgroups do about
+ * equal work; split products go through fp32 partials in the workspace
+ * (mg_gemm_group_workspace_bytes, 16-byte aligned) and one reduction in split
+ * order, so results repeat bit for bit. mg_gemm_group_fits: 1 where the
+ * products share a launch (d[0].K % 64 == 0, at most one 256 x 256 tile per CU
+ * in all, no MG_GEMM_DETERMINISTIC); otherwise mg_gemm_group
+ * fails and the caller runs them alone. N and the weight gradients' M are
+ * multiples of 8, lda and ldb too, ldc of 4; pointers 16-byte aligned; each
+ * operand spans less than 2 GiB. */
+typedef struct mg_gemm_desc {
+  const void* A;
+  const void* B;
+  void* C;
+  int64_t lda, ldb, ldc;
+  int M, N, K;
+  int accumulate;
+} mg_gemm_desc;
+int mg_gemm_group_fits(const mg_gemm_desc* d, int count, int flags);
+size_t mg_gemm_group_workspace_bytes(const mg_gemm_desc* d, int count, int flags);
+int mg_gemm_group(const mg_gemm_desc* d, int count, int flags, void* workspace, size_t workspace_bytes,
+                  void* stream);
+
 /* fp32 -> bf16 hi/lo pairs for MG_GEMM_HILO operands: out[r, c] =
  * bf16(x[r, c]) (RNE), out[r, cols + c] = bf16(x[r, c] - out[r, c]), for
  * rows x cols (cols % 4 == 0; ldx >= cols, ldo >= 2 cols, both % 4 == 0;

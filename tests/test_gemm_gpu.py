@@ -732,3 +732,54 @@ def test_gemm_f32_edges_match_fp64(M, N, K, a_layout, b_layout):
         assert bool((err <= bound + 2.0 ** -23 * old.double().abs()).all()), float(err.max())
         again = gemm_f32(a, a_layout, b, b_layout, M, N, K, out=old.to(DEV), accumulate=True, deterministic=det)
         assert torch.equal(z, again)
+
+
+@pytest.mark.parametrize("n,o,k,dws", [
+    (1, 64, 8, [(8, 8)]), (37, 128, 72, [(128, 72), (40, 264)]), (255, 512, 256, [(512, 256)]),
+    (257, 192, 328, [(192, 328), (328, 136)]), (2047, 6144, 1024, [(6144, 1024), (1024, 3072)]),
+    (2048, 1536, 1024, [(1024, 1536), (1536, 1024)])])
+def test_gemm_group_matches_fp64(n, o, k, dws):
+    """mg_gemm_group (dX and the weight gradients of a block's backward in one launch, reference
+    mingru/minGRU.py:45,71 and minLM.py:17-23 backward) at ragged sizes of its 256 x 256 x 64 tiles,
+    against float64. Weight gradients, written and accumulated (equal bit for bit to adding the
+    written one to the old value): fp32 accumulation's bound (n + 8) 2^-24 sum |a b|. dX: the same
+    with o terms, plus one bf16 ulp (2^-7) for the stochastic rounding."""
+    import ctypes
+
+    from gruboros_amd import _lib
+
+    class Desc(ctypes.Structure):
+        _fields_ = [("A", ctypes.c_void_p), ("B", ctypes.c_void_p), ("C", ctypes.c_void_p), ("lda", ctypes.c_int64),
+                    ("ldb", ctypes.c_int64), ("ldc", ctypes.c_int64), ("M", ctypes.c_int), ("N", ctypes.c_int),
+                    ("K", ctypes.c_int), ("accumulate", ctypes.c_int)]
+
+    L = _lib.lib()
+    g = torch.Generator().manual_seed(n + o + k)
+    bf = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)
+    dy, w = bf(n, o), bf(o, k)
+    pairs = [(bf(n, m), bf(n, kk)) for m, kk in dws]
+    dev = [t.to(DEV) for t in (dy, w)] + [t.to(DEV) for p in pairs for t in p]
+    old = [torch.randn(m, kk, generator=g).to(DEV) for m, kk in dws]
+    res = {}
+    for acc in (0, 1):
+        dx = torch.empty(n, k, dtype=torch.bfloat16, device=DEV)
+        outs = [x.clone() for x in old]
+        d = (Desc * (1 + len(dws)))()
+        d[0] = Desc(dev[0].data_ptr(), dev[1].data_ptr(), dx.data_ptr(), o, k, k, n, k, o, 0)
+        for i, (m, kk) in enumerate(dws):
+            d[i + 1] = Desc(dev[2 + 2 * i].data_ptr(), dev[3 + 2 * i].data_ptr(), outs[i].data_ptr(), m, kk, kk, m, kk, n, acc)
+        assert L.mg_gemm_group_fits(d, len(d), 0) == 1 and L.mg_gemm_group_fits(d, len(d), 2) == 0
+        wsb = L.mg_gemm_group_workspace_bytes(d, len(d), 0)
+        ws = torch.empty(max(wsb, 16), dtype=torch.uint8, device=DEV)
+        _lib.check(L.mg_gemm_group(d, len(d), 0, ws.data_ptr(), wsb, _lib.stream_of(dx)), "mg_gemm_group")
+        res[acc] = (dx, outs)
+    mag = dy.double().abs() @ w.double().abs()
+    ref = dy.double() @ w.double()
+    err = (res[0][0].double().cpu() - ref).abs()
+    assert bool((err <= (o + 8) * 2.0 ** -24 * mag + 2.0 ** -7 * ref.abs()).all()), float((err / mag).max())
+    assert torch.equal(res[0][0].view(torch.int16), res[1][0].view(torch.int16))
+    for i, (a, b) in enumerate(pairs):
+        ref, mag = a.double().t() @ b.double(), a.double().abs().t() @ b.double().abs()
+        err = (res[0][1][i].double().cpu() - ref).abs()
+        assert bool((err <= (n + 8) * 2.0 ** -24 * mag).all()), float((err / mag).max())
+        assert torch.equal(res[1][1][i], old[i] + res[0][1][i])
