@@ -93,6 +93,8 @@ SIGNATURES = {
     "mg_gemm_group_workspace_bytes": (_c_size, [_vp, _c_int, _c_int]),
     "mg_gemm_group": (_c_int, [_vp, _c_int, _c_int, _vp, _c_size, _vp]),
     "mg_gemm_hilo_prefix": (_c_int, [_vp, _c_i64, _vp, _c_i64, _c_int, _c_int, _c_int, _c_int, _vp, _c_i64, _vp]),
+    "mg_gemm_hilo_cols": (_c_int, [_vp, _c_i64, _vp, _c_i64, _c_int, _c_int, _c_int, _c_int, _vp, _c_i64, _vp]),
+    "mg_gemm_hilo_cols_fits": (_c_int, [_c_int, _c_int, _c_int, _c_int]),
     "mg_gemm_workspace_bytes": (_c_size, [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int]),
     "mg_gemm_wgrad_pair": (_c_int, [_vp, _c_i64, _vp, _c_i64, _c_int, _c_int, _fp, _c_i64,
                                     _vp, _c_i64, _vp, _c_i64, _c_int, _c_int, _fp, _c_i64, _c_int, _c_int,

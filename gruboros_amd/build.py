@@ -54,7 +54,7 @@ def _run(cmd, verbose):
 # whose instruction order keeps the hazards away only as written, so a spill the
 # compiler inserts between those instructions can change results. Their
 # register use is checked at every build.
-NO_SPILL_KERNELS = ("gemm_persist_w4m_kernel", "gemm_kernelILi256ELi256ELi2ELi2E", "gemm_pair_kernel", "gemm_group_kernel")
+NO_SPILL_KERNELS = ("gemm_persist_w4m_kernel", "gemm_kernelILi256ELi256ELi2ELi2E", "gemm_pair_kernel", "gemm_group_kernel", "gemm_t128_")
 
 
 def _spilled_kernels(remarks):

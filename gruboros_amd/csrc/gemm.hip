@@ -1557,8 +1557,10 @@ struct GroupParams {
   int splits0, splits1, splits2;
 };
 
+enum GroupOut { OUT_F32 = 0, OUT_BF16 = 1, OUT_BF16_SR = 2 };
+
 template <bool AK, bool BKM>
-__device__ __forceinline__ void group_tile(const Params& p, int L, int splits, bool bf16_out, uint4* sa, uint4* sb) {
+__device__ __forceinline__ void group_tile(const Params& p, int L, int splits, GroupOut out, uint4* sa, uint4* sb) {
   // (split, tile) pairs in split order, a contiguous range of them per XCD: an
   // XCD's workgroups share a split's k-slices in its L2
   const int T = p.tiles_m * p.tiles_n, per_xcd = (T * splits + 7) >> 3;
@@ -1600,7 +1602,9 @@ __device__ __forceinline__ void group_tile(const Params& p, int L, int splits, b
       if (m >= p.M || n >= p.N) continue;
       if (splits > 1) {
         io4<float>::store(p.part + (static_cast<int64_t>(split) * p.M + m) * p.N + n, x);
-      } else if (bf16_out) {
+      } else if (out == OUT_BF16) {
+        io4<bf16_t>::store(static_cast<bf16_t*>(p.C) + static_cast<int64_t>(m) * p.ldc + n, x);
+      } else if (out == OUT_BF16_SR) {
         io4<bf16_t>::store_grad(static_cast<bf16_t*>(p.C) + static_cast<int64_t>(m) * p.ldc + n, x,
                                 static_cast<uint32_t>(static_cast<int64_t>(m) * p.N + n), 0x9e5bu);
       } else {
@@ -1622,12 +1626,12 @@ __global__ __launch_bounds__(256) void gemm_group_kernel(GroupParams g) {
   __shared__ uint4 sb[2 * kW4Rows * 8];
   const int bx = blockIdx.x;
   if (bx < g.wg1) {
-    group_tile<true, false>(g.p0, bx, g.splits0, true, sa, sb);
+    group_tile<true, false>(g.p0, bx, g.splits0, OUT_BF16_SR, sa, sb);
   } else {
     Params p = g.p1;
     int L = bx - g.wg1, splits = g.splits1;
     if (bx >= g.wg2) p = g.p2, L = bx - g.wg2, splits = g.splits2;
-    group_tile<false, false>(p, L, splits, false, sa, sb);
+    group_tile<false, false>(p, L, splits, OUT_F32, sa, sb);
   }
 }
 
@@ -1664,6 +1668,254 @@ __global__ __launch_bounds__(256) void group_reduce_kernel(GroupParams g, int b1
       }
       store4_stream(cp, sum);
     }
+  }
+}
+
+// ---------------------------------------------------------------- 256 x 128 tiles, few rows
+//
+// K-contiguous products on 256 x 128 tiles for output sizes whose 256 x 256
+// tiles leave CUs idle: four waves (one per SIMD) of 128 x 64, 16x16x32 MFMAs
+// (128 accumulator registers), three LDS stages of 48 KB. A stage row is 128
+// bytes, laid out as M16Operand<true>'s:
+//   plain   64 k: k-step 0, k-step 1;
+//   hi/lo   the 32 hi and the 32 lo values of one 32-k step, so hi and lo tiles
+//           are loaded once and each serves two of the three limb products
+//           (the segment form, ktile(), loads each operand's hi tile twice).
+// What bounds these products is the latency of the LDS fill: 2048-row shapes
+// read their operands through L2 and the memory-side cache at 1.2 us a 48 KB
+// step with one step in flight (two stages: 65 us for to_hidden_and_gate at
+// d1024, expansion 3); with two in flight the matrix cores set the pace.
+// A step's phases, 32 MFMAs each (i outer):
+//   0: hi hi (plain: k-step 0), reading the step's lo (k-step 1) fragments;
+//      then wait for step t + 1, barrier: step t's stage is free
+//   1: lo hi (plain: k-step 1), with the loads of step t + 3 into that stage
+//   2: hi lo (hi/lo only), reading step t + 1's hi fragments (plain: in phase 1)
+template <bool HILO>
+struct T128Pipe {
+  static constexpr int kStageA = 256 * 8;           // uint4 of the A rows (B's 128 rows follow)
+  static constexpr int kStage = kStageA + 128 * 8;  // 48 KB
+  M16Operand<true> A, B;
+  bf16x8 ah[8], al[8], bh[4], bl[4];
+  uint32_t ar, br;
+  int wave;
+
+  __device__ __forceinline__ void init(const Params& p, int m0, int n0, int wave_, int lane) {
+    wave = wave_;
+    const Operand oa = make_operand(p.A, p.lda, p.a_span), ob = make_operand(p.B, p.ldb, p.b_span);
+    A.init(oa, (wave >> 1) * 128, wave, lane);
+    B.init(ob, (wave & 1) * 64, wave, lane);
+    // hi/lo: chunks 4 .. 7 of a stage row come from the row's lo half
+    const uint32_t lo = HILO ? static_cast<uint32_t>(p.K) * 2u - 64u : 0u;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint32_t c = static_cast<uint32_t>((lane & 7) ^ (lane >> 3) ^ (i & 1));
+      A.v[i] += c & 4u ? lo : 0u;
+      if (i < 4)  // B's loads cover 32 rows a wave
+        B.v[i] = static_cast<uint32_t>(wave * 32 + i * 8 + (lane >> 3)) * ob.ld2 + (c << 4) + (c & 4u ? lo : 0u);
+    }
+    ar = M16Operand<true>::origin(m0, oa.ld2);
+    br = M16Operand<true>::origin(n0, ob.ld2);
+  }
+  // load instruction i (0 .. 11) of a step, k offset ko bytes
+  __device__ __forceinline__ void load(uint4* st, int i, uint32_t ko) const {
+    if (i < 8)
+      A.load(st, wave, i, ko, ar);
+    else
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          B.rsrc, (__attribute__((address_space(3))) void*)(st + kStageA + (wave * 4 + i - 8) * 64), 16, B.v[i - 8] + br, ko, 0, 0);
+  }
+  __device__ __forceinline__ void opaque() {
+    A.opaque();
+    B.opaque();
+  }
+};
+constexpr int kT128Stage = T128Pipe<false>::kStage;
+
+// Steps [kt0, kt1) (of 32 k for hi/lo products, 64 k otherwise) of a tile.
+template <bool HILO>
+__device__ __forceinline__ void mainloop_t128(const Params& p, uint4* s0, uint4* s1, uint4* s2, int m0, int n0, int kt0,
+                                              int kt1, f32x4v (&acc)[8][4]) {
+  typedef T128Pipe<HILO> Pipe;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  Pipe P;
+  P.init(p, m0, n0, wave, lane);
+  const int n = kt1 - kt0;
+  auto ko = [&](int t) {  // past the end: the last step again
+    return static_cast<uint32_t>(min(kt0 + t, kt1 - 1)) * (HILO ? 64u : 128u);
+  };
+  auto load_all = [&](uint4* st, int t) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 12; ++i) P.load(st, i, ko(t));
+  };
+  // the next step has landed (the one after may still fly) and this wave's
+  // fragment reads are done; a bare barrier (a fence would wait for every load)
+  auto wait = [&]() __attribute__((always_inline)) {
+    asm volatile("s_waitcnt vmcnt(12) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  load_all(s0, 0);
+  load_all(s1, 1);
+  load_all(s2, 2);
+  asm volatile("s_waitcnt vmcnt(24)" ::: "memory");  // step 0
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+#pragma unroll
+  for (int j = 0; j < 4; ++j) P.bh[j] = P.B.frag(s0 + Pipe::kStageA, 0, j);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) P.ah[i] = P.A.frag(s0, 0, i);
+  // phase 0 of the step in `st` (A's second fragments first: phase 1 starts with all of B's first or its own)
+  auto phase0 = [&](const uint4* st, auto first) __attribute__((always_inline)) {
+    static_for(std::make_integer_sequence<int, 32>{}, [&](auto mc) __attribute__((always_inline)) {
+      constexpr int m = decltype(mc)::value, i = m >> 2, j = m & 3;
+      if constexpr (decltype(first)::value)
+        mfma16_agpr_first(acc[i][j], P.bh[j], P.ah[i]);
+      else
+        mfma16_agpr(acc[i][j], P.bh[j], P.ah[i]);
+      if constexpr (m % 2 == 0 && m / 2 < 12) {
+        constexpr int r = HILO ? m / 2 : (m / 2 + 8) % 12;  // plain: B's four first
+        if constexpr (r < 8)
+          P.al[r] = P.A.frag(st, 1, r);
+        else
+          P.bl[r - 8] = P.B.frag(st + Pipe::kStageA, 1, r - 8);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  phase0(s0, std::true_type{});
+  wait();  // step 1 is in s1 for every wave; every wave has read step 0
+  // from the barrier after step t's phase 0 to the one after step t + 1's
+  auto unit = [&](int t, uint4* cur, const uint4* nxt) __attribute__((always_inline)) {
+    P.opaque();
+    const uint32_t k3 = ko(t + 3);
+    static_for(std::make_integer_sequence<int, 32>{}, [&](auto mc) __attribute__((always_inline)) {
+      constexpr int m = decltype(mc)::value, i = m >> 2, j = m & 3;
+      mfma16_agpr(acc[i][j], HILO ? P.bh[j] : P.bl[j], P.al[i]);
+      if constexpr (m % 2 == 1 && m / 2 < 12) P.load(cur, m / 2, k3);
+      if constexpr (!HILO && m % 2 == 0 && m >= 4 && m < 28) {  // step t + 1's k-step 0 fragments
+        constexpr int r = (m - 4) / 2;
+        if constexpr (r < 4)
+          P.bh[r] = P.B.frag(nxt + Pipe::kStageA, 0, r);
+        else
+          P.ah[r - 4] = P.A.frag(nxt, 0, r - 4);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    if constexpr (HILO) {
+      static_for(std::make_integer_sequence<int, 32>{}, [&](auto mc) __attribute__((always_inline)) {
+        constexpr int m = decltype(mc)::value, i = m >> 2, j = m & 3;
+        mfma16_agpr(acc[i][j], P.bl[j], P.ah[i]);
+        // step t + 1's hi fragments: B's well after their last use, A's block i - 3 eight
+        // or more MFMAs after its own
+        if constexpr (m >= 4 && m < 8) P.bh[m - 4] = P.B.frag(nxt + Pipe::kStageA, 0, m - 4);
+        if constexpr (m >= 12 && j == 3) P.ah[i - 3] = P.A.frag(nxt, 0, i - 3);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+#pragma unroll
+      for (int i = 5; i < 8; ++i) P.ah[i] = P.A.frag(nxt, 0, i);
+    }
+    phase0(nxt, std::false_type{});
+    wait();  // step t + 2 is in its stage for every wave; every wave has read `nxt`
+  };
+  int t = 0;
+  for (; t + 3 < n; t += 3) {
+    unit(t, s0, s1);
+    unit(t + 1, s1, s2);
+    unit(t + 2, s2, s0);
+  }
+  if (t + 1 < n) unit(t, s0, s1);
+  if (t + 2 < n) unit(t + 1, s1, s2);
+  // the last step's remaining phases
+  static_for(std::make_integer_sequence<int, HILO ? 64 : 32>{}, [&](auto mc) __attribute__((always_inline)) {
+    constexpr int m = decltype(mc)::value, i = (m & 31) >> 2, j = m & 3;
+    if constexpr (m < 32)
+      mfma16_agpr(acc[i][j], HILO ? P.bh[j] : P.bl[j], P.al[i]);
+    else
+      mfma16_agpr(acc[i][j], P.bl[j], P.ah[i]);
+    __builtin_amdgcn_sched_barrier(0);
+  });
+  // 24 wait states after the MFMAs that wrote the last four rows of blocks (mfma16_agpr_drain)
+  asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7"
+               : "+a"(acc[4][0]), "+a"(acc[4][1]), "+a"(acc[4][2]), "+a"(acc[4][3]), "+a"(acc[5][0]), "+a"(acc[5][1]),
+                 "+a"(acc[5][2]), "+a"(acc[5][3]), "+a"(acc[6][0]), "+a"(acc[6][1]), "+a"(acc[6][2]), "+a"(acc[6][3]),
+                 "+a"(acc[7][0]), "+a"(acc[7][1]), "+a"(acc[7][2]), "+a"(acc[7][3]));
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+}
+
+enum T128Out { T128_BF16 = 0, T128_F32 = 1, T128_PART = 2 };
+
+// One 256 x 128 tile (split `split` of the steps) of a product.
+template <bool HILO>
+__device__ __forceinline__ void t128_tile(const Params& p, int pid, int split, T128Out out, uint4* sa, uint4* sb, uint4* sc) {
+  const int per_group = 8 * p.tiles_n, group = pid / per_group, first = group * 8;
+  const int gsize = min(p.tiles_m - first, 8), in_group = pid - group * per_group;
+  const int m0 = (first + in_group % gsize) * 256, n0 = (in_group / gsize) * 128;
+  const int kt0 = split * p.kt_per_split, kt1 = min(p.K / (HILO ? 32 : 64), kt0 + p.kt_per_split);
+  f32x4v acc[8][4];
+  mainloop_t128<HILO>(p, sa, sb, sc, m0, n0, kt0, kt1, acc);
+  // 32 rows of the wave's 128 x 64 at a time through a wave-private 8 KB of the first stage
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int row0 = m0 + (wave >> 1) * 128, col0 = n0 + (wave & 1) * 64;
+  unsigned char* stage = reinterpret_cast<unsigned char*>(sa) + wave * 8192;
+  const int hq = lane >> 4, rl = lane & 15, qc = lane & 15, n = col0 + 4 * qc;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      const int r = 16 * a + rl;
+#pragma unroll
+      for (int J = 0; J < 4; ++J) {
+        f4 x;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x.v[e] = acc[2 * i + a][J][e];
+        io4<float>::store(reinterpret_cast<float*>(stage + r * 256 + (((4 * J + hq) ^ (r & 15)) * 16)), x);
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      const int r = 4 * t + hq, m = row0 + 32 * i + r;
+      const f4 x = io4<float>::load(reinterpret_cast<const float*>(stage + r * 256 + ((qc ^ (r & 15)) * 16)));
+      if (m >= p.M || n >= p.N) continue;
+      if (out == T128_PART)
+        io4<float>::store(p.part + (static_cast<int64_t>(split) * p.M + m) * p.N + n, x);
+      else if (out == T128_F32)
+        io4<float>::store(static_cast<float*>(p.C) + static_cast<int64_t>(m) * p.ldc + n, x);
+      else
+        io4<bf16_t>::store(static_cast<bf16_t*>(p.C) + static_cast<int64_t>(m) * p.ldc + n, x);
+    }
+    __syncthreads();
+  }
+}
+
+// A whole product: workgroup (split, tile), a contiguous range of them per XCD.
+template <bool HILO>
+__global__ __launch_bounds__(256) void gemm_t128_kernel(Params p, int splits, int out) {
+  __shared__ uint4 sa[kT128Stage];
+  __shared__ uint4 sb[kT128Stage];
+  __shared__ uint4 sc[kT128Stage];
+  const int T = p.tiles_m * p.tiles_n, per_xcd = (T * splits + 7) >> 3, L = blockIdx.x;
+  const int g = (L & 7) * per_xcd + (L >> 3);
+  if (g >= T * splits) return;
+  const int split = g / T;
+  t128_tile<HILO>(p, g - split * T, split, static_cast<T128Out>(out), sa, sb, sc);
+}
+
+// to_hidden_and_gate's forward for few rows: p's hi/lo tiles first (one per CU
+// at most), then the gate half q's plain tiles of a third of the work, which
+// the remaining CUs take as they come free.
+__global__ __launch_bounds__(256) void gemm_t128_prefix_kernel(Params p, Params q) {
+  __shared__ uint4 sa[kT128Stage];
+  __shared__ uint4 sb[kT128Stage];
+  __shared__ uint4 sc[kT128Stage];
+  const int T = p.tiles_m * p.tiles_n, W = (T + 7) & ~7, bx = blockIdx.x;
+  if (bx < W) {
+    const int g = (bx & 7) * (W >> 3) + (bx >> 3);
+    if (g < T) t128_tile<true>(p, g, 0, T128_BF16, sa, sb, sc);
+  } else {
+    const int Tq = q.tiles_m * q.tiles_n, L = bx - W, g = (L & 7) * ((Tq + 7) >> 3) + (L >> 3);
+    if (g < Tq) t128_tile<false>(q, g, 0, T128_BF16, sa, sb, sc);
   }
 }
 
@@ -2450,6 +2702,36 @@ __global__ __launch_bounds__(256) void split_reduce_bf16_kernel(const float* __r
 
 constexpr int kCUs = 256;
 
+// Hi/lo products of few 256 x 128 tiles (gemm_t128_kernel), whole 32-k steps.
+// bf16 outputs (to_hidden_and_gate's hidden half; never split): up to 192
+// tiles. There the 256 x 256 tiles of the persistent kernel number 96 at most,
+// each CU's share is one tile of three times the gate half's work, and the rest
+// of the chip idles (to_hidden_and_gate, us: 128 rows d256 e3 18.5 -> 12.4, 333
+// rows d768 e2 42.4 -> 25.7, 1024 rows d512 e1.5 30.6 -> 19.3, 2048 rows d1024
+// e3 69 -> 60 in the block); with 256 tiles (2048 rows, d2048, e2) 124 -> 126.
+// fp32 outputs (to_out) split along K to at most one workgroup per CU, by
+// estimated time: 0.85 us per step, 8 us to start and store, partials written
+// and read at about 7.4 TB/s plus 4 us for their reduction. From 3e9
+// multiply-adds (2048 rows, d1024, e3: 57 -> 43 us in the block); smaller ones
+// are 1 to 3 us faster on 128 x 128 tiles, which start sooner.
+struct HiloPlan {
+  bool ok;
+  int kt_per_split, splits;
+};
+inline HiloPlan hilo_plan(int M, int N, int K, bool f32, bool whole) {
+  HiloPlan best{};
+  const int64_t T = int64_t((M + 255) / 256) * ((N + 127) / 128);
+  if (M < 1 || N < 1 || K < 32 || K % 32 || T > (f32 ? kCUs : 192) || (f32 && double(M) * N * K < 3e9)) return best;
+  const int steps = K / 32;
+  double least = 1e300;
+  for (int s = 1; s == 1 || (f32 && !whole && s * T <= kCUs && steps / s >= 4); ++s) {
+    const int kt = (steps + s - 1) / s, ys = (steps + kt - 1) / kt;
+    const double cost = 0.85 * kt + 8.0 + (ys > 1 ? 4.0 + double(ys) * M * N * 8.0 / 7.4e6 : 0.0);
+    if (cost < least) least = cost, best = HiloPlan{true, kt, ys};
+  }
+  return best;
+}
+
 // Tile size and K split of a product (measured on MI355X): 256 x 256 tiles for
 // weight gradients (both operands MN-contiguous) of whole 256 x 256 tiles, at
 // least 16 of them, K >= 4096, split along K to about one workgroup per CU, and
@@ -2698,6 +2980,25 @@ inline int launch_pair(Params p0, Params p1, const PairPlan& pp, hipStream_t s) 
   return check_launch("mg_gemm_wgrad_pair");
 }
 
+// to_hidden_and_gate's forward on 256 x 128 tiles: p holds the whole product.
+inline int launch_t128_prefix(Params p, int hilo_cols, hipStream_t s) {
+  Params q = p;  // the gate half: a plain product of the hi halves
+  p.b_span = static_cast<uint32_t>((int64_t(hilo_cols - 1) * p.ldb + 2 * p.K) * 2);
+  q.b_span = static_cast<uint32_t>((int64_t(p.N - hilo_cols - 1) * p.ldb + 2 * p.K) * 2);
+  q.B += int64_t(hilo_cols) * p.ldb;
+  q.C = static_cast<bf16_t*>(p.C) + hilo_cols;
+  q.N = p.N - hilo_cols;
+  p.N = hilo_cols;
+  p.tiles_m = q.tiles_m = (p.M + 255) / 256;
+  p.tiles_n = (p.N + 127) / 128;
+  q.tiles_n = (q.N + 127) / 128;
+  p.kt_per_split = p.K / 32;
+  q.kt_per_split = p.K / BK;
+  const int wgs = (p.tiles_m * p.tiles_n + 7) / 8 * 8 + (q.tiles_m * q.tiles_n + 7) / 8 * 8;
+  hipLaunchKernelGGL(gemm_t128_prefix_kernel, dim3(wgs), dim3(256), 0, s, p, q);
+  return check_launch("mg_gemm_hilo_prefix");
+}
+
 // One launch for a dX product and one or two weight gradients (mg_gemm_group).
 struct GroupPlan {
   bool ok;
@@ -2896,6 +3197,31 @@ extern "C" int mg_gemm(int a_layout, const void* A, int64_t lda, int b_layout, c
   p.hilo = hilo ? 1 : 0;
   p.nkt_seg = (K + gemm::BK - 1) / gemm::BK;
   if (K == 0 && accumulate) return MG_OK;
+  if (hilo && epilogue == MG_EPI_NONE && !accumulate) {
+    const gemm::HiloPlan hp = gemm::hilo_plan(M, N, K, c_dtype == MG_F32, deterministic || !workspace);
+    if (hp.ok) {
+      const size_t need = hp.splits > 1 ? static_cast<size_t>(hp.splits) * M * N * sizeof(float) : 0;
+      if (need && workspace_bytes < need)
+        return fail(MG_ERR_WORKSPACE, "%s: workspace %zu bytes < required %zu (mg_gemm_workspace_bytes)", fn, workspace_bytes,
+                    need);
+      if (need && !aligned(workspace, 16)) return fail(MG_ERR_ARG, "%s: workspace not 16-byte aligned", fn);
+      p.part = static_cast<float*>(workspace);
+      p.tiles_m = (M + 255) / 256;
+      p.tiles_n = (N + 127) / 128;
+      p.kt_per_split = hp.kt_per_split;
+      const int out = hp.splits > 1 ? gemm::T128_PART : c_dtype == MG_F32 ? gemm::T128_F32 : gemm::T128_BF16;
+      hipLaunchKernelGGL((gemm::gemm_t128_kernel<true>), dim3((p.tiles_m * p.tiles_n * hp.splits + 7) / 8 * 8), dim3(256), 0, s, p,
+                         hp.splits, out);
+      if (check_launch(fn)) return MG_ERR_HIP;
+      if (hp.splits > 1) {
+        const int64_t n4 = int64_t(M) * (N / 4);
+        hipLaunchKernelGGL(gemm::split_reduce_kernel, dim3(static_cast<int>(std::min<int64_t>((n4 + 255) / 256, 2048))),
+                           dim3(256), 0, s, p.part, hp.splits, M, N, static_cast<float*>(C), ldc, 0);
+        return check_launch(fn);
+      }
+      return MG_OK;
+    }
+  }
   // Without a workspace the product runs unsplit.
   gemm::Plan pl = gemm::plan(M, N, K, ak, bk, c_dtype, epilogue, deterministic || !workspace, hilo);
   if (pl.ysplits > 1) {
@@ -2923,6 +3249,42 @@ extern "C" int mg_gemm(int a_layout, const void* A, int64_t lda, int b_layout, c
   return check_launch(fn);
 }
 
+static int hilo_prefix_params(const char* fn, const void* A, int64_t lda, const void* B, int64_t ldb, int M, int N, int K,
+                              void* C, int64_t ldc, gemm::Params& p) {
+  if (lda < 2 * K || ldb < 2 * K || ldc < N || lda % 8 || ldb % 8 || ldc % 8)
+    return fail(MG_ERR_ARG, "%s: leading dimensions (rows of 2K hi/lo values, ldc >= N, multiples of 8)", fn);
+  if (!aligned(A, 16) || !aligned(B, 16) || !aligned(C, 16)) return fail(MG_ERR_ARG, "%s: operands must be 16-byte aligned", fn);
+  const int64_t a_span = (int64_t(M - 1) * lda + 2 * K) * 2, b_span = (int64_t(N - 1) * ldb + 2 * K) * 2;
+  if (a_span + 256 * lda * 2 >= (int64_t(1) << 31) || b_span + 256 * ldb * 2 >= (int64_t(1) << 31))
+    return fail(MG_ERR_ARG, "%s: operands must span less than 2 GiB", fn);
+  p.A = static_cast<const bf16_t*>(A);
+  p.B = static_cast<const bf16_t*>(B);
+  p.C = C;
+  p.lda = lda; p.ldb = ldb; p.ldc = ldc;
+  p.M = M; p.N = N; p.K = K;
+  p.a_span = static_cast<uint32_t>(a_span);
+  p.b_span = static_cast<uint32_t>(b_span);
+  return MG_OK;
+}
+
+extern "C" int mg_gemm_hilo_cols_fits(int M, int N, int K, int hilo_cols) {
+  return M >= 1 && K >= 64 && K % 64 == 0 && N % 8 == 0 && hilo_cols >= 8 && hilo_cols % 8 == 0 && hilo_cols < N &&
+                 gemm::hilo_plan(M, hilo_cols, K, false, true).ok
+             ? 1
+             : 0;
+}
+
+extern "C" int mg_gemm_hilo_cols(const void* A, int64_t lda, const void* B, int64_t ldb, int M, int N, int K, int hilo_cols,
+                                 void* C, int64_t ldc, void* stream) {
+  const char* fn = "mg_gemm_hilo_cols";
+  if (!A || !B || !C) return fail(MG_ERR_ARG, "%s: null operand", fn);
+  if (!mg_gemm_hilo_cols_fits(M, N, K, hilo_cols))
+    return fail(MG_ERR_ARG, "%s: M=%d N=%d K=%d hilo_cols=%d (mg_gemm_hilo_cols_fits)", fn, M, N, K, hilo_cols);
+  gemm::Params p{};
+  if (const int rc = hilo_prefix_params(fn, A, lda, B, ldb, M, N, K, C, ldc, p)) return rc;
+  return gemm::launch_t128_prefix(p, hilo_cols, static_cast<hipStream_t>(stream));
+}
+
 extern "C" int mg_gemm_hilo_prefix(const void* A, int64_t lda, const void* B, int64_t ldb, int M, int N, int K,
                                    int hilo_cols, void* C, int64_t ldc, void* stream) {
   const char* fn = "mg_gemm_hilo_prefix";
@@ -2932,20 +3294,9 @@ extern "C" int mg_gemm_hilo_prefix(const void* A, int64_t lda, const void* B, in
     return fail(MG_ERR_ARG, "%s: M=%d N=%d K=%d (N a multiple of 8, K of 128)", fn, M, N, K);
   if (hilo_cols < 256 || hilo_cols % 256 || hilo_cols >= N)
     return fail(MG_ERR_ARG, "%s: hilo_cols %d must be a multiple of 256 below N=%d", fn, hilo_cols, N);
-  if (lda < 2 * K || ldb < 2 * K || ldc < N || lda % 8 || ldb % 8 || ldc % 8)
-    return fail(MG_ERR_ARG, "%s: leading dimensions (rows of 2K hi/lo values, ldc >= N, multiples of 8)", fn);
-  if (!aligned(A, 16) || !aligned(B, 16) || !aligned(C, 16)) return fail(MG_ERR_ARG, "%s: operands must be 16-byte aligned", fn);
-  const int64_t a_span = (int64_t(M - 1) * lda + 2 * K) * 2, b_span = (int64_t(N - 1) * ldb + 2 * K) * 2;
-  if (a_span + 256 * lda * 2 >= (int64_t(1) << 31) || b_span + 256 * ldb * 2 >= (int64_t(1) << 31))
-    return fail(MG_ERR_ARG, "%s: operands must span less than 2 GiB", fn);
   gemm::Params p{};
-  p.A = static_cast<const bf16_t*>(A);
-  p.B = static_cast<const bf16_t*>(B);
-  p.C = C;
-  p.lda = lda; p.ldb = ldb; p.ldc = ldc;
-  p.M = M; p.N = N; p.K = K;
-  p.a_span = static_cast<uint32_t>(a_span);
-  p.b_span = static_cast<uint32_t>(b_span);
+  if (const int rc = hilo_prefix_params(fn, A, lda, B, ldb, M, N, K, C, ldc, p)) return rc;
+  if (gemm::hilo_plan(M, hilo_cols, K, false, true).ok) return gemm::launch_t128_prefix(p, hilo_cols, static_cast<hipStream_t>(stream));
   p.hilo = 1;
   p.nkt_seg = K / gemm::BK;  // even: K % 128 == 0
   p.hilo_cols = hilo_cols;
@@ -2960,6 +3311,10 @@ extern "C" int mg_gemm_hilo_prefix(const void* A, int64_t lda, const void* B, in
 extern "C" size_t mg_gemm_workspace_bytes(int a_layout, int b_layout, int M, int N, int K, int epilogue,
                                           int c_dtype, int flags) {
   if (M < 1 || N < 1 || K < 1) return 0;
+  if ((flags & MG_GEMM_HILO) && epilogue == MG_EPI_NONE && !(flags & MG_GEMM_ACCUMULATE)) {
+    const gemm::HiloPlan hp = gemm::hilo_plan(M, N, K, c_dtype == MG_F32, flags & MG_GEMM_DETERMINISTIC);
+    if (hp.ok) return hp.splits > 1 ? static_cast<size_t>(hp.splits) * M * N * sizeof(float) : 0;
+  }
   const gemm::Plan pl = gemm::plan(M, N, K, a_layout == MG_KCONTIG, b_layout == MG_KCONTIG, c_dtype, epilogue,
                                    flags & MG_GEMM_DETERMINISTIC, flags & MG_GEMM_HILO);
   return gemm::ws_bytes(pl, M, N);

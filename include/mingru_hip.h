@@ -386,6 +386,12 @@ int mg_gemm(int a_layout, const void* A, int64_t lda,
  * leading dimensions multiples of 8, 16-byte aligned operands. */
 int mg_gemm_hilo_prefix(const void* A, int64_t lda, const void* B, int64_t ldb, int M, int N, int K, int hilo_cols,
                         void* C, int64_t ldc, void* stream);
+/* mg_gemm_hilo_prefix for few rows: the same result for K % 64 == 0 and any
+ * hilo_cols that is a multiple of 8, where the hi/lo columns make at most 192
+ * tiles of 256 x 128 (mg_gemm_hilo_cols_fits returns 1; otherwise it fails). */
+int mg_gemm_hilo_cols(const void* A, int64_t lda, const void* B, int64_t ldb, int M, int N, int K, int hilo_cols,
+                      void* C, int64_t ldc, void* stream);
+int mg_gemm_hilo_cols_fits(int M, int N, int K, int hilo_cols);
 size_t mg_gemm_workspace_bytes(int a_layout, int b_layout, int M, int N, int K, int epilogue,
                                int c_dtype, int flags);
 

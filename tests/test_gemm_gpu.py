@@ -783,3 +783,31 @@ def test_gemm_group_matches_fp64(n, o, k, dws):
         err = (res[0][1][i].double().cpu() - ref).abs()
         assert bool((err <= (n + 8) * 2.0 ** -24 * mag).all()), float((err / mag).max())
         assert torch.equal(res[1][1][i], old[i] + res[0][1][i])
+
+
+@pytest.mark.parametrize("M,N,K,hc", [(1, 16, 64, 8), (255, 264, 64, 136), (257, 1344, 448, 672), (2047, 6144, 1024, 3072),
+                                      (300, 392, 192, 256)])
+def test_hilo_cols_matches_fp64(M, N, K, hc):
+    """mg_gemm_hilo_cols (to_hidden_and_gate's forward on 256 x 128 tiles, reference
+    mingru/minGRU.py:45) at ragged sizes against float64: the hi/lo columns within one bf16
+    rounding (2^-8) plus the dropped lo lo products' 2^-16 and fp32 accumulation's K 2^-22 of
+    sum |a b|; the others exact products of the hi halves but for K 2^-24 and the rounding."""
+    from gruboros_amd import _lib, gemm
+
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x = torch.randn(M, K, device=DEV, generator=g)
+    w = torch.randn(N, K, device=DEV, generator=g) / K ** 0.5
+    xp, wp = gemm.split_hilo(x), gemm.split_hilo(w)
+    out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+    L = _lib.lib()
+    assert L.mg_gemm_hilo_cols_fits(M, N, K, hc) == 1
+    _lib.check(L.mg_gemm_hilo_cols(xp.data_ptr(), 2 * K, wp.data_ptr(), 2 * K, M, N, K, hc, out.data_ptr(), N,
+                                   _lib.stream_of(out)), "mg_gemm_hilo_cols")
+    xd, wd = x.double().cpu(), w.double().cpu()
+    ref, mag = xd @ wd.t(), xd.abs() @ wd.abs().t()
+    err = (out.double().cpu() - ref).abs()
+    assert bool((err <= 2.0 ** -8 * ref.abs() + (2.0 ** -15 + K * 2.0 ** -22) * mag)[:, :hc].all()), float(err[:, :hc].max())
+    xh, wh = xp[:, :K].double().cpu(), wp[:, :K].double().cpu()
+    ref = xh @ wh.t()
+    err = (out.double().cpu() - ref).abs()
+    assert bool((err <= 2.0 ** -8 * ref.abs() + (K + 8) * 2.0 ** -24 * mag)[:, hc:].all()), float(err[:, hc:].max())
