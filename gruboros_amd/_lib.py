@@ -86,8 +86,8 @@ SIGNATURES = {
     "mg_embedding_bwd": (_c_int, [_vp, _fp, _c_i64, _c_i64, _c_int, _c_int, _fp, _c_i64, _vp, _c_size, _vp]),
     "mg_gemm": (_c_int, [_c_int, _vp, _c_i64, _c_int, _vp, _c_i64, _c_int, _c_int, _c_int, _c_int, _fp, _vp, _c_i64,
                          _c_int, _vp, _c_i64, _c_int, _vp, _c_size, _vp]),
-    "mg_gemm_f32": (_c_int, [_c_int, _fp, _c_i64, _c_int, _fp, _c_i64, _c_int, _c_int, _c_int, _fp, _fp, _c_i64, _c_int,
-                             _vp, _c_size, _vp]),
+    "mg_gemm_f32": (_c_int, [_c_int, _fp, _c_i64, _c_int, _fp, _c_i64, _c_int, _c_int, _c_int, _c_int, _fp, _fp, _c_i64,
+                             _fp, _c_i64, _c_int, _vp, _c_size, _vp]),
     "mg_gemm_f32_workspace_bytes": (_c_size, [_c_int, _c_int, _c_int, _c_int]),
     "mg_gemm_group_fits": (_c_int, [_vp, _c_int, _c_int]),
     "mg_gemm_group_workspace_bytes": (_c_size, [_vp, _c_int, _c_int]),

@@ -2,7 +2,13 @@
 // nn.Linear products of an fp32 model (reference mingru/minGRU.py:45,71;
 // mingru/minLM.py:17-23,75,138) and of their autograd backward.
 //
-//   C[m, n] (=|+=) sum_k A(m, k) B(k, n) (+ bias[n])
+//   C[m, n] (=|+=) epilogue(sum_k A(m, k) B(k, n))
+//
+// with mg_gemm's epilogues in fp32: bias, bias + GELU (keeping the
+// pre-activation for the backward) and the GELU gradient, applied where a sum
+// is complete (the tile's store, or the K-split reduction). The FeedForward's
+// GELU and its gradient were passes of their own (30 us of 430 at [4096, 512]
+// x 2048).
 //
 // Each fp32 value is split into three bf16 limbs h + m + l == x (h = bf16(x),
 // m = bf16(x - h), l = bf16(x - h - m); the differences are exact in fp32),
@@ -55,12 +61,44 @@ struct Params {
   const float* B;
   float* C;
   const float* bias;
+  float* aux;   // BIAS_GELU: receives the pre-activation (nullable); GELU_GRAD: holds it
   float* part;  // split partials: one dense [M, N] slice per split
-  int64_t lda, ldb, ldc;
+  int64_t lda, ldb, ldc, ldaux;
   int M, N, K;
   int tiles_m, tiles_n, kt_per_split;
-  int accumulate;
+  int accumulate, epilogue;
 };
+
+// gelu'(x) with the device library's erff and expf: the fp32 path keeps fp32
+// accuracy (mg_common.h's gelu_grad is a 1.5e-7 approximation for bf16 results).
+__device__ __forceinline__ float gelu_grad_f32(float x) {
+  return 0.5f * (1.0f + erff(x * 0.70710678118654752f)) + x * (expf(-0.5f * x * x) * 0.39894228040143268f);
+}
+
+// What happens to four consecutive sums of row m before they are stored at C.
+__device__ __forceinline__ void finish(const Params& p, int64_t m, int64_t c, f4 x) {
+  float* cp = p.C + m * p.ldc + c;
+  if (p.bias) {
+    const f4 bv = io4<float>::load(p.bias + c);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x.v[e] += bv.v[e];
+  }
+  if (p.epilogue == MG_EPI_BIAS_GELU) {
+    if (p.aux) io4<float>::store(p.aux + m * p.ldaux + c, x);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x.v[e] = gelu(x.v[e]);
+  } else if (p.epilogue == MG_EPI_GELU_GRAD) {
+    const f4 a = io4<float>::load(p.aux + m * p.ldaux + c);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x.v[e] *= gelu_grad_f32(a.v[e]);
+  }
+  if (p.accumulate) {
+    const f4 old = io4<float>::load(cp);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x.v[e] = old.v[e] + x.v[e];
+  }
+  io4<float>::store(cp, x);
+}
 
 // (x0, x1) -> their three limbs as packed bf16 pairs. The conversions round
 // to nearest; x - h and x - h - m are exact.
@@ -287,27 +325,15 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_kernel(Params p) {
       f4 x;
 #pragma unroll
       for (int e = 0; e < 4; ++e) x.v[e] = acc[i][j][e];
-      if constexpr (SPLIT) {
+      if constexpr (SPLIT)
         io4<float>::store(p.part + (static_cast<int64_t>(blockIdx.y) * p.M + m) * p.N + c, x);
-      } else {
-        float* cp = p.C + static_cast<int64_t>(m) * p.ldc + c;
-        if (p.bias) {
-          const f4 bv = io4<float>::load(p.bias + c);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) x.v[e] += bv.v[e];
-        }
-        if (p.accumulate) {
-          const f4 old = io4<float>::load(cp);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) x.v[e] = old.v[e] + x.v[e];
-        }
-        io4<float>::store(cp, x);
-      }
+      else
+        finish(p, m, c, x);
     }
   }
 }
 
-// C (+)= the partials' sum in split order (+ bias)
+// The partials' sum in split order, finished as an unsplit tile's
 __global__ __launch_bounds__(256) void reduce_kernel(Params p, int S) {
   const int64_t n4 = static_cast<int64_t>(p.M) * (p.N / 4), slice = static_cast<int64_t>(p.M) * p.N;
   for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < n4;
@@ -321,18 +347,7 @@ __global__ __launch_bounds__(256) void reduce_kernel(Params p, int S) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) sum.v[e] += v.v[e];
     }
-    float* cp = p.C + m * p.ldc + c;
-    if (p.bias) {
-      const f4 bv = io4<float>::load(p.bias + c);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) sum.v[e] += bv.v[e];
-    }
-    if (p.accumulate) {
-      const f4 old = io4<float>::load(cp);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) sum.v[e] = old.v[e] + sum.v[e];
-    }
-    io4<float>::store(cp, sum);
+    finish(p, m, c, sum);
   }
 }
 
@@ -384,8 +399,8 @@ extern "C" size_t mg_gemm_f32_workspace_bytes(int M, int N, int K, int flags) {
 }
 
 extern "C" int mg_gemm_f32(int a_layout, const float* A, int64_t lda, int b_layout, const float* B, int64_t ldb, int M,
-                           int N, int K, const float* bias, float* C, int64_t ldc, int flags, void* workspace,
-                           size_t workspace_bytes, void* stream) {
+                           int N, int K, int epilogue, const float* bias, float* aux, int64_t ldaux, float* C, int64_t ldc,
+                           int flags, void* workspace, size_t workspace_bytes, void* stream) {
   const char* fn = "mg_gemm_f32";
   if (flags & ~(MG_GEMM_ACCUMULATE | MG_GEMM_DETERMINISTIC)) return fail(MG_ERR_ARG, "%s: unknown flags %d", fn, flags);
   if (!A || !B || !C) return fail(MG_ERR_ARG, "%s: null operand", fn);
@@ -399,7 +414,13 @@ extern "C" int mg_gemm_f32(int a_layout, const float* A, int64_t lda, int b_layo
     return fail(MG_ERR_ARG, "%s: leading dimensions must cover a row and be multiples of 4", fn);
   if (!aligned(A, 16) || !aligned(B, 16) || !aligned(C, 16) || (bias && !aligned(bias, 16)))
     return fail(MG_ERR_ARG, "%s: operands must be 16-byte aligned", fn);
-  if ((flags & MG_GEMM_ACCUMULATE) && bias) return fail(MG_ERR_ARG, "%s: no bias when accumulating", fn);
+  if (epilogue < MG_EPI_NONE || epilogue > MG_EPI_GELU_GRAD) return fail(MG_ERR_ARG, "%s: bad epilogue %d", fn, epilogue);
+  const bool biased = epilogue == MG_EPI_BIAS || epilogue == MG_EPI_BIAS_GELU;
+  if (biased != (bias != nullptr)) return fail(MG_ERR_ARG, "%s: a bias with the bias epilogues, none without", fn);
+  if (epilogue == MG_EPI_GELU_GRAD && !aux) return fail(MG_ERR_ARG, "%s: the GELU gradient needs aux", fn);
+  if (aux && (ldaux < N || ldaux % 4 || !aligned(aux, 16))) return fail(MG_ERR_ARG, "%s: aux rows of N, 16-byte aligned", fn);
+  if ((flags & MG_GEMM_ACCUMULATE) && epilogue != MG_EPI_NONE)
+    return fail(MG_ERR_ARG, "%s: no epilogue when accumulating", fn);
   if (M == 0 || N == 0 || (K == 0 && (flags & MG_GEMM_ACCUMULATE))) return MG_OK;
   if (int64_t((M + 127) / 128) * ((N + 127) / 128) >= (int64_t(1) << 31)) return fail(MG_ERR_ARG, "%s: too many tiles", fn);
   gemm_f32::Plan pl = gemm_f32::plan(M, N, K, (flags & MG_GEMM_DETERMINISTIC) || !workspace);
@@ -412,8 +433,9 @@ extern "C" int mg_gemm_f32(int a_layout, const float* A, int64_t lda, int b_layo
     if (!aligned(workspace, 16)) return fail(MG_ERR_ARG, "%s: workspace not 16-byte aligned", fn);
     p.part = static_cast<float*>(workspace);
   }
-  p.A = A; p.B = B; p.C = C; p.bias = bias;
-  p.lda = lda; p.ldb = ldb; p.ldc = ldc;
+  p.A = A; p.B = B; p.C = C; p.bias = bias; p.aux = aux;
+  p.epilogue = epilogue;
+  p.lda = lda; p.ldb = ldb; p.ldc = ldc; p.ldaux = ldaux;
   p.M = M; p.N = N; p.K = K;
   p.tiles_m = (M + gemm_f32::BM - 1) / gemm_f32::BM;
   p.tiles_n = (N + gemm_f32::BN - 1) / gemm_f32::BN;

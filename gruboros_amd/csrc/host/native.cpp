@@ -205,7 +205,18 @@ std::optional<std::vector<Tensor>> group(const Tensor& dy, const Tensor& w, cons
   return out;
 }
 
-// sum_k A(m, k) B(k, n) (+ bias) in fp32 (mg_gemm_f32), into `out` or a new tensor
+// mg_gemm_f32 on raw operands
+void gemm_f32_raw(int al, const float* a, int64_t lda, int bl, const float* b, int64_t ldb, int64_t M, int64_t N, int64_t K,
+                  int epi, const float* bias, float* aux, float* c, int64_t ldc, int flags, const Tensor& like, int64_t stream) {
+  const size_t wsb = mg_gemm_f32_workspace_bytes(M, N, K, flags);
+  Tensor ws;
+  if (wsb) ws = bytes(wsb, like);
+  check(mg_gemm_f32(al, a, lda, bl, b, ldb, M, N, K, epi, bias, aux, aux ? N : 0, c, ldc, flags, wsb ? ptr(ws) : nullptr, wsb,
+                    st(stream)),
+        "mg_gemm_f32");
+}
+
+// sum_k A(m, k) B(k, n) (+ bias) in fp32, into `out` or a new tensor
 Tensor gemm_f32(const Tensor& a, int al, const Tensor& b, int bl, int64_t M, int64_t N, int64_t K, const Opt& out_,
                 const Opt& bias, int flags, int64_t stream) {
   need_cuda(a);
@@ -213,13 +224,59 @@ Tensor gemm_f32(const Tensor& a, int al, const Tensor& b, int bl, int64_t M, int
   if (a.scalar_type() != at::kFloat || b.scalar_type() != at::kFloat) fail("mg_gemm_f32 operands must be float32");
   Tensor out = out_ ? *out_ : make({M, N}, at::kFloat, a);
   const Mat am = mat(a, "A"), bm = mat(b, "B"), om = mat(out, "C");
-  const size_t wsb = mg_gemm_f32_workspace_bytes(M, N, K, flags);
-  Tensor ws;
-  if (wsb) ws = bytes(wsb, a);
-  check(mg_gemm_f32(al, static_cast<float*>(am.p), am.ld, bl, static_cast<float*>(bm.p), bm.ld, M, N, K, fp(bias),
-                    static_cast<float*>(om.p), om.ld, flags, wsb ? ptr(ws) : nullptr, wsb, st(stream)),
-        "mg_gemm_f32");
+  gemm_f32_raw(al, static_cast<float*>(am.p), am.ld, bl, static_cast<float*>(bm.p), bm.ld, M, N, K,
+               bias ? MG_EPI_BIAS : MG_EPI_NONE, fp(bias), nullptr, static_cast<float*>(om.p), om.ld, flags, a, stream);
   return out;
+}
+
+Tensor column_sum(const Tensor& x, int64_t stream);
+
+// The fp32 FeedForward: (pre or none, act, y) of rows x [N, D]; pre kept with `train`.
+std::tuple<Opt, Tensor, Tensor> ff_f32_forward(const Tensor& x, const Tensor& w1, const Tensor& b1, const Tensor& w2,
+                                               const Tensor& b2, bool train, int64_t stream) {
+  const int64_t N = x.size(0), D = x.size(1), F = w1.size(0), O = w2.size(0);
+  const int flags = deterministic() ? MG_GEMM_DETERMINISTIC : 0;
+  Opt pre;
+  if (train) pre = make({N, F}, at::kFloat, x);
+  Tensor act = make({N, F}, at::kFloat, x), y = make({N, O}, at::kFloat, x);
+  gemm_f32_raw(MG_KCONTIG, fp(x), row_stride(x, "x"), MG_KCONTIG, fp(w1), row_stride(w1, "w1"), N, F, D, MG_EPI_BIAS_GELU,
+               fp(b1), fp(pre), fp(act), F, flags, x, stream);
+  gemm_f32_raw(MG_KCONTIG, fp(act), F, MG_KCONTIG, fp(w2), row_stride(w2, "w2"), N, O, F, MG_EPI_BIAS, fp(b2), nullptr, fp(y),
+               O, flags, x, stream);
+  return {pre, act, y};
+}
+
+// (dx or none, dW1, db1, dW2, db2 or none each) for a contiguous dy [N, O]
+std::tuple<Opt, Opt, Opt, Opt, Opt> ff_f32_backward(const Tensor& x, const Tensor& pre, const Tensor& act, const Tensor& w1,
+                                                    const Tensor& w2, const Tensor& dy, bool want_x, bool want_w1, bool want_b1,
+                                                    bool want_w2, bool want_b2, int64_t stream) {
+  const int64_t N = x.size(0), D = x.size(1), F = pre.size(1), O = dy.size(1);
+  const int flags = deterministic() ? MG_GEMM_DETERMINISTIC : 0;
+  Opt dx, dw1, db1, dw2, db2;
+  const int64_t ldx = row_stride(x, "x"), ld1 = row_stride(w1, "w1"), ld2 = row_stride(w2, "w2");
+  if (want_w2) {
+    dw2 = make({O, F}, at::kFloat, x);
+    gemm_f32_raw(MG_MNCONTIG, fp(dy), O, MG_MNCONTIG, fp(act), F, O, F, N, MG_EPI_NONE, nullptr, nullptr, fp(dw2), F, flags, x,
+                 stream);
+  }
+  if (want_b2) db2 = column_sum(dy, stream);
+  if (want_x || want_w1 || want_b1) {
+    Tensor dpre = make({N, F}, at::kFloat, x);  // dy W2 * gelu'(pre)
+    gemm_f32_raw(MG_KCONTIG, fp(dy), O, MG_MNCONTIG, fp(w2), ld2, N, F, O, MG_EPI_GELU_GRAD, nullptr, fp(pre), fp(dpre), F, flags,
+                 x, stream);
+    if (want_b1) db1 = column_sum(dpre, stream);
+    if (want_w1) {
+      dw1 = make({F, D}, at::kFloat, x);
+      gemm_f32_raw(MG_MNCONTIG, fp(dpre), F, MG_MNCONTIG, fp(x), ldx, F, D, N, MG_EPI_NONE, nullptr, nullptr, fp(dw1), D, flags, x,
+                   stream);
+    }
+    if (want_x) {
+      dx = make({N, D}, at::kFloat, x);
+      gemm_f32_raw(MG_KCONTIG, fp(dpre), F, MG_MNCONTIG, fp(w1), ld1, N, D, F, MG_EPI_NONE, nullptr, nullptr, fp(dx), D, flags, x,
+                   stream);
+    }
+  }
+  return {dx, dw1, db1, dw2, db2};
 }
 
 // ------------------------------------------------------------------ norm
@@ -545,6 +602,53 @@ std::tuple<Tensor, Opt, Tensor, Opt> head_backward(const Tensor& xn, const Tenso
   return {*dx, dpend, dw, dW};
 }
 
+// One layer of the no-grad forward of a model whose activations and parameters share a dtype
+// (bf16: generate.py's cast; fp32), reference mingru/minLM.py:119-130: x [N, D] fp32 residual
+// stream, pending [N, D] or none; norm weights and biases fp32. Returns (x2, pending, h_last), x2
+// without the new pending; nullopt where a width or layout is not the kernels'. The scan writes what
+// the next product reads (bf16 h), or adds its state to the residual stream itself (no to_out), and
+// the GELU is the first product's epilogue.
+std::optional<std::tuple<Tensor, Tensor, Tensor>> infer_layer(const Tensor& x, const Opt& pending, const Tensor& w_norm,
+                                                              const Tensor& w_hg, const Opt& w_to, const Tensor& w_ff,
+                                                              const Tensor& w1, const Tensor& b1, const Tensor& w2,
+                                                              const Tensor& b2, const Opt& h0, int64_t B, int64_t T,
+                                                              const Tensor& ws, int64_t stream) {
+  const int64_t N = x.size(0), D = x.size(1), Di = w_hg.size(0) / 2, F = w1.size(0);
+  const bool f32 = w_hg.scalar_type() == at::kFloat;
+  for (const Tensor* w : {&w_hg, &w1, &w2, w_to ? &*w_to : &w_hg})
+    if (w->scalar_type() != w_hg.scalar_type() || w->dim() != 2 || w->stride(1) != 1 || w->size(0) % 8 || w->size(1) % 8 ||
+        w->stride(0) % 8 || reinterpret_cast<uintptr_t>(w->data_ptr()) % 16)
+      return std::nullopt;
+  if (N < 1 || D > 4096 || Di % 8 || (w_to && (w_to->size(0) != D || w_to->size(1) != Di)) || (!w_to && Di != D) ||
+      w1.size(1) != D || w2.size(0) != D || w2.size(1) != F || x.stride(1) != 1 || x.stride(0) != D)
+    return std::nullopt;
+  const int flags = deterministic() ? MG_GEMM_DETERMINISTIC : 0;
+  const auto linear = [&](const Tensor& a, const Tensor& w) {
+    if (!f32) return linear_fwd(a, w, nullptr, nullptr, stream);
+    Tensor y = make({a.size(0), w.size(0)}, at::kFloat, a);
+    gemm_f32_raw(MG_KCONTIG, fp(a), a.stride(0), MG_KCONTIG, fp(w), w.stride(0), a.size(0), w.size(0), w.size(1), MG_EPI_NONE,
+                 nullptr, nullptr, fp(y), w.size(0), flags, a, stream);
+    return y;
+  };
+  auto [x1_, n, rstd, none] = norm_fwd(x, pending, w_norm, !f32, false, stream);
+  Tensor x1 = x1_ ? *x1_ : x, hg = linear(n, w_hg), x2, n2, last;
+  HG s = split(hg);
+  s.B = B, s.T = T, s.sb = T * 2 * Di;
+  if (w_to) {
+    auto [h, l, no_ckpt] = scan_fwd_hg(s, h0, f32 ? at::kFloat : at::kBFloat16, false, ws, x, stream);
+    auto [x2_, n2_, r2, none2] = norm_fwd(x1, linear(h.view({N, Di}), *w_to), w_ff, !f32, false, stream);
+    x2 = *x2_, n2 = n2_, last = l;
+  } else {
+    auto [xr, l, ckpt] = scan_fwd_residual_hg(s, h0, x1.view({B, T, D}), ws, stream);
+    x2 = xr.view({N, D}), last = l;
+    n2 = std::get<1>(norm_fwd(x2, std::nullopt, w_ff, !f32, false, stream));
+  }
+  if (f32) return std::make_tuple(x2, std::get<2>(ff_f32_forward(n2, w1, b1, w2, b2, false, stream)), last);
+  Tensor pre = make({N, F}, at::kBFloat16, x);  // (the epilogue rounds it to bf16; its values are not used)
+  Tensor act = linear_fwd(n2, w1, fp(b1), &pre, stream);
+  return std::make_tuple(x2, linear_fwd(act, w2, fp(b2), nullptr, stream), last);
+}
+
 // Column sums of a 2-D fp32 or bf16 tensor with unit inner stride, fp32.
 Tensor column_sum(const Tensor& x, int64_t stream) {
   const int64_t N = x.size(0), C = x.size(1);
@@ -568,6 +672,8 @@ PYBIND11_MODULE(_native, m) {
   });
   m.def("set_error", [](py::object e) { g_error = new py::object(std::move(e)); });
   m.def("gemm_f32", &gemm_f32, nogil());
+  m.def("ff_f32_forward", &ff_f32_forward, nogil());
+  m.def("ff_f32_backward", &ff_f32_backward, nogil());
   m.def("norm_fwd", &norm_fwd, nogil());
   m.def("norm_bwd", &norm_bwd, nogil());
   m.def("scan_fwd", &scan_fwd, nogil());
@@ -580,5 +686,6 @@ PYBIND11_MODULE(_native, m) {
   m.def("ff_bias_bwd", &ff_bias_bwd, nogil());
   m.def("head_forward", &head_forward, nogil());
   m.def("head_backward", &head_backward, nogil());
+  m.def("infer_layer", &infer_layer, nogil());
   m.def("column_sum", &column_sum, nogil());
 }

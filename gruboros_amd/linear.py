@@ -280,6 +280,25 @@ def f32_linear(x, w, b=None):
     return y.view(*shape[:-1], w.shape[0])
 
 
+class F32FeedForward(torch.autograd.Function):
+    """Linear -> GELU -> Linear (reference mingru/minLM.py:17-23) for fp32 x [N, D] and fp32 weights and
+    biases, every product on mg_gemm_f32: the first with bias and GELU in its epilogue (the pre-activation
+    kept for the backward), the backward's dy W2 with the GELU gradient in its."""
+
+    @staticmethod
+    def forward(ctx, x, w1, b1, w2, b2):
+        train = any(ctx.needs_input_grad)
+        pre, act, y = native().ff_f32_forward(x, w1, b1.contiguous(), w2, b2.contiguous(), train, stream_of(x))
+        if train:
+            ctx.save_for_backward(x, pre, act, w1, w2)
+        return y
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, pre, act, w1, w2 = ctx.saved_tensors
+        return native().ff_f32_backward(x, pre, act, w1, w2, dy.contiguous(), *ctx.needs_input_grad, stream_of(x))
+
+
 class BF16Linear(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w, b, wb):
@@ -402,6 +421,10 @@ def feed_forward(x, ff):
     """ff = nn.Sequential(Linear, GELU, Linear) applied to x in x's dtype."""
     l1, l2 = ff[0], ff[2]
     if x.dtype == l1.weight.dtype:
+        if (f32_linear_applies(x, l1.weight) and f32_linear_applies(x, l2.weight) and l1.bias is not None and
+                l2.bias is not None and x.shape[-1] == l1.weight.shape[1] and l1.weight.shape[0] == l2.weight.shape[1]):
+            y = F32FeedForward.apply(x.reshape(-1, x.shape[-1]).contiguous(), l1.weight, l1.bias, l2.weight, l2.bias)
+            return y.view(*x.shape[:-1], l2.weight.shape[0])
         return linear(F.gelu(linear(x, l1)), l2)
     if x.dtype != torch.bfloat16 or l1.weight.dtype != torch.float32:
         return l2(F.gelu(l1(x.to(l1.weight.dtype)))).to(x.dtype)  # parameters cast to another dtype

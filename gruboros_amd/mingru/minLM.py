@@ -21,7 +21,7 @@ import torch.nn.functional as F
 from torch import nn
 from torch.nn import Module, ModuleList, RMSNorm
 
-from .. import blocks, decode
+from .. import _lib, blocks, decode
 from .. import scan as scan_errors
 from ..embed import embedding
 from ..linear import feed_forward
@@ -210,6 +210,11 @@ class minLM(Module):
         cd, accurate = self._dtypes()
         x = x.float()  # fp32 residual stream
 
+        if x.is_cuda and self._infer_applies(cd):
+            out = self._trunk_infer(x, prev_hiddens, cd)
+            if out is not None:
+                return out
+
         next_prev_hiddens = []
         prev_hiddens = iter(default(prev_hiddens, []))
 
@@ -244,6 +249,43 @@ class minLM(Module):
         else:
             _, embed, _ = add_rms_norm(x, pending, self.norm.weight, cd)
         return embed, next_prev_hiddens
+
+    def _infer_applies(self, cd):
+        """Whether the forward may run layer by layer in native code: no gradients of any mode, no
+        autocast, no conv and no active dropout, and parameters in the activation dtype."""
+        return (not torch.is_grad_enabled() and cd == self.token_emb.weight.dtype and not torch.is_autocast_enabled()
+                and torch.autograd.forward_ad._current_level < 0
+                and all(conv is None and (dropout is None or not self.training)
+                        for conv, _, _, _, _, dropout in self.layers))
+
+    def _trunk_infer(self, x, prev_hiddens, cd):
+        """_trunk without gradients (generate.py's prompt), one native call per layer; None where a
+        layer's widths are not the kernels' (then _trunk runs op by op)."""
+        native, f32 = _lib.native(), decode._f32
+        B, T, D = x.shape
+        stream = _lib.stream_of(x)
+        x, pending = x.reshape(B * T, D).contiguous(), None
+        prev_hiddens = iter(default(prev_hiddens, []))
+        next_prev_hiddens = []
+        for _, norm, mingru, ff_norm, ff, _ in self.layers:
+            w_hg = mingru.to_hidden_and_gate.weight
+            l1, l2 = ff[0], ff[2]
+            if l1.bias is None or l2.bias is None or w_hg.dtype != cd:
+                return None
+            Di = w_hg.shape[0] // 2
+            h0 = _prep_h0(next(prev_hiddens, None), B, Di, x.device)
+            out = native.infer_layer(x, pending, f32(norm.weight), w_hg,
+                                     mingru.to_out.weight if isinstance(mingru.to_out, nn.Linear) else None,
+                                     f32(ff_norm.weight), l1.weight, f32(l1.bias), l2.weight, f32(l2.bias), h0, B, T,
+                                     scan_errors._workspace(x.device, B, T, Di), stream)
+            if out is None:
+                return None
+            x, pending, h_last = out
+            next_prev_hiddens.append(h_last)
+        x = x.view(B, T, D)
+        if pending is None:
+            return rms_norm(x, self.norm.weight, cd), next_prev_hiddens
+        return add_rms_norm(x, pending.view(B, T, D), self.norm.weight, cd)[1], next_prev_hiddens
 
     def _initialize_weights(self):
         """Reference mingru/minLM.py:157-206: N(0, 0.02/sqrt(dim)) for the embedding,

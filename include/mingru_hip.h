@@ -469,7 +469,7 @@ int mg_split_limbs(const float* x, int64_t ldx, int64_t rows, int cols, int patt
                    void* out, int64_t ldo, void* stream);
 
 /* fp32 matrix product to fp32 accuracy on the bf16 matrix cores:
- *   C[m, n] (=|+=) sum_k A(m, k) B(k, n) (+ bias[n]),  A, B, C and bias fp32,
+ *   C[m, n] (=|+=) epilogue(sum_k A(m, k) B(k, n)),  A, B, C, bias and aux fp32,
  * operand layouts as mg_gemm's (MG_KCONTIG / MG_MNCONTIG, element strides).
  * Each value is split into three bf16 limbs (h + m + l == x) as its tile goes
  * from memory to LDS, and the six limb products through 2^-16 relative are
@@ -477,16 +477,18 @@ int mg_split_limbs(const float* x, int64_t ldx, int64_t rows, int cols, int patt
  * nn.Linear of an fp32 model and its backward (reference mingru/minGRU.py:45,
  * :71, mingru/minLM.py:17-23, :138 in fp32): Y = X W^T + b is (A = X, KCONTIG;
  * B = W, KCONTIG), dX = dY W (KCONTIG; MNCONTIG), dW = dY^T X (MNCONTIG;
- * MNCONTIG). bias nullable. flags: MG_GEMM_ACCUMULATE (no bias; C += ),
- * MG_GEMM_DETERMINISTIC (never split along K). Products whose tiles leave CUs
- * idle are split along K when a workspace of mg_gemm_f32_workspace_bytes(...)
- * bytes (0: never splits), 16-byte aligned, is given (NULL: unsplit); the
- * partials are added in split order, so results repeat bit for bit. N, a
- * K-contiguous operand's K and an MN-contiguous A's M are multiples of 4,
- * leading dimensions too; pointers 16-byte aligned. No size limit of its own. */
+ * MNCONTIG). Epilogues as mg_gemm's: MG_EPI_BIAS; MG_EPI_BIAS_GELU (aux
+ * nullable: receives acc + bias); MG_EPI_GELU_GRAD (C = acc * gelu'(aux)).
+ * flags: MG_GEMM_ACCUMULATE (no epilogue; C +=), MG_GEMM_DETERMINISTIC (never
+ * split along K). Products whose tiles leave CUs idle are split along K when a
+ * workspace of mg_gemm_f32_workspace_bytes(...) bytes (0: never splits),
+ * 16-byte aligned, is given (NULL: unsplit); the partials are added in split
+ * order, so results repeat bit for bit. N, a K-contiguous operand's K and an
+ * MN-contiguous A's M are multiples of 4, leading dimensions too; pointers
+ * 16-byte aligned. No size limit of its own. */
 int mg_gemm_f32(int a_layout, const float* A, int64_t lda, int b_layout, const float* B, int64_t ldb,
-                int M, int N, int K, const float* bias, float* C, int64_t ldc, int flags,
-                void* workspace, size_t workspace_bytes, void* stream);
+                int M, int N, int K, int epilogue, const float* bias, float* aux, int64_t ldaux,
+                float* C, int64_t ldc, int flags, void* workspace, size_t workspace_bytes, void* stream);
 size_t mg_gemm_f32_workspace_bytes(int M, int N, int K, int flags);
 
 /* fp32 -> bf16 with stochastic rounding (as the gradient stores, keyed by the

@@ -811,3 +811,34 @@ def test_hilo_cols_matches_fp64(M, N, K, hc):
     ref = xh @ wh.t()
     err = (out.double().cpu() - ref).abs()
     assert bool((err <= 2.0 ** -8 * ref.abs() + (K + 8) * 2.0 ** -24 * mag)[:, hc:].all()), float(err[:, hc:].max())
+
+
+@pytest.mark.parametrize("N,D,Fw", [(37, 64, 96), (300, 136, 520), (2048, 512, 2048)])
+@pytest.mark.parametrize("deterministic", [False, True])
+def test_f32_feed_forward_matches_fp64(N, D, Fw, deterministic):
+    """F32FeedForward (bias + GELU and the GELU gradient in mg_gemm_f32's epilogues, in the tile store
+    and, where the product is split along K, in the reduction) against float64: output and every
+    gradient within 2e-6 norm-relative, an fp32 product's accumulation error at these K; without
+    gradients the same output bit for bit."""
+    from gruboros_amd.linear import feed_forward
+
+    g = torch.Generator().manual_seed(N + D + Fw)
+    ff = torch.nn.Sequential(torch.nn.Linear(D, Fw), torch.nn.GELU(), torch.nn.Linear(Fw, D)).to(DEV)
+    x = torch.randn(N, D, generator=g).to(DEV).requires_grad_(True)
+    dy = torch.randn(N, D, generator=g).to(DEV)
+    torch.use_deterministic_algorithms(deterministic)
+    try:
+        y = feed_forward(x, ff)
+        y.backward(dy)
+        with torch.no_grad():
+            assert torch.equal(feed_forward(x, ff), y)
+    finally:
+        torch.use_deterministic_algorithms(False)
+    got = [y, x.grad] + [p.grad for p in ff.parameters()]
+    ref = torch.nn.Sequential(torch.nn.Linear(D, Fw), torch.nn.GELU(), torch.nn.Linear(Fw, D)).double()
+    ref.load_state_dict({k: v.double().cpu() for k, v in ff.state_dict().items()})
+    xr = x.detach().double().cpu().requires_grad_(True)
+    yr = ref(xr)
+    yr.backward(dy.double().cpu())
+    errs = [_rel(a, b) for a, b in zip(got, [yr, xr.grad] + [p.grad for p in ref.parameters()])]
+    assert all(e <= 2e-6 for e in errs), errs
