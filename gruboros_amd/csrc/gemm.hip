@@ -184,8 +184,14 @@ struct Loader<R, true, T> {
 // (ds_read_b64_tr_b16): in each group of 16 lanes, lane 4 j + q addresses
 // k-row j, columns 4 q .. 4 q + 3, and lane i receives column i of the 4
 // k-rows. With this h the 16 lanes of a group hit distinct banks, and so do
-// the 32 lanes of two neighbouring groups (4 k-rows x 2 segments).
+// the 32 lanes of two neighbouring groups (4 k-rows x 2 segments). A 64-row
+// tile's k-rows are 128 bytes, four segments, so k-rows r and r + 2 share banks:
+// there h(r) = 2 for the odd pairs of k-rows.
 __device__ __forceinline__ int tr_swz(int kr) { return ((kr & 3) << 1) | ((kr >> 1) & 1); }
+template <int R>
+__device__ __forceinline__ int tr_swz_of(int kr) {
+  return R == 64 ? kr & 2 : tr_swz(kr);
+}
 template <int R, int T>
 struct Loader<R, false, T> {
   static constexpr int kChunksRow = R / 8;                    // 16-byte chunks per k-row
@@ -203,7 +209,7 @@ struct Loader<R, false, T> {
     const int b = wave * kPerWave + i;
     const int chunk = b * 64 + lane;
     const int kr = chunk / kChunksRow, cpos = chunk % kChunksRow;
-    const int m = (((cpos >> 1) ^ tr_swz(kr)) << 4) + ((cpos & 1) << 3);  // tile column stored at this chunk
+    const int m = (((cpos >> 1) ^ tr_swz_of<R>(kr)) << 4) + ((cpos & 1) << 3);  // tile column stored at this chunk
     const uint32_t off = static_cast<uint32_t>(k0 + kr) * o.ld2 + static_cast<uint32_t>(r0 + m) * 2u;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(o.rsrc, (__attribute__((address_space(3))) void*)(stage + b * 64),
                                              16, (r0 + m < rmax && k0 + kr < kmax) ? off : kOutOfRange, 0, 0, 0);
@@ -223,7 +229,7 @@ __device__ __forceinline__ bf16x8 read_frag(const uint4* tile, int row, int s, i
     const int g = lane >> 4, j = (lane >> 2) & 3, q = lane & 3;
     const int kr = 16 * s + 8 * (g >> 1) + j;              // first k-row; the second read is 4 rows on
     const int mc = row + 16 * (g & 1) + 4 * q;
-    const int pos = (((mc >> 4) ^ tr_swz(kr)) << 5) + ((mc & 15) << 1);
+    const int pos = (((mc >> 4) ^ tr_swz_of<R>(kr)) << 5) + ((mc & 15) << 1);
     const char* base = reinterpret_cast<const char*>(tile) + kr * (R * 2) + pos;
     typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
     const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(base));
@@ -441,6 +447,92 @@ __device__ __forceinline__ void mainloop(const Params& p, uint4* smem, uint4* s1
   // the zero-reading loads issued for tile n may still be landing in LDS,
   // which the epilogue reuses
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+}
+
+// The R x R (128, or 64) main loop with four LDS stages, for products that do
+// not give every CU two workgroups of 128 x 128: the loads of k-tile t + 3 go
+// out while tile t is multiplied. With four stages (128 KB at 128 x 128) one
+// workgroup per CU keeps 96 KB in flight, where the two-stage loop needs two
+// workgroups, i.e. twice the splits along K and twice the partials, for 64 KB.
+// The stages are four distinct __shared__ arrays, run in turns of four so each
+// is static (an LDS read then waits only for the loads into its own stage).
+// Same MFMAs in the same order as mainloop's.
+template <int R, bool AK, bool BKM>
+__device__ __forceinline__ void mainloop_deep(const Params& p, uint4* s0, uint4* s1, uint4* s2, uint4* s3, int m0, int n0,
+                                              int kt0, int kt1, f32x16 (&acc)[R / 64][R / 64]) {
+  constexpr int T = 256, MB = R / 64, NB = R / 64, S = BK / 16;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wm = wave >> 1, wn = wave & 1;
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+  const Operand oa = make_operand(p.A, p.lda, p.a_span);
+  const Operand ob = make_operand(p.B, p.ldb, p.b_span);
+  Loader<R, AK, T> la;
+  Loader<R, BKM, T> lb;
+  constexpr int kLoads = decltype(la)::kPerWave + decltype(lb)::kPerWave;  // load instructions per k-tile and wave
+  auto issue_to = [&](int t, uint4* st) __attribute__((always_inline)) {   // tiles past kt1 read as zero
+    const KTile kt = ktile(p, kt0 + t, kt1);
+    la.load(oa, st, m0, p.M, kt.k0, kt.kmax, kt.aofs);
+    lb.load(ob, st + R * 8, n0, p.N, kt.k0, kt.kmax, kt.bofs);
+  };
+  int arow[MB], brow[NB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i) arow[i] = wm * (R / 2) + i * 32;
+#pragma unroll
+  for (int j = 0; j < NB; ++j) brow[j] = wn * (R / 2) + j * 32;
+  issue_to(0, s0);
+  issue_to(1, s1);
+  issue_to(2, s2);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kLoads) : "memory");  // tile 0 has landed
+  __builtin_amdgcn_s_barrier();
+  bf16x8 af[2][MB], bfr[2][NB];
+  auto tile = [&](int t, const uint4* cur, uint4* fill) __attribute__((always_inline)) {
+    issue_to(t + 3, fill);  // fill held tile t - 1, which every wave finished before the last barrier
+    const uint4* Bs = cur + R * 8;
+#pragma unroll
+    for (int i = 0; i < MB; ++i) af[0][i] = read_frag<R, AK>(cur, arow[i], 0, lane);
+#pragma unroll
+    for (int j = 0; j < NB; ++j) bfr[0][j] = read_frag<R, BKM>(Bs, brow[j], 0, lane);
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const int c = s & 1;
+      if (s + 1 < S) {
+#pragma unroll
+        for (int i = 0; i < MB; ++i) af[c ^ 1][i] = read_frag<R, AK>(cur, arow[i], s + 1, lane);
+#pragma unroll
+        for (int j = 0; j < NB; ++j) bfr[c ^ 1][j] = read_frag<R, BKM>(Bs, brow[j], s + 1, lane);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[c][j], af[c][i], acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // tile t + 1 has landed (t + 2 and t + 3 may still fly), this wave's reads of
+    // tile t were consumed by its MFMAs; a bare barrier (a fence would wait for
+    // every load in flight)
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kLoads) : "memory");
+    __builtin_amdgcn_s_barrier();
+  };
+  const int n = kt1 - kt0;
+  int t = 0;
+  for (; t + 3 < n; t += 4) {
+    tile(t, s0, s3);
+    tile(t + 1, s1, s0);
+    tile(t + 2, s2, s1);
+    tile(t + 3, s3, s2);
+  }
+  if (t < n) tile(t, s0, s3);
+  if (t + 1 < n) tile(t + 1, s1, s0);
+  if (t + 2 < n) tile(t + 2, s2, s1);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the zero-reading loads past kt1
   __syncthreads();
 }
 
@@ -1322,7 +1414,7 @@ __device__ __forceinline__ void mainloop_pp(const Params& p, uint4* smem, int m0
 enum CMode { C_STORE = 0, C_ADD = 1, C_SPLIT = 2 };
 
 // One workgroup tile: bx, by stand for blockIdx.x, blockIdx.y of a one-product launch.
-template <int BM, int BN, int WM, int WN, bool AK, bool BKM, int EPI, typename TC, int CMODE>
+template <int BM, int BN, int WM, int WN, bool AK, bool BKM, int EPI, typename TC, int CMODE, bool DEEP = false>
 __device__ __forceinline__ void gemm_tile(const Params& p, int bx, int by) {
   constexpr int MB = BM / WM / 32, NB = BN / WN / 32;  // 32x32 blocks per wave
   constexpr int kStage = (BM + BN) * 8;                 // uint4 per stage
@@ -1330,10 +1422,13 @@ __device__ __forceinline__ void gemm_tile(const Params& p, int bx, int by) {
   // interleaved schedule needs that); 256 x 256 tiles one array of two.
   constexpr bool kW8 = BM == 256 && BN == 256 && WM == 4 && WN == 2;  // mainloop_w8
   constexpr bool kW4M = BM == 256 && BN == 256 && WM == 2 && WN == 2 && EPI != EPI_GELU_GRAD && kUseW4M;
-  constexpr bool kSplit = BM != 256 || WM * WN == 4 || kW8;
+  constexpr bool kSplit = BM != 256 || WM * WN == 4 || kW8;  // two stage objects
   __shared__ uint4 smem[kSplit ? kStage : 2 * kStage];
   __shared__ uint4 smem_b[kSplit ? kStage : 1];
   uint4* const stage1 = kSplit ? smem_b : smem + kStage;
+  static_assert(!DEEP || (BM <= 128 && BM == BN && WM == 2 && WN == 2), "four stages: 128 x 128 or 64 x 64 tiles");
+  __shared__ uint4 smem_c[DEEP ? kStage : 1];
+  __shared__ uint4 smem_d[DEEP ? kStage : 1];
 
   int tm, tn, split;
   if (p.xcd_splits > 0) {
@@ -1351,7 +1446,9 @@ __device__ __forceinline__ void gemm_tile(const Params& p, int bx, int by) {
   const int L = lane & 31, half = lane >> 5;
   f32x16 acc[kW4M ? 1 : MB][kW4M ? 1 : NB];
   f32x4v acc16[kW4M ? 8 : 1][kW4M ? 8 : 1];
-  if constexpr (kW4M)
+  if constexpr (DEEP)
+    mainloop_deep<BM, AK, BKM>(p, smem, smem_b, smem_c, smem_d, m0, n0, kt0, kt1, acc);
+  else if constexpr (kW4M)
     mainloop_w4m<AK, BKM>(p, smem, stage1, m0, n0, kt0, kt1, acc16);
   else if constexpr (BM == 256 && BN == 256 && WM == 2 && WN == 4 && AK && !BKM)
     mainloop_pp<AK, BKM>(p, smem, m0, n0, kt0, kt1, acc);  // both stages in smem (kSplit is false)
@@ -1503,9 +1600,9 @@ __device__ __forceinline__ void gemm_tile(const Params& p, int bx, int by) {
   }
 }
 
-template <int BM, int BN, int WM, int WN, bool AK, bool BKM, int EPI, typename TC, int CMODE>
+template <int BM, int BN, int WM, int WN, bool AK, bool BKM, int EPI, typename TC, int CMODE, bool DEEP>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_kernel(Params p) {
-  gemm_tile<BM, BN, WM, WN, AK, BKM, EPI, TC, CMODE>(p, blockIdx.x, blockIdx.y);
+  gemm_tile<BM, BN, WM, WN, AK, BKM, EPI, TC, CMODE, DEEP>(p, blockIdx.x, blockIdx.y);
 }
 
 // Two K-split products in one launch (the FeedForward's two weight
@@ -2736,10 +2833,10 @@ inline HiloPlan hilo_plan(int M, int N, int K, bool f32, bool whole) {
 // weight gradients (both operands MN-contiguous) of whole 256 x 256 tiles, at
 // least 16 of them, K >= 4096, split along K to about one workgroup per CU, and
 // for the other layouts when that still gives every CU a tile; everything else
-// 128 x 128, split along K (outputs and epilogues that allow it) to about two
-// workgroups per CU. `ysplits` is the split count the launch uses (gridDim.y).
+// 128 x 128, split along K (outputs and epilogues that allow it) to about one
+// workgroup per CU. `ysplits` is the split count the launch uses (gridDim.y).
 struct Plan {
-  bool big;
+  bool big, deep, small;
   int tiles, kt_per_split, ysplits;
 };
 
@@ -2765,20 +2862,28 @@ inline Plan plan(int M, int N, int K, bool ak, bool bk, int c_dtype, int epilogu
   const int64_t tiles = pl.big ? t256 : t128;
   pl.tiles = static_cast<int>(tiles);
   const int nkt = (hilo ? 3 : 1) * ((K + BK - 1) / BK);
-  const int64_t want_wgs = !pl.big ? 2 * kCUs : kCUs;
+  // 64 x 64 tiles (four stages of 16 KB, two workgroups per CU) for short products of few
+  // tiles, whole instead of split along K (us, 2048 x 1024 x 1536 22.0 -> 13.9, 777 x 1024 x 1536 17.1 -> 9.9, weight gradient 1536 x 384 x
+  // 667 13.2 -> 7.2), and for the bias + GELU product,
+  // which is never split and whose erf runs after the tile's MFMAs, 64 values a thread on
+  // 128 x 128 tiles (777 x 1536 x 1024 23.3 -> 11.7, 2048 x 1536 x 1024 24.8 -> 19.7).
+  const int64_t t64 = int64_t((M + 63) / 64) * ((N + 63) / 64);
+  pl.small = !pl.big && !hilo && ((nkt <= 24 && t64 <= 2 * kCUs) || (epilogue == MG_EPI_BIAS_GELU && t128 <= kCUs));
   int splits = 1;
   // fp32 outputs and plain bf16 outputs (no epilogue or a bias, no hi/lo operands; a
   // stochastically rounded gradient among them) split K when the tiles leave CUs idle: partials
   // in fp32, then split_reduce_kernel (fp32) or split_reduce_bf16_kernel (bias added, rounded as
   // the unsplit epilogue would). Hi/lo bf16 products stay whole, equal to mg_gemm_hilo_prefix's
-  // columns. 128 x 128 tiles aim at two workgroups per CU (measured at [1, 2048] chunks of the
-  // d1024 expansion-3 model: 369 -> 351 ms per optimizer step against one; four: 378 ms).
+  // columns. 128 x 128 tiles aim at one workgroup per CU with four LDS stages (pl.deep); two per
+  // CU with two stages each, i.e. twice the partials, measured (us) 23.9 against 15.6 at 2048 x
+  // 1536 x 1024, 24.9 against 22.2 at 2048 x 1024 x 1536, 22.8 against 19.2 at 777 x 1024 x 3072.
   const bool split_ok = c_dtype == MG_F32 || (c_dtype == MG_BF16 && !hilo);
   const bool epi_ok = epilogue == MG_EPI_NONE || (epilogue == MG_EPI_BIAS && c_dtype == MG_BF16 && !hilo);
-  if (epi_ok && split_ok && tiles < want_wgs && !deterministic)
-    splits = static_cast<int>(std::min<int64_t>(std::max<int64_t>(want_wgs / tiles, 1), std::max(nkt / 4, 1)));
+  if (epi_ok && split_ok && tiles < kCUs && !deterministic && !pl.small)
+    splits = static_cast<int>(std::min<int64_t>(std::max<int64_t>(kCUs / tiles, 1), std::max(nkt / 4, 1)));
   pl.kt_per_split = std::max((nkt + splits - 1) / splits, 1);
   pl.ysplits = std::max((nkt + pl.kt_per_split - 1) / pl.kt_per_split, 1);
+  pl.deep = !pl.big && tiles * pl.ysplits <= kCUs;
   return pl;
 }
 
@@ -2798,15 +2903,17 @@ int launch(const Params& p0, const Plan& pl, hipStream_t stream) {
   // K-split products run as a 1-D grid laid out by split_tile_of when it can
   // (MG_GEMM_XCD_SPLIT=0 in the environment turns that off)
   const char* e = getenv("MG_GEMM_XCD_SPLIT");
-  if (CMODE == C_SPLIT && (tiles * pl.ysplits) % 8 == 0 && !(e && atoi(e) == 0)) {
-    p.xcd_splits = pl.ysplits;
-    hipLaunchKernelGGL((gemm_kernel<BM, BN, WM, WN, AK, BKM, EPI, TC, CMODE>), dim3(tiles * pl.ysplits), dim3(64 * WM * WN),
-                       0, stream, p);
-  } else {
-    p.xcd_splits = 0;
-    hipLaunchKernelGGL((gemm_kernel<BM, BN, WM, WN, AK, BKM, EPI, TC, CMODE>), dim3(tiles, pl.ysplits),
-                       dim3(64 * WM * WN), 0, stream, p);
+  const bool xcd = CMODE == C_SPLIT && (tiles * pl.ysplits) % 8 == 0 && !(e && atoi(e) == 0);
+  p.xcd_splits = xcd ? pl.ysplits : 0;
+  const dim3 grid = xcd ? dim3(tiles * pl.ysplits) : dim3(tiles, pl.ysplits);
+  if constexpr (BM <= 128) {
+    if (BM == 64 || pl.deep) {
+      hipLaunchKernelGGL((gemm_kernel<BM, BN, WM, WN, AK, BKM, EPI, TC, CMODE, true>), grid, dim3(64 * WM * WN), 0, stream, p);
+      return check_launch("mg_gemm");
+    }
   }
+  if constexpr (BM > 64)
+    hipLaunchKernelGGL((gemm_kernel<BM, BN, WM, WN, AK, BKM, EPI, TC, CMODE, false>), grid, dim3(64 * WM * WN), 0, stream, p);
   return check_launch("mg_gemm");
 }
 
@@ -2883,6 +2990,29 @@ int dispatch_epi(const Params& p, const Plan& pl, int epi, int c_dtype, hipStrea
     if (epi == EPI_SR) return launch<BM, BN, WM, WN, AK, BKM, EPI_SR, bf16_t, C_STORE>(p, pl, s);
   }
   return fail(MG_ERR_ARG, "mg_gemm: epilogue %d not available for this output dtype", epi);
+}
+
+// 64 x 64 tiles: never split.
+template <bool AK, bool BKM>
+int dispatch_small_epi(const Params& p, const Plan& pl, int epi, int c_dtype, hipStream_t s) {
+  if (c_dtype == MG_F32) {
+    if (p.accumulate) return launch<64, 64, 2, 2, AK, BKM, EPI_NONE, float, C_ADD>(p, pl, s);
+    if (epi == EPI_NONE) return launch<64, 64, 2, 2, AK, BKM, EPI_NONE, float, C_STORE>(p, pl, s);
+    if (epi == EPI_BIAS) return launch<64, 64, 2, 2, AK, BKM, EPI_BIAS, float, C_STORE>(p, pl, s);
+  } else {
+    if (epi == EPI_NONE) return launch<64, 64, 2, 2, AK, BKM, EPI_NONE, bf16_t, C_STORE>(p, pl, s);
+    if (epi == EPI_BIAS) return launch<64, 64, 2, 2, AK, BKM, EPI_BIAS, bf16_t, C_STORE>(p, pl, s);
+    if (epi == EPI_BIAS_GELU) return launch<64, 64, 2, 2, AK, BKM, EPI_BIAS_GELU, bf16_t, C_STORE>(p, pl, s);
+    if (epi == EPI_GELU_GRAD) return launch<64, 64, 2, 2, AK, BKM, EPI_GELU_GRAD, bf16_t, C_STORE>(p, pl, s);
+    if (epi == EPI_SR) return launch<64, 64, 2, 2, AK, BKM, EPI_SR, bf16_t, C_STORE>(p, pl, s);
+  }
+  return fail(MG_ERR_ARG, "mg_gemm: epilogue %d not available for this output dtype", epi);
+}
+inline int dispatch_small(const Params& p, const Plan& pl, bool ak, bool bk, int epi, int c_dtype, hipStream_t s) {
+  if (ak && bk) return dispatch_small_epi<true, true>(p, pl, epi, c_dtype, s);
+  if (ak && !bk) return dispatch_small_epi<true, false>(p, pl, epi, c_dtype, s);
+  if (!ak && !bk) return dispatch_small_epi<false, false>(p, pl, epi, c_dtype, s);
+  return dispatch_small_epi<false, true>(p, pl, epi, c_dtype, s);
 }
 
 // Whether a product meets the pipelined loops' no-mask conditions.
@@ -3234,7 +3364,8 @@ extern "C" int mg_gemm(int a_layout, const void* A, int64_t lda, int b_layout, c
   }
   p.accumulate = accumulate ? 1 : 0;
   const int epi = (flags & MG_GEMM_STOCHASTIC) && epilogue == MG_EPI_NONE ? gemm::EPI_SR : epilogue;
-  const int rc = pl.big ? gemm::dispatch_layout<256, 256>(p, pl, ak, bk, epi, c_dtype, s)
+  const int rc = pl.small ? gemm::dispatch_small(p, pl, ak, bk, epi, c_dtype, s)
+                 : pl.big ? gemm::dispatch_layout<256, 256>(p, pl, ak, bk, epi, c_dtype, s)
                         : gemm::dispatch_layout<128, 128>(p, pl, ak, bk, epi, c_dtype, s);
   if (rc || pl.ysplits <= 1) return rc;
   const int64_t n4 = int64_t(M) * (N / 4);
