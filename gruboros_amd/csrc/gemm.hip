@@ -2879,7 +2879,10 @@ inline Plan plan(int M, int N, int K, bool ak, bool bk, int c_dtype, int epilogu
   // 1536 x 1024, 24.9 against 22.2 at 2048 x 1024 x 1536, 22.8 against 19.2 at 777 x 1024 x 3072.
   const bool split_ok = c_dtype == MG_F32 || (c_dtype == MG_BF16 && !hilo);
   const bool epi_ok = epilogue == MG_EPI_NONE || (epilogue == MG_EPI_BIAS && c_dtype == MG_BF16 && !hilo);
-  if (epi_ok && split_ok && tiles < kCUs && !deterministic && !pl.small)
+  if (!pl.big && !pl.small && !hilo && epi_ok && split_ok && !deterministic && t64 <= kCUs) {
+    pl.small = true;  // longer ones split to two workgroups per CU (777 x 1024 x 3072 19.7 -> 16.3 us)
+    splits = static_cast<int>(std::min<int64_t>(2 * kCUs / t64, nkt / 6));
+  } else if (epi_ok && split_ok && tiles < kCUs && !deterministic && !pl.small)
     splits = static_cast<int>(std::min<int64_t>(std::max<int64_t>(kCUs / tiles, 1), std::max(nkt / 4, 1)));
   pl.kt_per_split = std::max((nkt + splits - 1) / splits, 1);
   pl.ysplits = std::max((nkt + pl.kt_per_split - 1) / pl.kt_per_split, 1);
@@ -2992,9 +2995,9 @@ int dispatch_epi(const Params& p, const Plan& pl, int epi, int c_dtype, hipStrea
   return fail(MG_ERR_ARG, "mg_gemm: epilogue %d not available for this output dtype", epi);
 }
 
-// 64 x 64 tiles: never split.
 template <bool AK, bool BKM>
 int dispatch_small_epi(const Params& p, const Plan& pl, int epi, int c_dtype, hipStream_t s) {
+  if (pl.ysplits > 1) return launch<64, 64, 2, 2, AK, BKM, EPI_NONE, float, C_SPLIT>(p, pl, s);
   if (c_dtype == MG_F32) {
     if (p.accumulate) return launch<64, 64, 2, 2, AK, BKM, EPI_NONE, float, C_ADD>(p, pl, s);
     if (epi == EPI_NONE) return launch<64, 64, 2, 2, AK, BKM, EPI_NONE, float, C_STORE>(p, pl, s);
