@@ -87,7 +87,7 @@ class MinGRUBlock(torch.autograd.Function):
                               bf16_copy(w_to) if w_to is not None else None)
         ctx.dims = (B, T, D, Di)
         ctx.has_pending = pending is not None
-        if ckpt is not None:  # expansion 1: x_next = x1 + h, h kept as checkpoints
+        if w_to is None and ckpt is not None:  # expansion 1: x_next = x1 + h, h kept as checkpoints
             return out, None, h_last
         x1 = x_out.view(B, T, D) if x_out is not None else x.view_as(x)
         return x1, out, h_last

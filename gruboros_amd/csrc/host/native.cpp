@@ -438,12 +438,17 @@ GruOut gru_forward(const Tensor& x, const Opt& pending, const Tensor& w_norm, co
     auto [x2, last, ckpt] = scan_fwd_residual_hg(s, h0, x1.view({B, T, D}), ws, stream);
     return {x_out, rstd, *pair, hg, std::nullopt, last, x2, std::nullopt, ckpt};
   }
-  auto [h, last, none] = scan_fwd_hg(s, h0, at::kFloat, false, ws, x, stream);
-  if (!to_pair) return {x_out, rstd, *pair, hg, h, last, h, std::nullopt, std::nullopt};
-  Tensor h_pair = make({N, 2 * Di}, at::kBFloat16, x), out = make({N, D}, at::kFloat, x);
-  check(mg_split_hilo(fp(h), Di, N, Di, ptr(h_pair), 2 * Di, st(stream)), "mg_split_hilo");
+  if (!to_pair) {
+    auto [h, last, none] = scan_fwd_hg(s, h0, at::kFloat, false, ws, x, stream);
+    return {x_out, rstd, *pair, hg, h, last, h, std::nullopt, std::nullopt};
+  }
+  Tensor h_pair = make({N, 2 * Di}, at::kBFloat16, x), last = make({B, 1, Di}, at::kFloat, x);
+  Tensor out = make({N, D}, at::kFloat, x), ckpt = make({static_cast<int64_t>(mg_scan_ckpt_elems(B, T, Di))}, at::kFloat, x);
+  check(mg_scan_fwd_pair(s.hidden, s.gate, s.sb, s.ld, fp(h0), ptr(h_pair), fp(last), fp(ckpt), B, T, Di, ptr(ws), ws.numel(),
+                         st(stream)),
+        "mg_scan_fwd_pair");
   linear_fwd_hilo(mat(h_pair, "h_pair"), mat(*to_pair, "to_pair"), N, D, Di, MG_F32, mat(out, "out"), x, stream);
-  return {x_out, rstd, *pair, hg, h, last, out.view({B, T, D}), h_pair, std::nullopt};
+  return {x_out, rstd, *pair, hg, std::nullopt, last, out.view({B, T, D}), h_pair, ckpt};
 }
 
 // MinGRUBlock.backward. dx1: the gradient of the residual stream [B, T, D] or none; dout: of
@@ -459,7 +464,7 @@ GruGrads gru_backward(const Tensor& xn, const Tensor& w_norm, const Tensor& rstd
   const int64_t N = xn.size(0), D = xn.size(1), Di = hg.size(1) / 2;
   Opt dh, dW_to, dW_hg, dh0;
   Tensor dob;
-  if (ckpt) {
+  if (ckpt && !h_pair) {
     dh = dx1;  // x_next = x1 + h: h and the residual get the same gradient
   } else if (dout && h_pair) {
     const Tensor d = dout->reshape({N, D}).to(at::kFloat).contiguous();

@@ -299,13 +299,19 @@ __device__ __forceinline__ int scan_runs(RunMaps<kSubs>& m, int s, int cl, f4 A,
 // kRes: the output is res + h (fp32, res with the output's strides): the scan
 // state joins the residual stream here, and h itself is kept only as the fp32
 // checkpoints the backward rebuilds it from.
-template <typename Tin, typename Tout, bool kNT, bool kRes = false>
+// kPair: the output is h as bf16 hi/lo pairs, hi = bf16(h) at the output's
+// element and lo = bf16(h - hi) g.Di columns on: to_out's operand, written here
+// instead of an fp32 h that a pass of its own read and split (2048 x 3072: the
+// scan 18.5 -> 20.6 us, the split's 10 us gone; the block's forward and backward
+// 284 -> 274). Plain stores: the product reads them at once.
+template <typename Tin, typename Tout, bool kNT, bool kRes = false, bool kPair = false>
 __global__ __launch_bounds__(kChLanes * kFwdSubs) void scan_fwd_kernel(
     const Tin* __restrict__ hidden, const Tin* __restrict__ gate, int64_t in_sb, int64_t in_ld,
     const float* __restrict__ h0, Tout* __restrict__ hout, int64_t out_sb, int64_t out_ld,
     float* __restrict__ h_last, float* __restrict__ ckpt, Geometry g, WsHeader* __restrict__ hdr,
     uint32_t* __restrict__ counters, uint64_t* __restrict__ status, const float* __restrict__ res) {
   static_assert(!kRes || sizeof(Tout) == 4, "the residual sum is fp32");
+  static_assert(!kPair || (!kRes && sizeof(Tout) == 2), "pairs are bf16");
   constexpr int kSubs = kFwdSubs, kRows = kFwdRows;
   __shared__ uint32_t s_ticket;
   __shared__ RunMaps<kSubs> s_maps;
@@ -403,6 +409,14 @@ __global__ __launch_bounds__(kChLanes * kFwdSubs) void scan_fwd_kernel(
 #pragma unroll
         for (int j = 0; j < kVec; ++j) o.v[j] = rv[i % kHalf].v[j] + h.v[j];
         if (kFull || t0 + i < g.T) io4<Tout>::store_nt(ob + i * old, o);
+      } else if constexpr (kPair) {
+        f4 lo;
+#pragma unroll
+        for (int j = 0; j < kVec; ++j) lo.v[j] = h.v[j] - bf16_to_f32(f32_to_bf16(h.v[j]));
+        if (kFull || t0 + i < g.T) {
+          io4<Tout>::store(ob + i * old, h);
+          io4<Tout>::store(ob + i * old + g.Di, lo);
+        }
       } else {
         if (kFull || t0 + i < g.T) io4<Tout>::store_nt(ob + i * old, h);
       }
@@ -724,11 +738,13 @@ constexpr int64_t kFwdNtBytes = int64_t(512) << 20;
 template <typename Tin, typename Tout>
 void launch_fwd(const void* hidden, const void* gate, int64_t in_sb, int64_t in_ld, const float* h0, void* h,
                 int64_t out_sb, int64_t out_ld, float* h_last, float* ckpt, const Geometry& g, void* ws,
-                hipStream_t st, const float* res = nullptr) {
+                hipStream_t st, const float* res = nullptr, bool pair = false) {
   const bool nt = 2 * int64_t(sizeof(Tin)) * g.B * g.T * g.Di > kFwdNtBytes;
   auto kern = nt ? scan_fwd_kernel<Tin, Tout, true> : scan_fwd_kernel<Tin, Tout, false>;
   if constexpr (sizeof(Tout) == 4) {
     if (res) kern = nt ? scan_fwd_kernel<Tin, Tout, true, true> : scan_fwd_kernel<Tin, Tout, false, true>;
+  } else {
+    if (pair) kern = nt ? scan_fwd_kernel<Tin, Tout, true, false, true> : scan_fwd_kernel<Tin, Tout, false, false, true>;
   }
   hipLaunchKernelGGL(kern, dim3(g.ncb * g.ntiles), dim3(kChLanes * kFwdSubs), 0, st,
                      static_cast<const Tin*>(hidden), static_cast<const Tin*>(gate), in_sb, in_ld, h0,
@@ -928,6 +944,21 @@ extern "C" int mg_scan_fwd(int in_dtype, const void* hidden, const void* gate, i
     return rc;
   return scan::fwd_launch(fn, in_dtype, hidden, gate, in_sb, in_ld, h0, out_dtype, h, out_sb, out_ld, h_last, ckpt, g,
                           workspace, stream);
+}
+
+extern "C" int mg_scan_fwd_pair(const void* hidden, const void* gate, int64_t in_sb, int64_t in_ld, const float* h0, void* pair,
+                                float* h_last, float* ckpt, int B, int T, int Di, void* workspace, size_t workspace_bytes,
+                                void* stream) {
+  const char* fn = "mg_scan_fwd_pair";
+  scan::Geometry g;
+  if (!ckpt) return fail(MG_ERR_ARG, "%s: ckpt is required (the backward rebuilds h from it)", fn);
+  const int64_t ld = 2 * int64_t(Di), sb = ld * T;
+  if (int rc = scan::fwd_check(fn, MG_BF16, hidden, gate, in_sb, in_ld, h0, MG_BF16, pair, sb, ld, h_last, ckpt, B, T, Di,
+                               workspace, workspace_bytes, 0, g))
+    return rc;
+  scan::launch_fwd<bf16_t, bf16_t>(hidden, gate, in_sb, in_ld, h0, pair, sb, ld, h_last, ckpt, g, workspace,
+                                   static_cast<hipStream_t>(stream), nullptr, true);
+  return check_launch(fn);
 }
 
 extern "C" int mg_scan_fwd_residual(int in_dtype, const void* hidden, const void* gate, int64_t in_sb,

@@ -143,6 +143,15 @@ int mg_scan_fwd_residual(int in_dtype, const void* hidden, const void* gate, int
                          float* h_last, float* ckpt, int B, int T, int Di, void* workspace,
                          size_t workspace_bytes, void* stream);
 
+/* mg_scan_fwd for bf16 inputs with h written as dense bf16 hi/lo pairs
+ * [B, T, 2 Di] (row: Di values hi = bf16(h), then Di values lo = bf16(h - hi)),
+ * mg_split_hilo's form and to_out's operand (reference mingru/minGRU.py:66-71);
+ * h itself is kept as fp32 checkpoints (ckpt, required), from which mg_scan_bwd
+ * (h = NULL and this ckpt) rebuilds it. */
+int mg_scan_fwd_pair(const void* hidden, const void* gate, int64_t in_sb, int64_t in_ld, const float* h0,
+                     void* pair, float* h_last, float* ckpt, int B, int T, int Di, void* workspace,
+                     size_t workspace_bytes, void* stream);
+
 /* Allocation-free mg_scan_fwd. No counterpart in the reference: it is for
  * callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc). Same arguments and

@@ -368,3 +368,33 @@ def test_residual_scan_matches_scan_plus_add(B, T, Di, with_h0, dtype):
         tol = TOL[dtype]
         assert _rel_norm(g_ck[..., :Di].float().cpu(), ref[2]) <= tol
         assert _rel_norm(g_ck[..., Di:].float().cpu(), ref[3]) <= tol
+
+
+@pytest.mark.parametrize("B,T,Di,with_h0", [(1, 1, 8, True), (2, 7, 64, False), (1, 129, 72, True), (3, 300, 264, True)])
+def test_pair_scan_matches_scan_and_split(B, T, Di, with_h0):
+    """mg_scan_fwd_pair (h as bf16 hi/lo pairs, reference mingru/minGRU.py:66-71) equals mg_scan_fwd's
+    fp32 h put through mg_split_hilo, bit for bit, with the same h_last, and its checkpoints are
+    h at every eighth step to fp32 rounding (2^-20 of the state's size)."""
+    from gruboros_amd import _lib
+    from gruboros_amd import scan as S
+    from gruboros_amd.gemm import split_hilo
+
+    g = torch.Generator().manual_seed(B + T + Di)
+    hg = torch.randn(B, T, 2 * Di, generator=g).to(torch.bfloat16).to(DEV)
+    h0 = torch.rand(B, Di, generator=g).to(DEV) if with_h0 else None
+    h, last, _ = S._launch_fwd(hg[..., :Di], hg[..., Di:], h0, torch.float32)
+    L = _lib.lib()
+    pair = torch.zeros(B * T, 2 * Di, dtype=torch.bfloat16, device=DEV)
+    last2 = torch.zeros(B, 1, Di, device=DEV)
+    ckpt = torch.zeros(L.mg_scan_ckpt_elems(B, T, Di), device=DEV)
+    ws = S._workspace(hg.device, B, T, Di)
+    _lib.check(L.mg_scan_fwd_pair(hg.data_ptr(), hg.data_ptr() + 2 * Di, T * 2 * Di, 2 * Di, _lib.ptr(h0), pair.data_ptr(),
+                                  last2.data_ptr(), ckpt.data_ptr(), B, T, Di, ws.data_ptr(), ws.numel(),
+                                  _lib.stream_of(hg)), "mg_scan_fwd_pair")
+    assert torch.equal(pair.view(torch.int16), split_hilo(h.view(B * T, Di)).view(torch.int16))
+    assert torch.equal(last, last2)
+    n = T // 8
+    if n:
+        c = ckpt.view(-1, B, Di)[:n]
+        ref = h[:, 7:8 * n:8].transpose(0, 1)
+        assert float((c - ref).abs().max()) <= 2.0 ** -20 * float(ref.abs().max())
