@@ -215,25 +215,65 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(Args a) {
   T* s_in = reinterpret_cast<T*>(lds);  // [BP][K]
   const T* W = static_cast<const T*>(a.W);
   __shared__ float s_part[kWaves][BP];
-  __shared__ float s_rstd[BP];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int K = a.K;
 
-  // 0. this wave's weight rows (MINGRU: rows d and D+d, hidden and gate of
-  // channel d), requested before anything else so that their latency
-  // overlaps the norm prologue
   const int g = blockIdx.x * kWaves + wave;  // row group
   int rows[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) rows[r] = MODE == MINGRU ? g + r * a.Di : g * R + r;
   const bool active = rows[0] < (MODE == MINGRU ? a.Di : a.rows);
+
+  // 0. Every load of the step is requested before the first wait. A wave's
+  // loads return in order, so a wait for one is a wait for all before it:
+  // first come the input rows and the norm weight, which the prologue waits
+  // for, with the weight rows behind them in flight during the prologue, its
+  // barriers and its LDS traffic; last the epilogue's own operands (state,
+  // bias, residual value), whose latency would otherwise follow the dot
+  // products. A step is bound by this one chain of latencies, not by its
+  // bytes. Against weights requested first and the norm weight and epilogue
+  // operands only where they are used, bf16, us a token: d1024 expansion 3
+  // ff_mult 1.5, 12 layers, batch 1 224 -> 184; 6 layers, batch 8 167 -> 149;
+  // d2048 expansion 3 ff_mult 4, 6 layers, batch 4 315 -> 284. Rows and columns past the end are clamped, so that nothing
+  // branches between the loads; what they return is not used.
+
+  // input rows: staged 16-byte pieces (the first kBatch of each thread), or
+  // columns 4 (tid + 256 q) .. +3 of the B rows and of the norm weight
+  constexpr int kPer16 = 16 / static_cast<int>(sizeof(T));  // elements per 16 bytes
+  constexpr int kPieces = (BP * NC * 512 / kPer16 + kThreads - 1) / kThreads;
+  constexpr int kBatch = kPieces < 8 ? kPieces : 8;
+  static_assert(kStagedInput || CPT % 4 == 0, "whole 4-column groups per thread");
+  constexpr int Q = kStagedInput ? 1 : CPT / 4;
+  const int row16 = K / kPer16, n16 = BP * row16;
+  const T* act = static_cast<const T*>(a.act);
+  auto piece = [&](int i) {
+    const int b = BP == 1 ? 0 : i / row16, c16 = BP == 1 ? i : i % row16;
+    return (i < n16 && b < a.B) ? *reinterpret_cast<const uint4*>(act + static_cast<int64_t>(b) * K + c16 * kPer16)
+                                : make_uint4(0, 0, 0, 0);
+  };
+  uint4 staged[kBatch];
+  f4 xin[BP][Q], nw[Q];
+  if constexpr (kStagedInput) {
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) staged[u] = piece(u * kThreads + tid);
+  } else {
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const int c = min(4 * (tid + q * kThreads), K - 4);
+#pragma unroll
+      for (int b = 0; b < BP; ++b) xin[b][q] = stream4_at<T, SRC>(a, min(b, a.B - 1), c);
+      nw[q] = io4<float>::load(a.norm_w + c);
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);  // the order of requests stands
+
+  // this wave's weight rows (MINGRU: rows d and Di + d, hidden and gate of
+  // channel d)
   Vec8<T> wv[NC][R];
 #pragma unroll
   for (int c = 0; c < NC; ++c)
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      // clamped, unconditional loads (nothing branches between them); rows
-      // past the end are never used, chunks past K are skipped below
       const int k0 = min(c * 512 + lane * 8, K - 8);
       const int row = active ? rows[r] : 0;
 #pragma unroll
@@ -241,37 +281,41 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(Args a) {
         wv[c][r].q[j] = reinterpret_cast<const uint4*>(W + static_cast<int64_t>(row) * K + k0)[j];
     }
 
-  // 1. the B input rows, as bf16, into LDS (rows B..BP-1 zero)
+  // the epilogue's operands: lane group idx holds value (er, eb) after the sums
+  constexpr int N = R * BP;
+  constexpr int kCopies = 64 / N;
+  const int idx = lane / kCopies, er = idx / BP, eb = idx % BP;
+  const int b_at = min(eb, a.B - 1), row_at = active ? rows[0] : 0;
+  float h_prev = 0.0f, x_at = 0.0f, bias_at = 0.0f;
+  if constexpr (MODE == MINGRU) {
+    h_prev = a.state[static_cast<int64_t>(b_at) * a.Di + row_at];
+    if (!a.h_out) x_at = stream_at<T, SRC>(a, b_at, row_at);
+  } else if constexpr (MODE == TO_OUT) {
+    x_at = stream_at<T, SRC>(a, b_at, row_at);
+  } else if constexpr (MODE == FF1 || MODE == FF2) {
+    bias_at = Elem<T>::get(static_cast<const T*>(a.bias), row_at + er);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
+  // 1. the B input rows, in the element type, into LDS (rows B..BP-1 zero)
   if constexpr (kStagedInput) {
-    // kBatch 16-byte loads per thread in flight before their LDS stores (a
-    // load-store pair per iteration would wait out one memory latency each)
-    constexpr int kBatch = 8;
-    constexpr int kPer16 = 16 / static_cast<int>(sizeof(T));  // elements per 16 bytes
-    const int n16 = BP * (K / kPer16);
-    const T* act = static_cast<const T*>(a.act);
-    for (int i0 = 0; i0 < n16; i0 += kBatch * kThreads) {
-      uint4 v[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const int i = u * kThreads + tid;
+      if (i < n16) reinterpret_cast<uint4*>(s_in)[i] = staged[u];
+    }
+    for (int i0 = kBatch * kThreads; i0 < n16; i0 += kBatch * kThreads) {
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) staged[u] = piece(i0 + u * kThreads + tid);
 #pragma unroll
       for (int u = 0; u < kBatch; ++u) {
         const int i = i0 + u * kThreads + tid;
-        const int b = i / (K / kPer16), c16 = i % (K / kPer16);
-        v[u] = make_uint4(0, 0, 0, 0);
-        if (i < n16 && b < a.B)
-          v[u] = *reinterpret_cast<const uint4*>(act + static_cast<int64_t>(b) * K + c16 * kPer16);
-      }
-#pragma unroll
-      for (int u = 0; u < kBatch; ++u) {
-        const int i = i0 + u * kThreads + tid;
-        if (i < n16) reinterpret_cast<uint4*>(s_in)[i] = v[u];
+        if (i < n16) reinterpret_cast<uint4*>(s_in)[i] = staged[u];
       }
     }
   } else {
-    // RMSNorm over D = K: the rows are read once into registers (columns
-    // 4 (tid + 256 q) .. +3 in one 16-byte load per row and q), the sum of
-    // squares reduced over the workgroup, then y = x r w goes to LDS
-    static_assert(CPT % 4 == 0, "whole 4-column groups per thread");
-    constexpr int Q = CPT / 4;
-    float xr[BP][CPT];
+    // RMSNorm over D = K: the sum of squares reduced over the workgroup, then
+    // y = x r w goes to LDS
     float ss[BP];
 #pragma unroll
     for (int b = 0; b < BP; ++b) {
@@ -279,11 +323,10 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(Args a) {
 #pragma unroll
       for (int q = 0; q < Q; ++q) {
         const int c = 4 * (tid + q * kThreads);
-        const f4 x = stream4_at<T, SRC>(a, min(b, a.B - 1), min(c, K - 4));  // unconditional load
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          xr[b][4 * q + e] = (b < a.B && c < K) ? x.v[e] : 0.0f;
-          ss[b] += xr[b][4 * q + e] * xr[b][4 * q + e];
+          xin[b][q].v[e] = (b < a.B && c < K) ? xin[b][q].v[e] : 0.0f;
+          ss[b] += xin[b][q].v[e] * xin[b][q].v[e];
         }
       }
     }
@@ -293,23 +336,23 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(Args a) {
       if (lane % (64 / BP) == 0) s_part[wave][lane / (64 / BP)] = s;
     }
     __syncthreads();
-    if (tid < BP) {
+    float rstd[BP];
+#pragma unroll
+    for (int b = 0; b < BP; ++b) {
       float s = 0.0f;
 #pragma unroll
-      for (int w = 0; w < kWaves; ++w) s += s_part[w][tid];
-      s_rstd[tid] = __builtin_amdgcn_rsqf(s / static_cast<float>(K) + a.eps);
+      for (int w = 0; w < kWaves; ++w) s += s_part[w][b];
+      rstd[b] = __builtin_amdgcn_rsqf(s / static_cast<float>(K) + a.eps);
     }
-    __syncthreads();
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
       const int c = 4 * (tid + q * kThreads);
       if (c < K) {
-        const f4 w = io4<float>::load(a.norm_w + c);
 #pragma unroll
         for (int b = 0; b < BP; ++b) {
           f4 y;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) y.v[e] = xr[b][4 * q + e] * s_rstd[b] * w.v[e];
+          for (int e = 0; e < 4; ++e) y.v[e] = xin[b][q].v[e] * rstd[b] * nw[q].v[e];
           Elem<T>::store4(s_in + b * K + c, y);
         }
       }
@@ -361,7 +404,6 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(Args a) {
       }
     }
   }
-  constexpr int N = R * BP;
   float flat[N];
 #pragma unroll
   for (int r = 0; r < R; ++r)
@@ -369,50 +411,49 @@ __global__ __launch_bounds__(kThreads) void decode_kernel(Args a) {
     for (int b = 0; b < BP; ++b) flat[r * BP + b] = acc[r][b];
   const float sum = wave_sum_n<N>(flat);
 
-  // 3. epilogue: the first lane holding value (r, b) = (idx / BP, idx % BP)
-  constexpr int kCopies = 64 / N;
-  const int idx = lane / kCopies, r = idx / BP, b = idx % BP;
+  // 3. epilogue: the first lane holding value (er, eb)
   if (MODE == MINGRU) {
     // hidden (r = 0) and gate (r = 1) of one batch row are 32 lanes apart
     const float other = __shfl_xor(sum, 32, 64);
-    if (lane % kCopies || r != 0 || b >= a.B) return;
-    const int d = g;
+    if (lane % kCopies || er != 0 || eb >= a.B) return;
     const float hid = Elem<T>::round(sum), gate = Elem<T>::round(other);
     float coef, v;
     fwd_coeffs(gate, hid, coef, v);
-    float* st = a.state + static_cast<int64_t>(b) * a.Di + d;
-    const float h = coef * *st + v;
-    *st = h;
-    if (a.h_out) Elem<T>::put(static_cast<T*>(a.h_out), static_cast<int64_t>(b) * a.Di + d, h);
-    else a.x_out[static_cast<int64_t>(b) * a.D + d] = stream_at<T, SRC>(a, b, d) + h;
+    const int64_t si = static_cast<int64_t>(eb) * a.Di + g;
+    const float h = coef * h_prev + v;
+    a.state[si] = h;
+    if (a.h_out) Elem<T>::put(static_cast<T*>(a.h_out), si, h);
+    else a.x_out[static_cast<int64_t>(eb) * a.D + g] = x_at + h;
     return;
   }
-  if (lane % kCopies || b >= a.B) return;
+  if (lane % kCopies || eb >= a.B) return;
   if constexpr (MODE == TO_OUT) {
-    const int d = rows[0] + r;
-    a.x_out[static_cast<int64_t>(b) * a.D + d] = stream_at<T, SRC>(a, b, d) + sum;
+    a.x_out[static_cast<int64_t>(eb) * a.D + rows[0] + er] = x_at + sum;
     return;
   }
   T* o = static_cast<T*>(a.out);
-  const int64_t oi = static_cast<int64_t>(b) * a.rows + rows[0] + r;
+  const int64_t oi = static_cast<int64_t>(eb) * a.rows + rows[0] + er;
   if constexpr (MODE == FF1) {
-    Elem<T>::put(o, oi, gelu(Elem<T>::round(sum + Elem<T>::get(static_cast<const T*>(a.bias), rows[0] + r))));
+    Elem<T>::put(o, oi, gelu(Elem<T>::round(sum + bias_at)));
   } else if constexpr (MODE == FF2) {
-    Elem<T>::put(o, oi, sum + Elem<T>::get(static_cast<const T*>(a.bias), rows[0] + r));
+    Elem<T>::put(o, oi, sum + bias_at);
   } else {
     Elem<T>::put(o, oi, sum);
   }
 }
 
-// The staged-input modes (FF2, TO_OUT) take K <= 8192 (NC 8 up to 4096, else
-// 16); the norm modes K = D <= 2048 (NC 2 up to 1024, else 4). Every wave's
-// lane covers its chunks with K <= 512 NC, which check_shape guarantees. fp32
-// rows take twice the LDS, so at batch 5-8 an fp32 staged row is at most 4096
-// long (the 16-chunk variant is not built there).
+// The staged-input modes (FF2, TO_OUT) take K <= 8192 (NC 4 up to 2048, 8 up to
+// 4096, else 16: a chunk past K costs a load whose value is not used); the norm
+// modes K = D <= 2048 (NC 2 up to 1024, else 4). Every wave's lane covers its
+// chunks with K <= 512 NC, which check_shape guarantees. fp32 rows take twice
+// the LDS, so at batch 5-8 an fp32 staged row is at most 4096 long (the
+// 16-chunk variant is not built there).
 template <typename T, int MODE, int SRC, int BP, int R>
 int launch_bp(const Args& a, dim3 grid, hipStream_t st) {
   if constexpr (MODE == FF2 || MODE == TO_OUT) {
-    if (a.K <= 4096) {
+    if (a.K <= 2048) {
+      hipLaunchKernelGGL((decode_kernel<T, MODE, SRC, BP, R, 4, 1>), grid, dim3(kThreads), 0, st, a);
+    } else if (a.K <= 4096) {
       hipLaunchKernelGGL((decode_kernel<T, MODE, SRC, BP, R, 8, 1>), grid, dim3(kThreads), 0, st, a);
     } else {
       if constexpr (sizeof(T) == 4 && BP == 8)

@@ -297,6 +297,17 @@ def test_decoder_fp32_model_matches_fp64_oracle(B, dim, expansion, ff_mult):
     _against_oracle(m, B, 6, f"fp32 d{dim} exp{expansion} ff{ff_mult}", tol=1e-4)
 
 
+@pytest.mark.parametrize("width", [8, 16, 2048, 2056, 4096])
+@pytest.mark.parametrize("B", [1, 3, 5])
+def test_decoder_staged_row_lengths(B, width):
+    """Scan and FeedForward widths at the edges of the staged-row variants (up to 2048, 4096,
+    beyond) and the shortest rows. fp32 sums of n terms in any order are within n eps = 4096 x
+    6e-8 = 2.4e-4 of the exact sum, and their random parts within sqrt(n) eps = 4e-6 a product;
+    1e-4 over the eight chained products."""
+    m = _model_f32(256, 2, seed=60 + B, expansion=width / 256, ff_mult=width / 256)
+    _against_oracle(m, B, 3, f"fp32 width {width}", tol=1e-4)
+
+
 def test_fp32_model_calls_run_on_the_decoder():
     """An fp32 model's one-token calls under no_grad route to the fp32 decode steps (their
     logits are fp32 and equal Decoder.step's bit for bit) and agree with the parallel path
