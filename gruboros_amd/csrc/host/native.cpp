@@ -56,11 +56,24 @@ Tensor make(at::IntArrayRef size, at::ScalarType type, const Tensor& like) {
   return at::empty(size, like.options().dtype(type).requires_grad(false));
 }
 Tensor bytes(size_t n, const Tensor& like) { return make({static_cast<int64_t>(n)}, at::kByte, like); }
-void* ptr(const Tensor& t) { return t.data_ptr(); }
-void* ptr(const Opt& t) { return t ? t->data_ptr() : nullptr; }
-float* fp(const Tensor& t) { return static_cast<float*>(t.data_ptr()); }
-float* fp(const Opt& t) { return t ? static_cast<float*>(t->data_ptr()) : nullptr; }
-int16_t* h16(const Tensor& t) { return static_cast<int16_t*>(t.data_ptr()); }
+// Pointers for the kernels: every tensor is checked to be on the GPU, and the
+// fp32 ones to be fp32, where its pointer is taken.
+void* ptr(const Tensor& t) {
+  need_cuda(t);
+  return t.data_ptr();
+}
+void* ptr(const Opt& t) { return t ? ptr(*t) : nullptr; }
+float* fp(const Tensor& t) {
+  if (t.scalar_type() != at::kFloat) fail(std::string("expected a float32 tensor, got ") + c10::toString(t.scalar_type()));
+  return static_cast<float*>(ptr(t));
+}
+float* fp(const Opt& t) { return t ? fp(*t) : nullptr; }
+// a dense vector of n fp32 values (a bias, a norm weight)
+float* vec(const Tensor& t, int64_t n, const char* name) {
+  if (t.numel() != n || !t.is_contiguous()) fail(std::string(name) + ": expected " + std::to_string(n) + " contiguous float32 values");
+  return fp(t);
+}
+int16_t* h16(const Tensor& t) { return static_cast<int16_t*>(ptr(t)); }
 void* st(int64_t stream) { return reinterpret_cast<void*>(stream); }
 bool deterministic() { return at::globalContext().deterministicAlgorithms(); }
 
@@ -90,7 +103,7 @@ struct Mat {
   Mat rows(int64_t r0) const { return {static_cast<char*>(p) + r0 * ld * esize, ld, esize}; }
   Mat cols(int64_t c0) const { return {static_cast<char*>(p) + c0 * esize, ld, esize}; }
 };
-Mat mat(const Tensor& t, const char* name) { return {t.data_ptr(), row_stride(t, name), int64_t(t.element_size())}; }
+Mat mat(const Tensor& t, const char* name) { return {ptr(t), row_stride(t, name), int64_t(t.element_size())}; }
 
 // ------------------------------------------------------------------ products
 
@@ -225,7 +238,7 @@ Tensor gemm_f32(const Tensor& a, int al, const Tensor& b, int bl, int64_t M, int
   Tensor out = out_ ? *out_ : make({M, N}, at::kFloat, a);
   const Mat am = mat(a, "A"), bm = mat(b, "B"), om = mat(out, "C");
   gemm_f32_raw(al, static_cast<float*>(am.p), am.ld, bl, static_cast<float*>(bm.p), bm.ld, M, N, K,
-               bias ? MG_EPI_BIAS : MG_EPI_NONE, fp(bias), nullptr, static_cast<float*>(om.p), om.ld, flags, a, stream);
+               bias ? MG_EPI_BIAS : MG_EPI_NONE, bias ? vec(*bias, N, "bias") : nullptr, nullptr, fp(out), om.ld, flags, a, stream);
   return out;
 }
 
@@ -240,9 +253,9 @@ std::tuple<Opt, Tensor, Tensor> ff_f32_forward(const Tensor& x, const Tensor& w1
   if (train) pre = make({N, F}, at::kFloat, x);
   Tensor act = make({N, F}, at::kFloat, x), y = make({N, O}, at::kFloat, x);
   gemm_f32_raw(MG_KCONTIG, fp(x), row_stride(x, "x"), MG_KCONTIG, fp(w1), row_stride(w1, "w1"), N, F, D, MG_EPI_BIAS_GELU,
-               fp(b1), fp(pre), fp(act), F, flags, x, stream);
-  gemm_f32_raw(MG_KCONTIG, fp(act), F, MG_KCONTIG, fp(w2), row_stride(w2, "w2"), N, O, F, MG_EPI_BIAS, fp(b2), nullptr, fp(y),
-               O, flags, x, stream);
+               vec(b1, F, "b1"), fp(pre), fp(act), F, flags, x, stream);
+  gemm_f32_raw(MG_KCONTIG, fp(act), F, MG_KCONTIG, fp(w2), row_stride(w2, "w2"), N, O, F, MG_EPI_BIAS, vec(b2, O, "b2"), nullptr,
+               fp(y), O, flags, x, stream);
   return {pre, act, y};
 }
 
@@ -334,12 +347,12 @@ struct HG {
 };
 HG split(const Tensor& hg) {  // [B, T, 2 Di] (or [N, 2 Di] with B, T set by the caller), contiguous
   const int64_t Di = hg.size(-1) / 2;
-  char* p = static_cast<char*>(hg.data_ptr());
+  char* p = static_cast<char*>(ptr(hg));
   return {code(hg), p, p + Di * hg.element_size(), hg.dim() == 3 ? hg.size(1) * 2 * Di : 0, 2 * Di,
           hg.dim() == 3 ? hg.size(0) : 0, hg.dim() == 3 ? hg.size(1) : 0, Di};
 }
 HG two(const Tensor& hidden, const Tensor& gate) {
-  return {code(hidden), static_cast<char*>(hidden.data_ptr()), static_cast<char*>(gate.data_ptr()), hidden.stride(0),
+  return {code(hidden), static_cast<char*>(ptr(hidden)), static_cast<char*>(ptr(gate)), hidden.stride(0),
           hidden.stride(1), hidden.size(0), hidden.size(1), hidden.size(2)};
 }
 
@@ -530,8 +543,8 @@ FFOut ff_forward(const Tensor& x1, const Opt& out, const Tensor& w_norm, const T
                  const Tensor& b2, int64_t stream) {
   auto [x2, n2, rstd, none] = norm_fwd(x1, out, w_norm, true, false, stream);
   Tensor pre = make({x1.size(0), w1.size(0)}, at::kBFloat16, x1);
-  Tensor act = linear_fwd(n2, w1, fp(b1), &pre, stream);     // pre = n2 W1^T + b1, act = gelu(pre)
-  Tensor pend = linear_fwd(act, w2, fp(b2), nullptr, stream);  // act W2^T + b2
+  Tensor act = linear_fwd(n2, w1, vec(b1, w1.size(0), "b1"), &pre, stream);     // pre = n2 W1^T + b1, act = gelu(pre)
+  Tensor pend = linear_fwd(act, w2, vec(b2, w2.size(0), "b2"), nullptr, stream);  // act W2^T + b2
   return {x2, n2, rstd, pre, act, pend};
 }
 
@@ -587,7 +600,7 @@ std::tuple<Tensor, Opt, Tensor, Tensor, Tensor> head_forward(const Tensor& x, co
   const int64_t N = x.size(0), D = x.size(1), V = w.size(0);
   auto [x_out, embed, rstd, none] = norm_fwd(x, pending, w_norm, true, false, stream);
   Tensor dl = make({N, V}, at::kBFloat16, x), part = make({mg_logits_cross_entropy_partials(N)}, at::kFloat, x);
-  check(mg_logits_cross_entropy(ptr(embed), D, ptr(w), row_stride(w, "w"), static_cast<int64_t*>(labels.data_ptr()), ptr(dl), V,
+  check(mg_logits_cross_entropy(ptr(embed), D, ptr(w), row_stride(w, "w"), static_cast<int64_t*>(ptr(labels)), ptr(dl), V,
                                 fp(part), nullptr, N, D, V, static_cast<float>(1.0 / N), st(stream)),
         "mg_logits_cross_entropy");
   return {part.sum() / N, x_out, embed, rstd, dl};

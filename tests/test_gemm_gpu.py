@@ -842,3 +842,26 @@ def test_f32_feed_forward_matches_fp64(N, D, Fw, deterministic):
     yr.backward(dy.double().cpu())
     errs = [_rel(a, b) for a, b in zip(got, [yr, xr.grad] + [p.grad for p in ref.parameters()])]
     assert all(e <= 2e-6 for e in errs), errs
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("op", ["linear", "feed_forward"])
+@pytest.mark.parametrize("bad", ["weight on the CPU", "bias on the CPU", "bfloat16 bias", "short bias"])
+def test_f32_layers_refuse_what_the_kernels_cannot_read(op, bad):
+    """fp32 products read their weights and biases through raw pointers: what is not on the GPU, not
+    fp32 or not of the layer's width is an error on the host, before any launch."""
+    from gruboros_amd._lib import MingruHipError
+    from gruboros_amd.linear import feed_forward, linear
+
+    last = torch.nn.Linear(64, 32, device="cuda")
+    if bad == "weight on the CPU":
+        last.weight = torch.nn.Parameter(last.weight.detach().cpu())
+    else:
+        b = last.bias.detach()
+        last.bias = torch.nn.Parameter({"bias on the CPU": b.cpu(), "bfloat16 bias": b.bfloat16(), "short bias": b[:16]}[bad])
+    with pytest.raises(MingruHipError):
+        if op == "linear":
+            linear(torch.randn(8, 64, device="cuda"), last)
+        else:
+            first = torch.nn.Linear(32, 64, device="cuda")
+            feed_forward(torch.randn(8, 32, device="cuda"), torch.nn.Sequential(first, torch.nn.GELU(), last))
