@@ -637,8 +637,11 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> infer_layer(const Tensor& x, c
     if (w->scalar_type() != w_hg.scalar_type() || w->dim() != 2 || w->stride(1) != 1 || w->size(0) % 8 || w->size(1) % 8 ||
         w->stride(0) % 8 || reinterpret_cast<uintptr_t>(w->data_ptr()) % 16)
       return std::nullopt;
+  for (const Tensor* t : {&w_hg, &w1, &w2, w_to ? &*w_to : &w_hg, &w_norm, &w_ff, &b1, &b2})
+    if (t->device() != x.device()) return std::nullopt;
   if (N < 1 || D > 4096 || Di % 8 || (w_to && (w_to->size(0) != D || w_to->size(1) != Di)) || (!w_to && Di != D) ||
-      w1.size(1) != D || w2.size(0) != D || w2.size(1) != F || x.stride(1) != 1 || x.stride(0) != D)
+      w_hg.size(1) != D || w1.size(1) != D || w2.size(0) != D || w2.size(1) != F || w_norm.numel() != D || w_ff.numel() != D ||
+      b1.numel() != F || b2.numel() != D || x.stride(1) != 1 || x.stride(0) != D)
     return std::nullopt;
   const int flags = deterministic() ? MG_GEMM_DETERMINISTIC : 0;
   const auto linear = [&](const Tensor& a, const Tensor& w) {

@@ -211,6 +211,7 @@ class minLM(Module):
         x = x.float()  # fp32 residual stream
 
         if x.is_cuda and self._infer_applies(cd):
+            prev_hiddens = list(prev_hiddens) if exists(prev_hiddens) else None  # (an iterator is read once)
             out = self._trunk_infer(x, prev_hiddens, cd)
             if out is not None:
                 return out
@@ -252,31 +253,47 @@ class minLM(Module):
 
     def _infer_applies(self, cd):
         """Whether the forward may run layer by layer in native code: no gradients of any mode, no
-        autocast, no conv and no active dropout, and parameters in the activation dtype."""
+        autocast, no conv, no dropout that acts (each layer's own mode counts: dropout may be kept on
+        in an eval() model), plain minGRU layers without biases, and parameters in the activation dtype."""
         return (not torch.is_grad_enabled() and cd == self.token_emb.weight.dtype and not torch.is_autocast_enabled()
                 and torch.autograd.forward_ad._current_level < 0
-                and all(conv is None and (dropout is None or not self.training)
-                        for conv, _, _, _, _, dropout in self.layers))
+                and all(conv is None and (dropout is None or (type(dropout) is nn.Dropout and not dropout.training))
+                        and type(mingru) is minGRU and mingru.to_hidden_and_gate.bias is None
+                        and getattr(mingru.to_out, "bias", None) is None
+                        for conv, _, mingru, _, _, dropout in self.layers))
+
+    def _infer_vectors(self):
+        """(norm weight, FeedForward norm weight, biases) of every layer in fp32. Those of a model in
+        another dtype are gathered and converted together on each call, two launches for the whole
+        model: a copy kept between calls would miss changes made through .data."""
+        vecs = [v for _, norm, _, ff_norm, ff, _ in self.layers for v in (norm.weight, ff_norm.weight, ff[0].bias, ff[2].bias)]
+        if any(v is None for v in vecs):
+            return None
+        if any(v.dtype != torch.float32 or not v.is_contiguous() for v in vecs):
+            vecs = torch.cat(vecs).float().split([v.numel() for v in vecs])
+        return [vecs[i:i + 4] for i in range(0, len(vecs), 4)]
 
     def _trunk_infer(self, x, prev_hiddens, cd):
         """_trunk without gradients (generate.py's prompt), one native call per layer; None where a
         layer's widths are not the kernels' (then _trunk runs op by op)."""
-        native, f32 = _lib.native(), decode._f32
+        native = _lib.native()
+        vectors = self._infer_vectors()
+        if vectors is None:
+            return None
         B, T, D = x.shape
         stream = _lib.stream_of(x)
         x, pending = x.reshape(B * T, D).contiguous(), None
         prev_hiddens = iter(default(prev_hiddens, []))
         next_prev_hiddens = []
-        for _, norm, mingru, ff_norm, ff, _ in self.layers:
+        for (_, _, mingru, _, ff, _), (w_norm, w_ff, b1, b2) in zip(self.layers, vectors):
             w_hg = mingru.to_hidden_and_gate.weight
-            l1, l2 = ff[0], ff[2]
-            if l1.bias is None or l2.bias is None or w_hg.dtype != cd:
+            if w_hg.dtype != cd:
                 return None
             Di = w_hg.shape[0] // 2
             h0 = _prep_h0(next(prev_hiddens, None), B, Di, x.device)
-            out = native.infer_layer(x, pending, f32(norm.weight), w_hg,
+            out = native.infer_layer(x, pending, w_norm, w_hg,
                                      mingru.to_out.weight if isinstance(mingru.to_out, nn.Linear) else None,
-                                     f32(ff_norm.weight), l1.weight, f32(l1.bias), l2.weight, f32(l2.bias), h0, B, T,
+                                     w_ff, ff[0].weight, b1, ff[2].weight, b2, h0, B, T,
                                      scan_errors._workspace(x.device, B, T, Di), stream)
             if out is None:
                 return None
