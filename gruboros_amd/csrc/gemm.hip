@@ -2799,29 +2799,38 @@ __global__ __launch_bounds__(256) void split_reduce_bf16_kernel(const float* __r
 
 constexpr int kCUs = 256;
 
-// Hi/lo products of few 256 x 128 tiles (gemm_t128_kernel), whole 32-k steps.
-// bf16 outputs (to_hidden_and_gate's hidden half; never split): up to 192
-// tiles. There the 256 x 256 tiles of the persistent kernel number 96 at most,
-// each CU's share is one tile of three times the gate half's work, and the rest
-// of the chip idles (to_hidden_and_gate, us: 128 rows d256 e3 18.5 -> 12.4, 333
-// rows d768 e2 42.4 -> 25.7, 1024 rows d512 e1.5 30.6 -> 19.3, 2048 rows d1024
-// e3 69 -> 60 in the block); with 256 tiles (2048 rows, d2048, e2) 124 -> 126.
-// fp32 outputs (to_out) split along K to at most one workgroup per CU, by
-// estimated time: 0.85 us per step, 8 us to start and store, partials written
-// and read at about 7.4 TB/s plus 4 us for their reduction. From 3e9
-// multiply-adds (2048 rows, d1024, e3: 57 -> 43 us in the block); smaller ones
-// are 1 to 3 us faster on 128 x 128 tiles, which start sooner.
+// Whether mg_gemm_hilo_cols takes a product: whole 32-k steps and at most 192
+// tiles of 256 x 128 in its hi/lo columns. There the 256 x 256 tiles of
+// mg_gemm_hilo_prefix's persistent kernel leave CUs idle, each tile takes three
+// times the gate half's work and the rest of the chip waits (us, the prefix
+// kernel -> this one: 128 rows d256 e3 18.5 -> 12.4, 333 rows d768 e2 42.4 ->
+// 25.7, 1024 rows d512 e1.5 30.6 -> 19.3, 2048 rows d1024 e3 69 -> 60 in the
+// block; over 187 sizes from 16 to 8192 rows, d256 to d2048, 0.68 of the time on
+// average and none slower); with 256 tiles (2048 rows, d2048, e2) 124 -> 126. A
+// lone hi/lo product with a bf16 result stays on plan()'s tiles: without the
+// gate half's tiles to fill the chip, 256 x 128 ones measured slower at 155 of
+// 223 sizes, by up to 42% (300 x 256 x 256, 10.8 -> 15.3 us).
+inline bool hilo_cols_ok(int M, int N, int K) {
+  return M >= 1 && N >= 1 && K >= 32 && K % 32 == 0 && int64_t((M + 255) / 256) * ((N + 127) / 128) <= 192;
+}
+
+// fp32 hi/lo products (to_out) of at most one 256 x 128 tile per CU
+// (gemm_t128_kernel), whole 32-k steps, from 3e9 multiply-adds: split along K
+// to at most one workgroup per CU, by estimated time: 0.85 us per step, 8 us to
+// start and store, partials written and read at about 7.4 TB/s plus 4 us for
+// their reduction (2048 rows, d1024, e3: 57 -> 43 us in the block). Smaller
+// ones are 1 to 3 us faster on 128 x 128 tiles, which start sooner.
 struct HiloPlan {
   bool ok;
   int kt_per_split, splits;
 };
-inline HiloPlan hilo_plan(int M, int N, int K, bool f32, bool whole) {
+inline HiloPlan hilo_plan(int M, int N, int K, bool whole) {
   HiloPlan best{};
   const int64_t T = int64_t((M + 255) / 256) * ((N + 127) / 128);
-  if (M < 1 || N < 1 || K < 32 || K % 32 || T > (f32 ? kCUs : 192) || (f32 && double(M) * N * K < 3e9)) return best;
+  if (M < 1 || N < 1 || K < 32 || K % 32 || T > kCUs || double(M) * N * K < 3e9) return best;
   const int steps = K / 32;
   double least = 1e300;
-  for (int s = 1; s == 1 || (f32 && !whole && s * T <= kCUs && steps / s >= 4); ++s) {
+  for (int s = 1; s == 1 || (!whole && s * T <= kCUs && steps / s >= 4); ++s) {
     const int kt = (steps + s - 1) / s, ys = (steps + kt - 1) / kt;
     const double cost = 0.85 * kt + 8.0 + (ys > 1 ? 4.0 + double(ys) * M * N * 8.0 / 7.4e6 : 0.0);
     if (cost < least) least = cost, best = HiloPlan{true, kt, ys};
@@ -3114,7 +3123,7 @@ inline int launch_pair(Params p0, Params p1, const PairPlan& pp, hipStream_t s) 
 }
 
 // to_hidden_and_gate's forward on 256 x 128 tiles: p holds the whole product.
-inline int launch_t128_prefix(Params p, int hilo_cols, hipStream_t s) {
+inline int launch_hilo_cols(Params p, int hilo_cols, hipStream_t s) {
   Params q = p;  // the gate half: a plain product of the hi halves
   p.b_span = static_cast<uint32_t>((int64_t(hilo_cols - 1) * p.ldb + 2 * p.K) * 2);
   q.b_span = static_cast<uint32_t>((int64_t(p.N - hilo_cols - 1) * p.ldb + 2 * p.K) * 2);
@@ -3129,7 +3138,7 @@ inline int launch_t128_prefix(Params p, int hilo_cols, hipStream_t s) {
   q.kt_per_split = p.K / BK;
   const int wgs = (p.tiles_m * p.tiles_n + 7) / 8 * 8 + (q.tiles_m * q.tiles_n + 7) / 8 * 8;
   hipLaunchKernelGGL(gemm_t128_prefix_kernel, dim3(wgs), dim3(256), 0, s, p, q);
-  return check_launch("mg_gemm_hilo_prefix");
+  return check_launch("mg_gemm_hilo_cols");
 }
 
 // One launch for a dX product and one or two weight gradients (mg_gemm_group).
@@ -3330,8 +3339,8 @@ extern "C" int mg_gemm(int a_layout, const void* A, int64_t lda, int b_layout, c
   p.hilo = hilo ? 1 : 0;
   p.nkt_seg = (K + gemm::BK - 1) / gemm::BK;
   if (K == 0 && accumulate) return MG_OK;
-  if (hilo && epilogue == MG_EPI_NONE && !accumulate) {
-    const gemm::HiloPlan hp = gemm::hilo_plan(M, N, K, c_dtype == MG_F32, deterministic || !workspace);
+  if (hilo && epilogue == MG_EPI_NONE && !accumulate && c_dtype == MG_F32) {
+    const gemm::HiloPlan hp = gemm::hilo_plan(M, N, K, deterministic || !workspace);
     if (hp.ok) {
       const size_t need = hp.splits > 1 ? static_cast<size_t>(hp.splits) * M * N * sizeof(float) : 0;
       if (need && workspace_bytes < need)
@@ -3342,7 +3351,7 @@ extern "C" int mg_gemm(int a_layout, const void* A, int64_t lda, int b_layout, c
       p.tiles_m = (M + 255) / 256;
       p.tiles_n = (N + 127) / 128;
       p.kt_per_split = hp.kt_per_split;
-      const int out = hp.splits > 1 ? gemm::T128_PART : c_dtype == MG_F32 ? gemm::T128_F32 : gemm::T128_BF16;
+      const int out = hp.splits > 1 ? gemm::T128_PART : gemm::T128_F32;
       hipLaunchKernelGGL((gemm::gemm_t128_kernel<true>), dim3((p.tiles_m * p.tiles_n * hp.splits + 7) / 8 * 8), dim3(256), 0, s, p,
                          hp.splits, out);
       if (check_launch(fn)) return MG_ERR_HIP;
@@ -3403,7 +3412,7 @@ static int hilo_prefix_params(const char* fn, const void* A, int64_t lda, const 
 
 extern "C" int mg_gemm_hilo_cols_fits(int M, int N, int K, int hilo_cols) {
   return M >= 1 && K >= 64 && K % 64 == 0 && N % 8 == 0 && hilo_cols >= 8 && hilo_cols % 8 == 0 && hilo_cols < N &&
-                 gemm::hilo_plan(M, hilo_cols, K, false, true).ok
+                 gemm::hilo_cols_ok(M, hilo_cols, K)
              ? 1
              : 0;
 }
@@ -3416,7 +3425,7 @@ extern "C" int mg_gemm_hilo_cols(const void* A, int64_t lda, const void* B, int6
     return fail(MG_ERR_ARG, "%s: M=%d N=%d K=%d hilo_cols=%d (mg_gemm_hilo_cols_fits)", fn, M, N, K, hilo_cols);
   gemm::Params p{};
   if (const int rc = hilo_prefix_params(fn, A, lda, B, ldb, M, N, K, C, ldc, p)) return rc;
-  return gemm::launch_t128_prefix(p, hilo_cols, static_cast<hipStream_t>(stream));
+  return gemm::launch_hilo_cols(p, hilo_cols, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int mg_gemm_hilo_prefix(const void* A, int64_t lda, const void* B, int64_t ldb, int M, int N, int K,
@@ -3430,7 +3439,6 @@ extern "C" int mg_gemm_hilo_prefix(const void* A, int64_t lda, const void* B, in
     return fail(MG_ERR_ARG, "%s: hilo_cols %d must be a multiple of 256 below N=%d", fn, hilo_cols, N);
   gemm::Params p{};
   if (const int rc = hilo_prefix_params(fn, A, lda, B, ldb, M, N, K, C, ldc, p)) return rc;
-  if (gemm::hilo_plan(M, hilo_cols, K, false, true).ok) return gemm::launch_t128_prefix(p, hilo_cols, static_cast<hipStream_t>(stream));
   p.hilo = 1;
   p.nkt_seg = K / gemm::BK;  // even: K % 128 == 0
   p.hilo_cols = hilo_cols;
@@ -3445,8 +3453,8 @@ extern "C" int mg_gemm_hilo_prefix(const void* A, int64_t lda, const void* B, in
 extern "C" size_t mg_gemm_workspace_bytes(int a_layout, int b_layout, int M, int N, int K, int epilogue,
                                           int c_dtype, int flags) {
   if (M < 1 || N < 1 || K < 1) return 0;
-  if ((flags & MG_GEMM_HILO) && epilogue == MG_EPI_NONE && !(flags & MG_GEMM_ACCUMULATE)) {
-    const gemm::HiloPlan hp = gemm::hilo_plan(M, N, K, c_dtype == MG_F32, flags & MG_GEMM_DETERMINISTIC);
+  if ((flags & MG_GEMM_HILO) && epilogue == MG_EPI_NONE && !(flags & MG_GEMM_ACCUMULATE) && c_dtype == MG_F32) {
+    const gemm::HiloPlan hp = gemm::hilo_plan(M, N, K, flags & MG_GEMM_DETERMINISTIC);
     if (hp.ok) return hp.splits > 1 ? static_cast<size_t>(hp.splits) * M * N * sizeof(float) : 0;
   }
   const gemm::Plan pl = gemm::plan(M, N, K, a_layout == MG_KCONTIG, b_layout == MG_KCONTIG, c_dtype, epilogue,

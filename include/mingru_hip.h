@@ -395,9 +395,11 @@ int mg_gemm(int a_layout, const void* A, int64_t lda,
  * leading dimensions multiples of 8, 16-byte aligned operands. */
 int mg_gemm_hilo_prefix(const void* A, int64_t lda, const void* B, int64_t ldb, int M, int N, int K, int hilo_cols,
                         void* C, int64_t ldc, void* stream);
-/* mg_gemm_hilo_prefix for few rows: the same result for K % 64 == 0 and any
+/* mg_gemm_hilo_prefix for few rows: the same products for K % 64 == 0 and any
  * hilo_cols that is a multiple of 8, where the hi/lo columns make at most 192
- * tiles of 256 x 128 (mg_gemm_hilo_cols_fits returns 1; otherwise it fails). */
+ * tiles of 256 x 128 (mg_gemm_hilo_cols_fits returns 1; otherwise it fails).
+ * The three hi/lo products are summed per 32 k, not one after the other over
+ * all of K as mg_gemm and mg_gemm_hilo_prefix do. */
 int mg_gemm_hilo_cols(const void* A, int64_t lda, const void* B, int64_t ldb, int M, int N, int K, int hilo_cols,
                       void* C, int64_t ldc, void* stream);
 int mg_gemm_hilo_cols_fits(int M, int N, int K, int hilo_cols);

@@ -323,6 +323,27 @@ def test_hilo_product_is_fp32_accurate(M, N, K, out_dtype):
     assert bool((buf[:, N:] == 3.0).all())  # the other half of the packed buffer is untouched
 
 
+@pytest.mark.parametrize("M,N,K", [(37, 64, 32), (300, 392, 192), (777, 1536, 768), (2047, 1032, 1024)])
+def test_hilo_product_rounds_as_asked(M, N, K):
+    """MG_GEMM_HILO with a bf16 C rounds the fp32 hi/lo sum once: to nearest, or with
+    MG_GEMM_STOCHASTIC by the gradient stores' hash of the element index (salt 0x9e5b). The fp32
+    sum is the unsplit fp32 product's, which adds in the same order, so both are equal to it
+    rounded by torch and by mg_round_bf16_sr, bit for bit; and the two differ."""
+    from gruboros_amd.gemm import KCONTIG, gemm, round_bf16_sr, split_hilo
+
+    gen = torch.Generator(device=DEV).manual_seed(M + N + K)
+    a = split_hilo(torch.randn(M, K, device=DEV, generator=gen))
+    b = split_hilo(torch.randn(N, K, device=DEV, generator=gen) / K ** 0.5)
+    f32 = torch.empty(M, N, device=DEV)
+    gemm(a, KCONTIG, b, KCONTIG, M, N, K, f32, hilo=True, deterministic=True)
+    rn, sr = torch.empty(M, N, device=DEV, dtype=torch.bfloat16), torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
+    gemm(a, KCONTIG, b, KCONTIG, M, N, K, rn, hilo=True)
+    gemm(a, KCONTIG, b, KCONTIG, M, N, K, sr, hilo=True, stochastic=True)
+    assert torch.equal(rn, f32.to(torch.bfloat16))
+    assert torch.equal(sr, round_bf16_sr(f32, salt=0x9e5b))
+    assert float((sr != rn).float().mean()) > 0.1
+
+
 def _dev_operand(rows, k, layout, g, scale=1.0):
     """bf16 operand [rows, k] (logical) stored K-contiguous ([rows, k]) or MN-contiguous ([k, rows])."""
     logical = (torch.randn(rows, k, device=DEV, generator=g) * scale).to(torch.bfloat16)
