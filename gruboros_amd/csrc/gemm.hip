@@ -2819,7 +2819,10 @@ inline bool hilo_cols_ok(int M, int N, int K) {
 // to at most one workgroup per CU, by estimated time: 0.85 us per step, 8 us to
 // start and store, partials written and read at about 7.4 TB/s plus 4 us for
 // their reduction (2048 rows, d1024, e3: 57 -> 43 us in the block). Smaller
-// ones are 1 to 3 us faster on 128 x 128 tiles, which start sooner.
+// ones are 1 to 3 us faster on 128 x 128 tiles, which start sooner. Never with
+// MG_GEMM_DETERMINISTIC: these tiles sum the three hi/lo products per 32 k, the
+// others one after the other over all of K, and there a row's result must not
+// depend on how many rows come with it.
 struct HiloPlan {
   bool ok;
   int kt_per_split, splits;
@@ -3339,8 +3342,8 @@ extern "C" int mg_gemm(int a_layout, const void* A, int64_t lda, int b_layout, c
   p.hilo = hilo ? 1 : 0;
   p.nkt_seg = (K + gemm::BK - 1) / gemm::BK;
   if (K == 0 && accumulate) return MG_OK;
-  if (hilo && epilogue == MG_EPI_NONE && !accumulate && c_dtype == MG_F32) {
-    const gemm::HiloPlan hp = gemm::hilo_plan(M, N, K, deterministic || !workspace);
+  if (hilo && epilogue == MG_EPI_NONE && !accumulate && c_dtype == MG_F32 && !deterministic) {
+    const gemm::HiloPlan hp = gemm::hilo_plan(M, N, K, !workspace);
     if (hp.ok) {
       const size_t need = hp.splits > 1 ? static_cast<size_t>(hp.splits) * M * N * sizeof(float) : 0;
       if (need && workspace_bytes < need)
@@ -3453,8 +3456,9 @@ extern "C" int mg_gemm_hilo_prefix(const void* A, int64_t lda, const void* B, in
 extern "C" size_t mg_gemm_workspace_bytes(int a_layout, int b_layout, int M, int N, int K, int epilogue,
                                           int c_dtype, int flags) {
   if (M < 1 || N < 1 || K < 1) return 0;
-  if ((flags & MG_GEMM_HILO) && epilogue == MG_EPI_NONE && !(flags & MG_GEMM_ACCUMULATE) && c_dtype == MG_F32) {
-    const gemm::HiloPlan hp = gemm::hilo_plan(M, N, K, flags & MG_GEMM_DETERMINISTIC);
+  if ((flags & MG_GEMM_HILO) && epilogue == MG_EPI_NONE && !(flags & (MG_GEMM_ACCUMULATE | MG_GEMM_DETERMINISTIC)) &&
+      c_dtype == MG_F32) {
+    const gemm::HiloPlan hp = gemm::hilo_plan(M, N, K, false);
     if (hp.ok) return hp.splits > 1 ? static_cast<size_t>(hp.splits) * M * N * sizeof(float) : 0;
   }
   const gemm::Plan pl = gemm::plan(M, N, K, a_layout == MG_KCONTIG, b_layout == MG_KCONTIG, c_dtype, epilogue,

@@ -432,7 +432,7 @@ GruOut gru_forward(const Tensor& x, const Opt& pending, const Tensor& w_norm, co
   const auto span = [](int64_t rows, int64_t ld) { return (rows + 256) * ld * 2 < (int64_t(1) << 31); };
   const bool pair_ok = one_launch && wm.ld % 8 == 0 && wm.ld >= 2 * D && reinterpret_cast<uintptr_t>(wm.p) % 16 == 0 &&
                        span(N, pm.ld) && span(2 * Di, wm.ld);
-  if (pair_ok && mg_gemm_hilo_cols_fits(N, 2 * Di, D, Di)) {
+  if (pair_ok && !deterministic() && mg_gemm_hilo_cols_fits(N, 2 * Di, D, Di)) {  // (its sum order is its own)
     check(mg_gemm_hilo_cols(pm.p, pm.ld, wm.p, wm.ld, N, 2 * Di, D, Di, hm.p, hm.ld, st(stream)), "mg_gemm_hilo_cols");
   } else if (pair_ok && D % 128 == 0 && Di % 256 == 0) {
     check(mg_gemm_hilo_prefix(pm.p, pm.ld, wm.p, wm.ld, N, 2 * Di, D, Di, hm.p, hm.ld, st(stream)), "mg_gemm_hilo_prefix");

@@ -335,7 +335,8 @@ int mg_sf_adamw_step(const void* tensors, int ntensors, int64_t nchunks,
  *   gelu(x) = x/2 (1 + erf(x/sqrt(2))), nn.GELU()'s exact form.
  * flags (bit set):
  *   MG_GEMM_ACCUMULATE (fp32 C, no epilogue): C += A B.
- *   MG_GEMM_DETERMINISTIC: never split along K.
+ *   MG_GEMM_DETERMINISTIC: never split along K, and the sum order depends on K
+ *     alone (a row's result does not depend on M).
  *   MG_GEMM_STOCHASTIC: a bf16 C (epilogue NONE) is rounded stochastically,
  *     as gradients are (see the conventions above); the GELU-gradient
  *     epilogue always is.

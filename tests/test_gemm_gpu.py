@@ -344,6 +344,50 @@ def test_hilo_product_rounds_as_asked(M, N, K):
     assert float((sr != rn).float().mean()) > 0.1
 
 
+@pytest.mark.parametrize("N,K", [(1024, 1024), (1024, 3072), (512, 256)])
+@pytest.mark.parametrize("hilo", [False, True])
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
+def test_deterministic_rows_do_not_depend_on_the_row_count(N, K, hilo, out_dtype):
+    """With the deterministic flag the sum order depends only on K: a row's result is the same bit for
+    bit whatever tiles the number of rows leads to (64 x 64, 128 x 128, 256 x 256, persistent)."""
+    from gruboros_amd.gemm import KCONTIG, gemm
+
+    gen = torch.Generator(device=DEV).manual_seed(N + K)
+    w = 2 if hilo else 1
+    a = torch.randn(16376, w * K, device=DEV, generator=gen).to(torch.bfloat16)
+    b = torch.randn(N, w * K, device=DEV, generator=gen).to(torch.bfloat16)
+    first = None
+    for M in (64, 300, 2048, 4096, 16376):
+        out = torch.empty(M, N, device=DEV, dtype=out_dtype)
+        gemm(a[:M], KCONTIG, b, KCONTIG, M, N, K, out, hilo=hilo, deterministic=True)
+        first = out if first is None else first
+        assert torch.equal(out[:64], first), M
+
+
+def test_deterministic_block_samples_do_not_depend_on_the_batch():
+    """The minGRU block's outputs for one sample under torch.use_deterministic_algorithms are the same
+    bit for bit alone (300 rows) and in a batch of 16 (4800 rows, other tiles for to_hidden_and_gate
+    and for to_out)."""
+    from gruboros_amd import blocks
+    from gruboros_amd.mingru import minGRU
+
+    torch.manual_seed(5)
+    with torch.device(DEV):
+        layer, norm = minGRU(512, expansion_factor=3.0), torch.nn.RMSNorm(512)
+        x, pending = torch.randn(16, 300, 512), torch.randn(16, 300, 512).to(torch.bfloat16)
+    outs = []
+    torch.use_deterministic_algorithms(True)
+    try:
+        with torch.no_grad():
+            for n in (1, 16):
+                outs.append(blocks.MinGRUBlock.apply(x[:n], pending[:n], norm.weight, layer.to_hidden_and_gate.weight, None,
+                                                     layer.to_out.weight))
+    finally:
+        torch.use_deterministic_algorithms(False)
+    for one, all_ in zip(*outs):
+        assert torch.equal(one, all_[:1])
+
+
 def _dev_operand(rows, k, layout, g, scale=1.0):
     """bf16 operand [rows, k] (logical) stored K-contiguous ([rows, k]) or MN-contiguous ([k, rows])."""
     logical = (torch.randn(rows, k, device=DEV, generator=g) * scale).to(torch.bfloat16)
