@@ -93,13 +93,15 @@ def _native_cmds(objdir):
 
 
 def _link(cmd, path, verbose):
-    fd, tmp = tempfile.mkstemp(prefix=os.path.basename(path) + ".tmp", dir=HERE)
-    os.close(fd)
-    rc, out = _run([*cmd, "-o", tmp], verbose)
-    if rc != 0:
-        os.unlink(tmp)
-        raise RuntimeError(f"linking {os.path.basename(path)} failed ({rc}):\n{out}")
-    os.replace(tmp, path)
+    """Runs the link command into a directory of its own beside `path` and moves the result there:
+    the linker creates the file, so its mode is the umask's (a mkstemp file is 0600, and a linker
+    that writes into it leaves a library only its builder can read)."""
+    name = os.path.basename(path)
+    with tempfile.TemporaryDirectory(prefix=name + ".tmp", dir=os.path.dirname(path)) as tmp:
+        rc, out = _run([*cmd, "-o", os.path.join(tmp, name)], verbose)
+        if rc != 0:
+            raise RuntimeError(f"linking {name} failed ({rc}):\n{out}")
+        os.replace(os.path.join(tmp, name), path)
 
 
 def build(verbose: bool = False) -> str:

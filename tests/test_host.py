@@ -3,6 +3,7 @@ drop-in minLM (reference mingru/minLM.py:157-206) and the `mingru` alias with
 its default compute dtype."""
 import math
 
+import pytest
 import torch
 from torch import nn
 
@@ -188,3 +189,28 @@ def test_decoder_applies_to_fp32_models_within_their_staged_limit():
     assert "4096" in unsupported_reason(m2, 8)
     assert unsupported_reason(m2.half(), 8) is None  # 16-bit rows: the full 8192
     assert "fp32 model" in unsupported_reason(m.double(), 1)
+
+
+def test_linked_libraries_are_readable_by_every_user(tmp_path):
+    """What build._link writes has the umask's mode, whoever links it (hipcc replaces its output
+    file, g++ writes into an existing one), and leaves nothing else behind."""
+    import os
+    import stat
+
+    from gruboros_amd import build
+
+    src = tmp_path / "f.c"
+    src.write_text("int f(void) { return 1; }\n")
+    out = tmp_path / "out" / "f.so"
+    out.parent.mkdir()
+    old = os.umask(0o022)
+    try:
+        for _ in range(2):  # also over a file that is there
+            build._link(["g++", "-shared", "-fPIC", str(src)], str(out), False)
+    finally:
+        os.umask(old)
+    assert stat.S_IMODE(out.stat().st_mode) == 0o755
+    assert os.listdir(out.parent) == ["f.so"]
+    with pytest.raises(RuntimeError, match="linking f.so failed"):
+        build._link(["g++", "-shared", str(tmp_path / "missing.c")], str(out), False)
+    assert os.listdir(out.parent) == ["f.so"]
