@@ -86,6 +86,17 @@ int64_t row_stride(const Tensor& t, const char* name) {
   return t.stride(0);
 }
 
+// A matrix operand of a product: rows x cols exactly, so that a launch reads and writes inside it
+// (the C ABI sees leading dimensions only).
+const Tensor& extent(const Tensor& t, int64_t rows, int64_t cols, const char* name) {
+  if (t.dim() != 2 || t.size(0) != rows || t.size(1) != cols) {
+    std::string s = std::string(name) + ": expected [" + std::to_string(rows) + ", " + std::to_string(cols) + "], got [";
+    for (int64_t i = 0; i < t.dim(); ++i) s += (i ? ", " : "") + std::to_string(t.size(i));
+    fail(s + "]");
+  }
+  return t;
+}
+
 // Rows per launch of a row-parallel product over n rows whose operands take
 // `row_bytes` per row at most: each operand then spans under 2 GiB, mg_gemm's
 // buffer range with 256 rows of slack; a multiple of 256.
@@ -236,6 +247,9 @@ Tensor gemm_f32(const Tensor& a, int al, const Tensor& b, int bl, int64_t M, int
   need_cuda(b);
   if (a.scalar_type() != at::kFloat || b.scalar_type() != at::kFloat) fail("mg_gemm_f32 operands must be float32");
   Tensor out = out_ ? *out_ : make({M, N}, at::kFloat, a);
+  extent(a, al == MG_KCONTIG ? M : K, al == MG_KCONTIG ? K : M, "A");
+  extent(b, bl == MG_KCONTIG ? N : K, bl == MG_KCONTIG ? K : N, "B");
+  extent(out, M, N, "C");
   const Mat am = mat(a, "A"), bm = mat(b, "B"), om = mat(out, "C");
   gemm_f32_raw(al, static_cast<float*>(am.p), am.ld, bl, static_cast<float*>(bm.p), bm.ld, M, N, K,
                bias ? MG_EPI_BIAS : MG_EPI_NONE, bias ? vec(*bias, N, "bias") : nullptr, nullptr, fp(out), om.ld, flags, a, stream);
@@ -248,6 +262,8 @@ Tensor column_sum(const Tensor& x, int64_t stream);
 std::tuple<Opt, Tensor, Tensor> ff_f32_forward(const Tensor& x, const Tensor& w1, const Tensor& b1, const Tensor& w2,
                                                const Tensor& b2, bool train, int64_t stream) {
   const int64_t N = x.size(0), D = x.size(1), F = w1.size(0), O = w2.size(0);
+  extent(w1, F, D, "w1");
+  extent(w2, O, F, "w2");
   const int flags = deterministic() ? MG_GEMM_DETERMINISTIC : 0;
   Opt pre;
   if (train) pre = make({N, F}, at::kFloat, x);
@@ -264,6 +280,11 @@ std::tuple<Opt, Opt, Opt, Opt, Opt> ff_f32_backward(const Tensor& x, const Tenso
                                                     const Tensor& w2, const Tensor& dy, bool want_x, bool want_w1, bool want_b1,
                                                     bool want_w2, bool want_b2, int64_t stream) {
   const int64_t N = x.size(0), D = x.size(1), F = pre.size(1), O = dy.size(1);
+  extent(w1, F, D, "w1");
+  extent(w2, O, F, "w2");
+  extent(pre, N, F, "pre");
+  extent(act, N, F, "act");
+  extent(dy, N, O, "dy");
   const int flags = deterministic() ? MG_GEMM_DETERMINISTIC : 0;
   Opt dx, dw1, db1, dw2, db2;
   const int64_t ldx = row_stride(x, "x"), ld1 = row_stride(w1, "w1"), ld2 = row_stride(w2, "w2");

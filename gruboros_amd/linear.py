@@ -267,10 +267,16 @@ class F32Linear(torch.autograd.Function):
         return dx, dw, db
 
 
-def f32_linear_applies(x, w):
-    """Whether F32Linear takes x [.., K] and w [O, K]: fp32 CUDA tensors, O and K multiples of 8."""
+def _f32_weight(x, w):
+    """Whether w [O, K] is a weight for the fp32 products of x's path: fp32 on the GPU, O and K multiples of 8."""
     return x.is_cuda and x.dtype == torch.float32 and w.dtype == torch.float32 and w.dim() == 2 and \
         w.shape[0] % 8 == 0 and w.shape[1] % 8 == 0
+
+
+def f32_linear_applies(x, w):
+    """Whether F32Linear takes x [.., K] and w [O, K]: fp32 CUDA tensors, O and K multiples of 8.
+    Widths that differ are not taken, so that nn.Linear's own error is raised for them."""
+    return _f32_weight(x, w) and x.shape[-1:] == w.shape[1:]
 
 
 def f32_linear(x, w, b=None):
@@ -421,8 +427,8 @@ def feed_forward(x, ff):
     """ff = nn.Sequential(Linear, GELU, Linear) applied to x in x's dtype."""
     l1, l2 = ff[0], ff[2]
     if x.dtype == l1.weight.dtype:
-        if (f32_linear_applies(x, l1.weight) and f32_linear_applies(x, l2.weight) and l1.bias is not None and
-                l2.bias is not None and x.shape[-1] == l1.weight.shape[1] and l1.weight.shape[0] == l2.weight.shape[1]):
+        if (f32_linear_applies(x, l1.weight) and _f32_weight(x, l2.weight) and l1.bias is not None and
+                l2.bias is not None and l1.weight.shape[0] == l2.weight.shape[1]):
             y = F32FeedForward.apply(x.reshape(-1, x.shape[-1]).contiguous(), l1.weight, l1.bias, l2.weight, l2.bias)
             return y.view(*x.shape[:-1], l2.weight.shape[0])
         return linear(F.gelu(linear(x, l1)), l2)

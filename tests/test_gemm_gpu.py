@@ -930,3 +930,44 @@ def test_f32_layers_refuse_what_the_kernels_cannot_read(op, bad):
         else:
             first = torch.nn.Linear(32, 64, device="cuda")
             feed_forward(torch.randn(8, 32, device="cuda"), torch.nn.Sequential(first, torch.nn.GELU(), last))
+
+
+@pytest.mark.parametrize("op", ["linear", "feed_forward", "feed_forward, second layer", "loss"])
+def test_f32_layers_refuse_an_input_of_another_width(op):
+    """An fp32 input narrower or wider than the layer is nn.Linear's error, not a product with the first
+    columns of the weight."""
+    from gruboros_amd.linear import feed_forward, linear
+    from gruboros_amd.loss import logits_cross_entropy
+
+    with torch.device(DEV):
+        layer, inner = torch.nn.Linear(64, 32), torch.nn.Linear(32, 128)
+        labels = torch.zeros(8, dtype=torch.long)
+    for width in (56, 72):
+        x = torch.randn(8, width, device=DEV)
+        with pytest.raises(RuntimeError):
+            if op == "linear":
+                linear(x, layer)
+            elif op == "feed_forward":
+                feed_forward(x, torch.nn.Sequential(layer, torch.nn.GELU(), inner))
+            elif op == "feed_forward, second layer":
+                feed_forward(torch.randn(8, 64, device=DEV), torch.nn.Sequential(
+                    torch.nn.Linear(64, width, device=DEV), torch.nn.GELU(), layer))
+            else:
+                logits_cross_entropy(x, layer, labels)
+
+
+@pytest.mark.parametrize("a_layout,b_layout", [(0, 0), (0, 1), (1, 1), (1, 0)])
+@pytest.mark.parametrize("short", ["a rows", "a columns", "b rows", "b columns", "out rows", "out columns"])
+def test_gemm_f32_refuses_operands_of_other_extents(a_layout, b_layout, short):
+    """gemm_f32 compares every operand with M, N and K on the host: the kernel would read or write past
+    a smaller one."""
+    from gruboros_amd._lib import MingruHipError
+    from gruboros_amd.gemm import gemm_f32
+
+    M, N, K = 136, 72, 264
+    t = {"a": torch.randn((M, K) if a_layout == 0 else (K, M), device=DEV),
+         "b": torch.randn((N, K) if b_layout == 0 else (K, N), device=DEV), "out": torch.zeros(M, N, device=DEV)}
+    name, dim = short.split()
+    t[name] = t[name][:-8] if dim == "rows" else t[name][:, :-8]
+    with pytest.raises(MingruHipError, match="expected"):
+        gemm_f32(t["a"], a_layout, t["b"], b_layout, M, N, K, out=t["out"])
