@@ -131,7 +131,7 @@ void gemm(int al, Mat a, int bl, Mat b, int64_t M, int64_t N, int64_t K, int epi
 
 // x w^T (+ bias, + GELU with the pre-activation kept) [N, O], bf16; x [N, K], w [O, K]
 Tensor linear_fwd(const Tensor& x, const Tensor& w, const float* bias, const Tensor* pre, int64_t stream) {
-  const int64_t n = x.size(0), k = x.size(1), o = w.size(0);
+  const int64_t n = x.size(0), k = x.size(1), o = extent(w, w.size(0), k, "w").size(0);
   Tensor y = make({n, o}, at::kBFloat16, x);
   const Mat xm = mat(x, "x"), wm = mat(w, "w"), ym = mat(y, "y");
   const int epi = pre ? MG_EPI_BIAS_GELU : bias ? MG_EPI_BIAS : MG_EPI_NONE;
@@ -153,7 +153,7 @@ void linear_fwd_hilo(Mat x, Mat w, int64_t n, int64_t o, int64_t k, int c_dtype,
 
 // dy w [N, K] for dy [N, O] bf16, w [O, K] bf16: bf16 rounded stochastically, or fp32
 Tensor linear_dx(const Tensor& dy, const Tensor& w, bool f32, int64_t stream) {
-  const int64_t n = dy.size(0), o = dy.size(1), k = w.size(1);
+  const int64_t n = dy.size(0), o = dy.size(1), k = extent(w, o, w.size(-1), "w").size(1);
   Tensor dx = make({n, k}, f32 ? at::kFloat : at::kBFloat16, dy);
   const Mat dm = mat(dy, "dy"), wm = mat(w, "w"), xm = mat(dx, "dx");
   const int64_t step = row_step(n, std::max(2 * dm.ld, k * xm.esize));
@@ -203,7 +203,7 @@ struct DW {
   Opt into;
 };
 std::optional<std::vector<Tensor>> group(const Tensor& dy, const Tensor& w, const std::vector<DW>& dws, int64_t stream) {
-  const int64_t n = dy.size(0), o = dy.size(1), k = w.size(1);
+  const int64_t n = dy.size(0), o = dy.size(1), k = extent(w, o, w.size(-1), "w").size(1);
   const Mat dm = mat(dy, "dy"), wm = mat(w, "w");
   const auto span = [](int64_t rows, int64_t ld) { return (rows + 512) * ld * 2 < (int64_t(1) << 31); };
   bool ok = span(n, dm.ld) && span(o, wm.ld) && (dws.size() == 1 || dws.size() == 2);
@@ -320,6 +320,7 @@ typedef std::tuple<Opt, Tensor, Tensor, Opt> NormOut;
 // (x + delta or none, y, rstd, pair or none) of rows x [..., D]; with_lo: y is the first half of pair
 NormOut norm_fwd(const Tensor& x, const Opt& delta, const Tensor& w, bool bf16, bool with_lo, int64_t stream) {
   const int64_t D = x.size(-1), N = x.numel() / std::max<int64_t>(D, 1);
+  if (delta && delta->numel() != x.numel()) fail("delta: expected as many values as x has");
   Opt pair, x_out;
   Tensor y;
   if (with_lo) {
@@ -332,7 +333,7 @@ NormOut norm_fwd(const Tensor& x, const Opt& delta, const Tensor& w, bool bf16, 
   }
   Tensor rstd = make({N}, at::kFloat, x);
   if (delta) x_out = make(x.sizes(), at::kFloat, x);
-  check(mg_add_rmsnorm_fwd(fp(x), delta ? code(*delta) : 0, ptr(delta), fp(w), fp(x_out), bf16 || with_lo ? MG_BF16 : MG_F32,
+  check(mg_add_rmsnorm_fwd(fp(x), delta ? code(*delta) : 0, ptr(delta), vec(w, D, "norm weight"), fp(x_out), bf16 || with_lo ? MG_BF16 : MG_F32,
                            ptr(y), with_lo ? h16(*pair) + D : nullptr, with_lo ? 2 * D : D, fp(rstd), N, D, kEps, st(stream)),
         "mg_add_rmsnorm_fwd");
   return {x_out, y, rstd, pair};
@@ -351,7 +352,8 @@ std::tuple<Opt, Opt, Tensor> norm_bwd(const Tensor& xn, const Tensor& w, const T
   Tensor dw = make({D}, at::kFloat, xn);
   const size_t wsb = mg_add_rmsnorm_bwd_workspace_bytes(N, D);
   Tensor ws = bytes(wsb, xn);
-  check(mg_add_rmsnorm_bwd_scaled(fp(xn), fp(w), fp(rstd), code(dy), ptr(dy), fp(scale), fp(dres), fp(dx),
+  if (dy.numel() != xn.numel() || (dres && dres->numel() != xn.numel())) fail("norm gradient: expected as many values as x has");
+  check(mg_add_rmsnorm_bwd_scaled(fp(xn), vec(w, D, "norm weight"), vec(rstd, N, "rstd"), code(dy), ptr(dy), fp(scale), fp(dres), fp(dx),
                                   std::max(delta_type, 0), ptr(dd), fp(dw), N, D, ptr(ws), wsb, st(stream)),
         "mg_add_rmsnorm_bwd");
   return {dx, dd, dw};
@@ -447,6 +449,12 @@ GruOut gru_forward(const Tensor& x, const Opt& pending, const Tensor& w_norm, co
                    const Opt& to_pair, const Opt& h0, int64_t B, int64_t T, bool residual, bool one_launch, const Tensor& ws,
                    int64_t stream) {
   const int64_t N = x.size(0), D = x.size(1), Di = w_pair.size(0) / 2;
+  if (N != B * T) fail("x: expected B * T rows");
+  extent(w_pair, 2 * Di, 2 * D, "w_pair");
+  extent(w_bf16, 2 * Di, D, "w_bf16");
+  if (to_pair) extent(*to_pair, D, 2 * Di, "to_out's pair");
+  else if (residual && Di != D) fail("without to_out the scan's width is x's");
+  if (h0) vec(*h0, B * Di, "h0");
   auto [x_out, n, rstd, pair] = norm_fwd(x, pending, w_norm, true, true, stream);
   Tensor hg = make({N, 2 * Di}, at::kBFloat16, x);
   const Mat pm = mat(*pair, "pair"), wm = mat(w_pair, "w_pair"), hm = mat(hg, "hg");
@@ -496,6 +504,11 @@ GruGrads gru_backward(const Tensor& xn, const Tensor& w_norm, const Tensor& rstd
                       bool want_to, bool want_dh0, bool pair_launch, const Opt& into_hg, const Opt& into_to, const Tensor& ws,
                       int64_t stream) {
   const int64_t N = xn.size(0), D = xn.size(1), Di = hg.size(1) / 2;
+  extent(hg, N, 2 * Di, "hg");
+  extent(pair, N, 2 * D, "pair");
+  extent(w_bf16, 2 * Di, D, "w_bf16");
+  if (h_pair) extent(*h_pair, N, 2 * Di, "h_pair");
+  if (to_bf16) extent(*to_bf16, D, Di, "to_out's weight");
   Opt dh, dW_to, dW_hg, dh0;
   Tensor dob;
   if (ckpt && !h_pair) {
@@ -562,6 +575,8 @@ GruGrads gru_backward(const Tensor& xn, const Tensor& w_norm, const Tensor& rstd
 typedef std::tuple<Opt, Tensor, Tensor, Tensor, Tensor, Tensor> FFOut;
 FFOut ff_forward(const Tensor& x1, const Opt& out, const Tensor& w_norm, const Tensor& w1, const Tensor& b1, const Tensor& w2,
                  const Tensor& b2, int64_t stream) {
+  extent(w1, w1.size(0), x1.size(1), "w1");
+  extent(w2, w2.size(0), w1.size(0), "w2");
   auto [x2, n2, rstd, none] = norm_fwd(x1, out, w_norm, true, false, stream);
   Tensor pre = make({x1.size(0), w1.size(0)}, at::kBFloat16, x1);
   Tensor act = linear_fwd(n2, w1, vec(b1, w1.size(0), "b1"), &pre, stream);     // pre = n2 W1^T + b1, act = gelu(pre)
@@ -588,6 +603,9 @@ FFGrads ff_backward(const Tensor& x2, const Tensor& w_norm, const Tensor& rstd, 
                     const Tensor& act, const Tensor& w1, const Tensor& w2, const Opt& dx2, const Tensor& dp, bool pair_launch,
                     const Opt& into1, const Opt& into2, int64_t stream) {
   const int64_t N = x2.size(0), D = x2.size(1), F = pre.size(1);
+  extent(n2, N, D, "n2");
+  extent(act, N, F, "act");
+  extent(dp, N, D, "dpend");
   Tensor dact = linear_dx(dp, w2, false, stream);
   auto [dpre, db1, db2] = ff_bias_bwd(dact, pre, dp, stream);
   const Mat dpm = mat(dp, "dpend"), am = mat(act, "act"), dm = mat(dpre, "dpre"), nm = mat(n2, "n2");
@@ -618,7 +636,9 @@ FFGrads ff_backward(const Tensor& x2, const Tensor& w_norm, const Tensor& rstd, 
 // FinalNormCE.forward: (loss, x + pending or none, embed, rstd, dlogits); w bf16 [V, D]
 std::tuple<Tensor, Opt, Tensor, Tensor, Tensor> head_forward(const Tensor& x, const Opt& pending, const Tensor& w_norm,
                                                              const Tensor& w, const Tensor& labels, int64_t stream) {
-  const int64_t N = x.size(0), D = x.size(1), V = w.size(0);
+  const int64_t N = x.size(0), D = x.size(1), V = extent(w, w.size(0), D, "w").size(0);
+  if (labels.scalar_type() != at::kLong || labels.numel() != N || !labels.is_contiguous())
+    fail("labels: expected one contiguous int64 value per row");
   auto [x_out, embed, rstd, none] = norm_fwd(x, pending, w_norm, true, false, stream);
   Tensor dl = make({N, V}, at::kBFloat16, x), part = make({mg_logits_cross_entropy_partials(N)}, at::kFloat, x);
   check(mg_logits_cross_entropy(ptr(embed), D, ptr(w), row_stride(w, "w"), static_cast<int64_t*>(ptr(labels)), ptr(dl), V,
@@ -687,8 +707,8 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> infer_layer(const Tensor& x, c
   }
   if (f32) return std::make_tuple(x2, std::get<2>(ff_f32_forward(n2, w1, b1, w2, b2, false, stream)), last);
   Tensor pre = make({N, F}, at::kBFloat16, x);  // (the epilogue rounds it to bf16; its values are not used)
-  Tensor act = linear_fwd(n2, w1, fp(b1), &pre, stream);
-  return std::make_tuple(x2, linear_fwd(act, w2, fp(b2), nullptr, stream), last);
+  Tensor act = linear_fwd(n2, w1, vec(b1, F, "b1"), &pre, stream);
+  return std::make_tuple(x2, linear_fwd(act, w2, vec(b2, D, "b2"), nullptr, stream), last);
 }
 
 // Column sums of a 2-D fp32 or bf16 tensor with unit inner stride, fp32.

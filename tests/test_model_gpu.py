@@ -829,3 +829,31 @@ def test_prompt_follows_what_a_program_changes(dtype, change):
         assert _rel(before, outs[1][0]) > 0.1
     for got, ref in zip(*outs):
         assert _rel(got, ref) < (2e-2 if dtype == torch.bfloat16 else 1e-5)
+
+
+@pytest.mark.parametrize("bad", ["norm weight", "pending", "to_hidden_and_gate", "to_out", "h0", "ff norm weight", "w1", "w2",
+                                 "b1", "labels", "int32 labels", "head weight"])
+def test_blocks_refuse_operands_of_other_extents(bad):
+    """The block passes read their operands through raw pointers: one that is smaller or wider than the
+    block's sizes is an error on the host, before any launch."""
+    from gruboros_amd import blocks
+    from gruboros_amd._lib import MingruHipError
+
+    B, T, D, Di, Fw, V = 2, 9, 64, 128, 96, 32
+    with torch.device("cuda"):
+        t = {"x": torch.randn(B, T, D), "pending": torch.randn(B, T, D).bfloat16(), "norm weight": torch.ones(D),
+             "to_hidden_and_gate": torch.randn(2 * Di, D), "to_out": torch.randn(D, Di), "h0": torch.rand(B, 1, Di),
+             "ff norm weight": torch.ones(D), "w1": torch.randn(Fw, D), "b1": torch.randn(Fw), "w2": torch.randn(D, Fw),
+             "b2": torch.randn(D), "head weight": torch.randn(V, D), "labels": torch.zeros(B, T, dtype=torch.long)}
+    if bad == "int32 labels":
+        t["labels"] = t["labels"].int()
+    elif bad == "labels":
+        t["labels"] = t["labels"][:, :-1]
+    elif bad == "pending":
+        t[bad] = t[bad][:, :, :-8].contiguous()
+    else:
+        t[bad] = t[bad][..., :-8].contiguous()
+    with torch.no_grad(), pytest.raises((MingruHipError, RuntimeError), match="expected|shape|invalid"):
+        blocks.MinGRUBlock.apply(t["x"], t["pending"], t["norm weight"], t["to_hidden_and_gate"], t["h0"], t["to_out"])
+        blocks.FFBlock.apply(t["x"], None, t["ff norm weight"], t["w1"], t["b1"], t["w2"], t["b2"])
+        blocks.FinalNormCE.apply(t["x"], t["pending"], t["norm weight"], t["head weight"], t["labels"])
