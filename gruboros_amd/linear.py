@@ -289,11 +289,13 @@ def f32_linear(x, w, b=None):
 class F32FeedForward(torch.autograd.Function):
     """Linear -> GELU -> Linear (reference mingru/minLM.py:17-23) for fp32 x [N, D] and fp32 weights and
     biases, every product on mg_gemm_f32: the first with bias and GELU in its epilogue (the pre-activation
-    kept for the backward), the backward's dy W2 with the GELU gradient in its."""
+    kept for the backward), the backward's dy W2 with the GELU gradient in its. grad: whether gradients are
+    on at the call (inside forward nothing tells: needs_input_grad is true for a parameter under no_grad
+    too); without them the pre-activation is neither kept nor written."""
 
     @staticmethod
-    def forward(ctx, x, w1, b1, w2, b2):
-        train = any(ctx.needs_input_grad)
+    def forward(ctx, x, w1, b1, w2, b2, grad):
+        train = grad and any(ctx.needs_input_grad)
         pre, act, y = native().ff_f32_forward(x, w1, b1.contiguous(), w2, b2.contiguous(), train, stream_of(x))
         if train:
             ctx.save_for_backward(x, pre, act, w1, w2)
@@ -302,7 +304,7 @@ class F32FeedForward(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         x, pre, act, w1, w2 = ctx.saved_tensors
-        return native().ff_f32_backward(x, pre, act, w1, w2, dy.contiguous(), *ctx.needs_input_grad, stream_of(x))
+        return (*native().ff_f32_backward(x, pre, act, w1, w2, dy.contiguous(), *ctx.needs_input_grad[:5], stream_of(x)), None)
 
 
 class BF16Linear(torch.autograd.Function):
@@ -429,7 +431,8 @@ def feed_forward(x, ff):
     if x.dtype == l1.weight.dtype:
         if (f32_linear_applies(x, l1.weight) and _f32_weight(x, l2.weight) and l1.bias is not None and
                 l2.bias is not None and l1.weight.shape[0] == l2.weight.shape[1]):
-            y = F32FeedForward.apply(x.reshape(-1, x.shape[-1]).contiguous(), l1.weight, l1.bias, l2.weight, l2.bias)
+            y = F32FeedForward.apply(x.reshape(-1, x.shape[-1]).contiguous(), l1.weight, l1.bias, l2.weight, l2.bias,
+                                     torch.is_grad_enabled())
             return y.view(*x.shape[:-1], l2.weight.shape[0])
         return linear(F.gelu(linear(x, l1)), l2)
     if x.dtype != torch.bfloat16 or l1.weight.dtype != torch.float32:

@@ -971,3 +971,34 @@ def test_gemm_f32_refuses_operands_of_other_extents(a_layout, b_layout, short):
     t[name] = t[name][:-8] if dim == "rows" else t[name][:, :-8]
     with pytest.raises(MingruHipError, match="expected"):
         gemm_f32(t["a"], a_layout, t["b"], b_layout, M, N, K, out=t["out"])
+
+
+@pytest.mark.parametrize("D,Fw", [(64, 96), (512, 2048)])
+def test_f32_feed_forward_keeps_the_pre_activation_only_for_a_backward(D, Fw, monkeypatch):
+    """Under no_grad, and for inputs and weights that need no gradient, the fp32 FeedForward runs the
+    epilogue that writes no pre-activation, with the same output bit for bit; with gradients it keeps it."""
+    from gruboros_amd import linear as lin
+
+    kept = []
+
+    class Native:
+        def __getattr__(self, name):
+            return getattr(real, name)
+
+        def ff_f32_forward(self, *args):
+            out = real.ff_f32_forward(*args)
+            kept.append(out[0] is not None)
+            return out
+
+    real = lin.native()
+    monkeypatch.setattr(lin, "native", lambda: Native())
+    torch.manual_seed(3)
+    ff = torch.nn.Sequential(torch.nn.Linear(D, Fw), torch.nn.GELU(), torch.nn.Linear(Fw, D)).to(DEV)
+    x = torch.randn(333, D, device=DEV)
+    y = lin.feed_forward(x, ff)
+    with torch.no_grad():
+        without = lin.feed_forward(x, ff)
+    ff.requires_grad_(False)
+    frozen = lin.feed_forward(x, ff)
+    assert kept == [True, False, False] and y.requires_grad and not without.requires_grad and not frozen.requires_grad
+    assert torch.equal(without, y) and torch.equal(frozen, y)
