@@ -73,6 +73,12 @@ def _ff(x, ff):
     return feed_forward(x, ff)
 
 
+def _idle(dropout):
+    """Whether calling this dropout does nothing: off, and no hook of its own or of all modules runs."""
+    return (type(dropout) is nn.Dropout and not dropout.training and not dropout._forward_hooks
+            and not dropout._forward_pre_hooks and not torch.nn.modules.module._has_any_global_hook())
+
+
 class minLM(Module):
     """Reference mingru/minLM.py:43-206.
 
@@ -253,11 +259,11 @@ class minLM(Module):
 
     def _infer_applies(self, cd):
         """Whether the forward may run layer by layer in native code: no gradients of any mode, no
-        autocast, no conv, no dropout that acts (each layer's own mode counts: dropout may be kept on
-        in an eval() model), plain minGRU layers without biases, and parameters in the activation dtype."""
+        autocast, no conv, no dropout that acts or is watched (each layer's own mode counts: dropout may
+        be kept on in an eval() model), plain minGRU layers without biases, and parameters in the activation dtype."""
         return (not torch.is_grad_enabled() and cd == self.token_emb.weight.dtype and not torch.is_autocast_enabled()
                 and torch.autograd.forward_ad._current_level < 0
-                and all(conv is None and (dropout is None or (type(dropout) is nn.Dropout and not dropout.training))
+                and all(conv is None and (dropout is None or _idle(dropout))
                         and type(mingru) is minGRU and mingru.to_hidden_and_gate.bias is None
                         and getattr(mingru.to_out, "bias", None) is None
                         for conv, _, mingru, _, _, dropout in self.layers))

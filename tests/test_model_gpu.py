@@ -791,8 +791,9 @@ def test_prompt_follows_what_a_program_changes(dtype, change):
     """The no-grad forward runs layer by layer in native code where its kernels say the same as the op by
     op one. A dropout that stays on in an eval() model, a bias a program gave to_out, a parameter changed
     through .data after a first call, and a layer only the op by op path takes (with the states handed over
-    as an iterator) give the forward with gradients' result. Both paths round at the same places but for
-    the GELU's input and the residual's branches: 4e-3 in bf16 over 12 layers, 1e-6 in fp32."""
+    as an iterator) give the forward with gradients' result. Both paths round at the same places: at these
+    sizes (two layers, 37 positions) they measured equal bit for bit in both types; where a product's sum is
+    split another way, bf16 roundings flip (5e-3 over 12 layers of d1024), hence 2e-2 and, in fp32, 1e-5."""
     from gruboros_amd.mingru.minLM import minLM
 
     torch.manual_seed(5)
@@ -857,3 +858,36 @@ def test_blocks_refuse_operands_of_other_extents(bad):
         blocks.MinGRUBlock.apply(t["x"], t["pending"], t["norm weight"], t["to_hidden_and_gate"], t["h0"], t["to_out"])
         blocks.FFBlock.apply(t["x"], None, t["ff norm weight"], t["w1"], t["b1"], t["w2"], t["b2"])
         blocks.FinalNormCE.apply(t["x"], t["pending"], t["norm weight"], t["head weight"], t["labels"])
+
+
+@pytest.mark.parametrize("where", ["forward", "pre", "global"])
+def test_prompt_runs_the_hooks_of_an_idle_dropout(where):
+    """A hook on a dropout that is off (a program watching the residual stream) runs in the no-grad
+    forward too, once per layer, and what it returns is used."""
+    from gruboros_amd.mingru.minLM import minLM
+
+    torch.manual_seed(6)
+    with torch.device(DEV):
+        model = minLM(num_tokens=256, dim=64, depth=3, ff_mult=2, expansion=1.0, dropout=0.5).eval()
+    ids = torch.randint(0, 256, (2, 17), device=DEV)
+    calls = []
+
+    def hook(module, args, out=None):
+        if type(module) is torch.nn.Dropout:
+            calls.append(tuple(args[0].shape))
+            return args[0] * 0 if out is None else out * 0
+
+    with torch.no_grad():
+        before = model(ids)
+        if where == "global":
+            handles = [torch.nn.modules.module.register_module_forward_hook(hook)]
+        else:
+            handles = [getattr(layer[5], f"register_forward_{'pre_' if where == 'pre' else ''}hook")(hook) for layer in model.layers]
+        try:
+            hooked = model(ids)
+        finally:
+            for h in handles:
+                h.remove()
+        after = model(ids)
+    assert calls == [(2, 17, 64)] * 3
+    assert torch.equal(before, after) and float(hooked.abs().max()) == 0.0  # norm of zeros
