@@ -1553,6 +1553,18 @@ __device__ __forceinline__ void gemm_tile(const Params& p, int bx, int by) {
       // The GELU epilogues stay runtime loops (unrolled they are more code
       // than the instruction cache holds); the others are unrolled.
       constexpr int kStoreUnroll = (EPI == EPI_BIAS_GELU || EPI == EPI_GELU_GRAD) ? 2 : 32;
+      // C's old values, with one workgroup per CU: all of the block's loads go out before its
+      // first store (a load after a store to the same array waits for it, one memory latency per
+      // row group: 1421 x 1536 x 1536 26.1 against 23 us); clamped, so unconditional. Several
+      // workgroups hide each other's waits (4096 x 2048 x 300: 21.4 batched, 19.4 not).
+      constexpr bool kBatchOld = CMODE == C_ADD && DEEP;
+      f4 old[kBatchOld ? 32 / RPI : 1];
+      if constexpr (kBatchOld) {
+        const float* cp = static_cast<const float*>(p.C) + min(ncol, p.N - 4);
+#pragma unroll
+        for (int t = 0; t < 32 / RPI; ++t)
+          old[t] = io4<float>::load(cp + static_cast<int64_t>(min(row0 + i * 32 + t * RPI + lane / CQ, p.M - 1)) * p.ldc);
+      }
 #pragma unroll kStoreUnroll
       for (int t = 0; t < 32 / RPI; ++t) {
         const int r = t * RPI + lane / CQ;
@@ -1583,9 +1595,9 @@ __device__ __forceinline__ void gemm_tile(const Params& p, int bx, int by) {
             x.v[3] *= gelu_grad(__uint_as_float(w.y & 0xffff0000u));
           }
           if constexpr (CMODE == C_ADD) {
-            const f4 old = io4<float>::load(reinterpret_cast<const float*>(cp));
+            if constexpr (!kBatchOld) old[0] = io4<float>::load(reinterpret_cast<const float*>(cp));
 #pragma unroll
-            for (int e = 0; e < 4; ++e) x.v[e] = old.v[e] + x.v[e];
+            for (int e = 0; e < 4; ++e) x.v[e] = old[kBatchOld ? t : 0].v[e] + x.v[e];
           }
           if constexpr (EPI == EPI_GELU_GRAD || EPI == EPI_SR)  // gradients: stochastic rounding (mg_common.h)
             io4<TC>::store_grad(cp, x, static_cast<uint32_t>(static_cast<int64_t>(m) * p.N + n), 0x9e5bu);
@@ -2814,23 +2826,27 @@ inline bool hilo_cols_ok(int M, int N, int K) {
   return M >= 1 && N >= 1 && K >= 32 && K % 32 == 0 && int64_t((M + 255) / 256) * ((N + 127) / 128) <= 192;
 }
 
-// fp32 hi/lo products (to_out) of at most one 256 x 128 tile per CU
-// (gemm_t128_kernel), whole 32-k steps, from 3e9 multiply-adds: split along K
-// to at most one workgroup per CU, by estimated time: 0.85 us per step, 8 us to
-// start and store, partials written and read at about 7.4 TB/s plus 4 us for
-// their reduction (2048 rows, d1024, e3: 57 -> 43 us in the block). Smaller
-// ones are 1 to 3 us faster on 128 x 128 tiles, which start sooner. Never with
-// MG_GEMM_DETERMINISTIC: these tiles sum the three hi/lo products per 32 k, the
-// others one after the other over all of K, and there a row's result must not
-// depend on how many rows come with it.
+// fp32 hi/lo products (to_out) on 256 x 128 tiles (gemm_t128_kernel), whole
+// 32-k steps, at most one tile per CU, split along K to at most one workgroup
+// per CU by estimated time: 0.85 us per step, 8 us to start and store, partials
+// written and read at about 7.4 TB/s plus 4 us for their reduction. They take a
+// product where the 128 x 128 tiles are too many to split (over 256) and K is
+// 1024 or more, or where it has 6e9 multiply-adds and fills 80% of the chip's
+// tile slots. Against plan()'s tiles, us: 4226 x 1536 x 6144 253 -> 209, 2048 x
+// 1024 x 3072 48.3 -> 47.0, 2048 x 2048 x 8192 191 -> 172; outside the rule
+// 13798 x 384 x 768 33.7 -> 35.2, 2048 x 1024 x 1536 32.5 -> 34.3 (3.2e9), 6040 x
+// 512 x 8192 156 -> 173 (74% of the slots). Never with MG_GEMM_DETERMINISTIC:
+// these tiles sum the three hi/lo products per 32 k, the others one after the
+// other over all of K, and there a row's result must not depend on how many rows
+// come with it.
 struct HiloPlan {
   bool ok;
   int kt_per_split, splits;
 };
 inline HiloPlan hilo_plan(int M, int N, int K, bool whole) {
   HiloPlan best{};
-  const int64_t T = int64_t((M + 255) / 256) * ((N + 127) / 128);
-  if (M < 1 || N < 1 || K < 32 || K % 32 || T > kCUs || double(M) * N * K < 3e9) return best;
+  const int64_t T = int64_t((M + 255) / 256) * ((N + 127) / 128), t128 = int64_t((M + 127) / 128) * ((N + 127) / 128);
+  if (M < 1 || N < 1 || K < 32 || K % 32 || T > kCUs) return best;
   const int steps = K / 32;
   double least = 1e300;
   for (int s = 1; s == 1 || (!whole && s * T <= kCUs && steps / s >= 4); ++s) {
@@ -2838,24 +2854,43 @@ inline HiloPlan hilo_plan(int M, int N, int K, bool whole) {
     const double cost = 0.85 * kt + 8.0 + (ys > 1 ? 4.0 + double(ys) * M * N * 8.0 / 7.4e6 : 0.0);
     if (cost < least) least = cost, best = HiloPlan{true, kt, ys};
   }
+  best.ok = (t128 > kCUs && K >= 1024) ||
+            (double(M) * N * K >= 6e9 && double(best.splits) * M * N >= 0.8 * kCUs * 256 * 128);
   return best;
 }
 
-// Tile size and K split of a product (measured on MI355X): 256 x 256 tiles for
-// weight gradients (both operands MN-contiguous) of whole 256 x 256 tiles, at
-// least 16 of them, K >= 4096, split along K to about one workgroup per CU, and
-// for the other layouts when that still gives every CU a tile; everything else
-// 128 x 128, split along K (outputs and epilogues that allow it) to about one
-// workgroup per CU. `ysplits` is the split count the launch uses (gridDim.y).
+// Tile size and K split of a product. 256 x 256 tiles (`big`) for weight
+// gradients (both operands MN-contiguous) of whole 256 x 256 tiles, at least 16
+// of them, K >= 4096, split along K to about one workgroup per CU, and for the
+// other layouts when that still gives every CU a tile. Everything else on
+// smaller tiles, split along K where output and epilogue allow it:
+//   small  64 x 64, four LDS stages, two workgroups per CU;
+//   deep   128 x 128, four stages, one workgroup per CU;
+//   else   128 x 128, two stages, two workgroups per CU.
+// A workgroup's k-tile costs the four-stage loop about 0.50 us (0.63 with an
+// MN-contiguous B) and two two-stage workgroups of a CU 0.92 (1.0) together, so
+// the two-stage loop wins where a workgroup has many k-tiles, the four-stage one
+// where the fixed cost of a workgroup and the partials of twice the splits
+// weigh more. The lines between them are numbers of k-tiles per workgroup,
+// taken from 505 sizes of 16 to 16376 rows, N and K 256 to 8192, each timed on
+// every plan (us, small | deep | two stages):
+//   2048 x 1024 x 1536   13.9 |  -   | 22.0     24 k-tiles, whole
+//    777 x 1024 x 3072   16.3 | 19.2 | 22.8     24
+//    827 x 1152 x 8192   39.0 | 43.1 | 28.4     64
+//   1200 x 3072 x 1152     -  | 17.0 | 25.1     18, whole
+//    777 x 2048 x 8192     -  | 43.3 | 38.5     64
+//   1896 x 1304 x 5832     -  | 60.4 | 52.9     92, whole
+// `ysplits` is the split count the launch uses (gridDim.y).
 struct Plan {
   bool big, deep, small;
   int tiles, kt_per_split, ysplits;
 };
 
 inline Plan plan(int M, int N, int K, bool ak, bool bk, int c_dtype, int epilogue, bool deterministic, bool hilo) {
-  Plan pl;
+  Plan pl{};
   const int64_t t256 = int64_t((M + 255) / 256) * ((N + 255) / 256);
   const int64_t t128 = int64_t((M + 127) / 128) * ((N + 127) / 128);
+  const int64_t t64 = int64_t((M + 63) / 64) * ((N + 63) / 64);
   const bool wgrad = !ak && !bk;
   // weight gradients whose output dimensions are multiples of 256 run 256 x 256
   // tiles (half the L2 traffic per flop of 128 x 128), split along K to about
@@ -2874,31 +2909,64 @@ inline Plan plan(int M, int N, int K, bool ak, bool bk, int c_dtype, int epilogu
   const int64_t tiles = pl.big ? t256 : t128;
   pl.tiles = static_cast<int>(tiles);
   const int nkt = (hilo ? 3 : 1) * ((K + BK - 1) / BK);
-  // 64 x 64 tiles (four stages of 16 KB, two workgroups per CU) for short products of few
-  // tiles, whole instead of split along K (us, 2048 x 1024 x 1536 22.0 -> 13.9, 777 x 1024 x 1536 17.1 -> 9.9, weight gradient 1536 x 384 x
-  // 667 13.2 -> 7.2), and for the bias + GELU product,
-  // which is never split and whose erf runs after the tile's MFMAs, 64 values a thread on
-  // 128 x 128 tiles (777 x 1536 x 1024 23.3 -> 11.7, 2048 x 1536 x 1024 24.8 -> 19.7).
-  const int64_t t64 = int64_t((M + 63) / 64) * ((N + 63) / 64);
-  pl.small = !pl.big && !hilo && ((nkt <= 24 && t64 <= 2 * kCUs) || (epilogue == MG_EPI_BIAS_GELU && t128 <= kCUs));
-  int splits = 1;
   // fp32 outputs and plain bf16 outputs (no epilogue or a bias, no hi/lo operands; a
   // stochastically rounded gradient among them) split K when the tiles leave CUs idle: partials
   // in fp32, then split_reduce_kernel (fp32) or split_reduce_bf16_kernel (bias added, rounded as
   // the unsplit epilogue would). Hi/lo bf16 products stay whole, equal to mg_gemm_hilo_prefix's
-  // columns. 128 x 128 tiles aim at one workgroup per CU with four LDS stages (pl.deep); two per
-  // CU with two stages each, i.e. twice the partials, measured (us) 23.9 against 15.6 at 2048 x
-  // 1536 x 1024, 24.9 against 22.2 at 2048 x 1024 x 1536, 22.8 against 19.2 at 777 x 1024 x 3072.
-  const bool split_ok = c_dtype == MG_F32 || (c_dtype == MG_BF16 && !hilo);
-  const bool epi_ok = epilogue == MG_EPI_NONE || (epilogue == MG_EPI_BIAS && c_dtype == MG_BF16 && !hilo);
-  if (!pl.big && !pl.small && !hilo && epi_ok && split_ok && !deterministic && t64 <= kCUs) {
-    pl.small = true;  // longer ones split to two workgroups per CU (777 x 1024 x 3072 19.7 -> 16.3 us)
-    splits = static_cast<int>(std::min<int64_t>(2 * kCUs / t64, nkt / 6));
-  } else if (epi_ok && split_ok && tiles < kCUs && !deterministic && !pl.small)
-    splits = static_cast<int>(std::min<int64_t>(std::max<int64_t>(kCUs / tiles, 1), std::max(nkt / 4, 1)));
-  pl.kt_per_split = std::max((nkt + splits - 1) / splits, 1);
-  pl.ysplits = std::max((nkt + pl.kt_per_split - 1) / pl.kt_per_split, 1);
-  pl.deep = !pl.big && tiles * pl.ysplits <= kCUs;
+  // columns.
+  const bool may_split = !deterministic && (c_dtype == MG_F32 || !hilo) &&
+                         (epilogue == MG_EPI_NONE || (epilogue == MG_EPI_BIAS && c_dtype == MG_BF16 && !hilo));
+  const auto split = [&](int64_t want) {
+    const int64_t n = std::max<int64_t>(want, 1);
+    pl.kt_per_split = std::max(static_cast<int>((nkt + n - 1) / n), 1);
+    pl.ysplits = std::max((nkt + pl.kt_per_split - 1) / pl.kt_per_split, 1);
+    return pl.kt_per_split;
+  };
+  // splits that give `slots` workgroups, each at least 4 k-tiles
+  const auto fill = [&](int64_t slots) { return may_split ? std::min<int64_t>(slots / tiles, nkt / 4) : 1; };
+  // Whether the launch is split and its workgroups do not divide evenly over the XCDs (launch()'s
+  // 1-D grid): then an XCD's L2 holds the operands of more splits, and the lines come sooner (819 x
+  // 768 x 8192, 22 k-tiles: 34.3 us on 252 four-stage workgroups, 25.0 on 504 two-stage ones; 819 x
+  // 1536 x 3072, 16: 25.5, 23.4)
+  const auto uneven = [&](int64_t tiles_here) { return pl.ysplits > 1 && tiles_here * pl.ysplits % 8 != 0; };
+  if (pl.big) {
+    split(fill(kCUs));
+    return pl;
+  }
+  if (!hilo) {
+    // whole: short products of few tiles, and bias + GELU, never split, whose erf runs after the
+    // tile's MFMAs, 64 values a thread on 128 x 128 tiles (777 x 1536 x 1024 23.3 -> 11.7 us; with
+    // more than two tiles per CU and a long K the four-stage tiles: 1896 x 1304 x 5832 88 -> 68)
+    pl.small = (nkt <= 24 && t64 <= 2 * kCUs) ||
+               (epilogue == MG_EPI_BIAS_GELU && t128 <= kCUs && (t64 <= 2 * kCUs || nkt <= 24));
+    if (pl.small) {
+      split(1);
+      return pl;
+    }
+    if (may_split && t64 <= kCUs) {
+      const int64_t n = std::min<int64_t>(2 * kCUs / t64, nkt / 6);
+      // (an MN-contiguous B with rows that start inside a cache line costs its 64-column loads
+      // two lines each: 224 x 2448 x 3384 24.3 against 21.0 us; a weight gradient's two splits
+      // lose from 29 k-tiles on, four from 49: 376 x 2072 x 4033 32.3 against 28.2)
+      const int most = ak ? (bk || N % 64 == 0 ? 32 : 16) : n >= 4 ? 40 : 28;
+      const int kt = split(n);
+      if (kt <= (uneven(t64) ? 16 : most)) {
+        pl.small = true;
+        return pl;
+      }
+    }
+  }
+  if (tiles <= kCUs) {
+    const int kt = split(fill(kCUs));
+    const bool whole = pl.ysplits == 1;
+    if (may_split)  // (with 6 k-tiles or less the prologue's third stage is not made up for: 0.6 us)
+      pl.deep = kt >= 7 && kt <= (whole ? (ak && bk ? 40 : 32) : hilo ? (nkt <= 256 ? 20 : 0) : ak ? (bk ? 24 : 20) : 12) &&
+                (kt <= 12 || !uneven(tiles));
+    else  // the same loop on both sides but for the stages: a longer prologue against latency hidden
+      pl.deep = nkt >= (tiles > 128 ? 20 : tiles > 32 ? 25 : 48);
+    if (pl.deep) return pl;
+  }
+  split(fill(2 * kCUs));
   return pl;
 }
 

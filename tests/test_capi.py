@@ -200,3 +200,32 @@ def test_product_refuses_cpu_tensors():
     x = torch.zeros(1, 4, 8)
     with pytest.raises(RuntimeError, match="GPU only"):
         gate_scan(x, x)
+
+
+# (A K-contiguous, B K-contiguous, bf16 C, hi/lo, M, N, K, splits): both sides of the lines between
+# the 64 x 64, four-stage 128 x 128 and two-stage 128 x 128 tiles, each as the faster one measured
+@pytest.mark.parametrize("ak,bk,bf16,hilo,M,N,K,splits", [
+    (1, 1, 1, 0, 2048, 1024, 1536, 1),   # 64 x 64, whole: 24 k-tiles
+    (1, 1, 1, 0, 777, 1024, 3072, 2),    # 64 x 64, two workgroups per CU, 24 k-tiles each
+    (1, 1, 1, 0, 827, 1152, 8192, 8),    # 64 would be left: two-stage 128 x 128
+    (1, 1, 1, 0, 1200, 3072, 1152, 1),   # four stages, whole: 18 k-tiles
+    (1, 1, 1, 0, 237, 8192, 3072, 2),    # four stages, 24 k-tiles each
+    (1, 1, 1, 0, 777, 2048, 8192, 4),    # 64 each in four stages: two
+    (1, 1, 1, 0, 1896, 1304, 5832, 3),   # 92, whole, in four: two
+    (1, 1, 1, 0, 819, 768, 8192, 12),    # 252 four-stage workgroups are not whole splits per XCD: two
+    (1, 0, 1, 0, 2048, 1024, 6144, 4),   # an MN-contiguous B: four stages to 20 k-tiles per split
+    (1, 0, 1, 0, 988, 3072, 3072, 2),    # 48, whole
+    (1, 0, 1, 0, 224, 2448, 3384, 6),    # rows of B that start inside a cache line: no 64 x 64 above 16
+    (0, 0, 0, 0, 1440, 1200, 16376, 4),  # weight gradients: four stages to 12 k-tiles per split
+    (0, 0, 0, 0, 384, 768, 13798, 7),    # 64 x 64 with four splits or more: to 40
+    (1, 1, 0, 1, 2048, 1024, 3072, 4),   # fp32 hi/lo on 256 x 128 tiles
+    (1, 1, 0, 1, 2048, 1024, 1536, 4),   # 3.2e9 multiply-adds: 128 x 128
+    (1, 1, 0, 1, 771, 3072, 8192, 3),    # 256 x 128 tiles would fill 57% of the chip
+])
+def test_product_plans(L, ak, bk, bf16, hilo, M, N, K, splits):
+    """The split count of a product's plan, from the workspace it asks for (M x N fp32 partials per
+    split, none unsplit); the deterministic flag never splits."""
+    args = (0 if ak else 1, 0 if bk else 1, M, N, K, 0, _lib.MG_BF16 if bf16 else _lib.MG_F32)
+    want = splits * M * N * 4 if splits > 1 else 0
+    assert L.mg_gemm_workspace_bytes(*args, 4 if hilo else 0) == want
+    assert L.mg_gemm_workspace_bytes(*args, (4 if hilo else 0) | 2) == 0
