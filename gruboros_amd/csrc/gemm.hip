@@ -1666,10 +1666,8 @@ struct GroupParams {
   int splits0, splits1, splits2;
 };
 
-enum GroupOut { OUT_F32 = 0, OUT_BF16 = 1, OUT_BF16_SR = 2 };
-
-template <bool AK, bool BKM>
-__device__ __forceinline__ void group_tile(const Params& p, int L, int splits, GroupOut out, uint4* sa, uint4* sb) {
+template <bool AK, bool BKM, bool BF16_SR>
+__device__ __forceinline__ void group_tile(const Params& p, int L, int splits, uint4* sa, uint4* sb) {
   // (split, tile) pairs in split order, a contiguous range of them per XCD: an
   // XCD's workgroups share a split's k-slices in its L2
   const int T = p.tiles_m * p.tiles_n, per_xcd = (T * splits + 7) >> 3;
@@ -1689,6 +1687,7 @@ __device__ __forceinline__ void group_tile(const Params& p, int L, int splits, G
   const int row0 = m0 + (wave >> 1) * 128, col0 = n0 + (wave & 1) * 128;
   unsigned char* stage = reinterpret_cast<unsigned char*>(sa) + wave * 16384;
   const int hq = lane >> 4, rl = lane & 15, qc = lane & 31, n = col0 + 4 * qc;
+  const bool add = !BF16_SR && splits == 1 && p.accumulate;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
 #pragma unroll
@@ -1703,27 +1702,36 @@ __device__ __forceinline__ void group_tile(const Params& p, int L, int splits, G
       }
     }
     __syncthreads();
+    auto row = [&](int t) { return 2 * t + (lane >> 5); };
+    auto staged = [&](int r) { return io4<float>::load(reinterpret_cast<const float*>(stage + r * 512 + ((qc ^ r) * 16))); };
+    if (add) {
+      // C's old values: all 16 loads go out before the first store (a load after a store to the
+      // same array waits for it: 16 memory latencies instead of one); clamped, so unconditional
+      float* const cp = static_cast<float*>(p.C) + min(n, p.N - 4);
+      f4 old[16];
 #pragma unroll
-    for (int t = 0; t < 16; ++t) {
-      const int r = 2 * t + (lane >> 5);
-      const int m = row0 + 32 * i + r;
-      f4 x = io4<float>::load(reinterpret_cast<const float*>(stage + r * 512 + ((qc ^ r) * 16)));
-      if (m >= p.M || n >= p.N) continue;
-      if (splits > 1) {
-        io4<float>::store(p.part + (static_cast<int64_t>(split) * p.M + m) * p.N + n, x);
-      } else if (out == OUT_BF16) {
-        io4<bf16_t>::store(static_cast<bf16_t*>(p.C) + static_cast<int64_t>(m) * p.ldc + n, x);
-      } else if (out == OUT_BF16_SR) {
-        io4<bf16_t>::store_grad(static_cast<bf16_t*>(p.C) + static_cast<int64_t>(m) * p.ldc + n, x,
-                                static_cast<uint32_t>(static_cast<int64_t>(m) * p.N + n), 0x9e5bu);
-      } else {
-        float* cp = static_cast<float*>(p.C) + static_cast<int64_t>(m) * p.ldc + n;
-        if (p.accumulate) {
-          const f4 old = io4<float>::load(cp);
+      for (int t = 0; t < 16; ++t) old[t] = io4<float>::load(cp + static_cast<int64_t>(min(row0 + 32 * i + row(t), p.M - 1)) * p.ldc);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) x.v[e] = old.v[e] + x.v[e];
-        }
-        io4<float>::store(cp, x);
+      for (int t = 0; t < 16; ++t) {
+        const int m = row0 + 32 * i + row(t);
+        f4 x = staged(row(t));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x.v[e] = old[t].v[e] + x.v[e];
+        if (m < p.M && n < p.N) io4<float>::store(cp + static_cast<int64_t>(m) * p.ldc, x);
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < 16; ++t) {
+        const int m = row0 + 32 * i + row(t);
+        const f4 x = staged(row(t));
+        if (m >= p.M || n >= p.N) continue;
+        if (splits > 1)
+          io4<float>::store(p.part + (static_cast<int64_t>(split) * p.M + m) * p.N + n, x);
+        else if (BF16_SR)
+          io4<bf16_t>::store_grad(static_cast<bf16_t*>(p.C) + static_cast<int64_t>(m) * p.ldc + n, x,
+                                  static_cast<uint32_t>(static_cast<int64_t>(m) * p.N + n), 0x9e5bu);
+        else
+          io4<float>::store(static_cast<float*>(p.C) + static_cast<int64_t>(m) * p.ldc + n, x);
       }
     }
     __syncthreads();
@@ -1735,12 +1743,12 @@ __global__ __launch_bounds__(256) void gemm_group_kernel(GroupParams g) {
   __shared__ uint4 sb[2 * kW4Rows * 8];
   const int bx = blockIdx.x;
   if (bx < g.wg1) {
-    group_tile<true, false>(g.p0, bx, g.splits0, OUT_BF16_SR, sa, sb);
+    group_tile<true, false, true>(g.p0, bx, g.splits0, sa, sb);
   } else {
     Params p = g.p1;
     int L = bx - g.wg1, splits = g.splits1;
     if (bx >= g.wg2) p = g.p2, L = bx - g.wg2, splits = g.splits2;
-    group_tile<false, false>(p, L, splits, OUT_F32, sa, sb);
+    group_tile<false, false, false>(p, L, splits, sa, sb);
   }
 }
 
@@ -3221,12 +3229,18 @@ struct GroupPlan {
 // Splits for a group. L, the longest share of k-tiles a workgroup takes, is
 // chosen by estimated time: 1.25 us per k-tile (a 256 x 256 x 64 step), 8 us to
 // start, fill and store a workgroup, and split products' partials written and
-// read at about 7.4 TB/s plus 4 us for their reduction; all workgroups at once
-// (one per CU). The group applies while its tiles fit the CUs at one each.
+// read at about 7.4 TB/s plus 4 us for their reduction; all workgroups at once,
+// on every XCD (one per CU; 4900 rows, 1408 x 2816: 252 of them, but 33 on seven
+// of the XCDs, 152 -> 174). The group applies while its tiles fit so.
 // Measured against the products alone (us): expansion-3 minGRU block of 2048
 // rows, d1024 108.1 -> 64.5; FeedForward of 2048 rows, 1024 x 1536: 62.1 -> 41.7,
 // 1024 x 4096: 84.5 -> 58.2; expansion 2, d768, 333 rows: 34.6 -> 24.3; with
 // more tiles than CUs (8192 rows, d1024, expansion 3) 284 -> 287 to 320.
+// Where a workgroup's share is long (48 k-tiles or more) the group must keep the
+// chip busy, 40% of its multiply-adds over that time (two products: 50%), or one
+// long unsplit product holds up the rest: 838 rows, d1536, e4 (19%) 94 -> 126,
+// 1772 rows, d1408, e2 (37%) 108 -> 122, 5758 rows, d1408, e1 (47%) 111 -> 128;
+// inside the rule 1639 rows, 1536 x 3072 (46%) 88 -> 73.
 inline GroupPlan group_plan(const mg_gemm_desc* d, int count, bool deterministic) {
   GroupPlan best{};
   if (deterministic || count < 2 || count > 3) return best;
@@ -3240,7 +3254,9 @@ inline GroupPlan group_plan(const mg_gemm_desc* d, int count, bool deterministic
     if (int64_t(d[i].M) * d[i].N >= (int64_t(1) << 31) || T[i] > 4096) return best;
   }
   if (d[0].K % BK || T[0] + T[1] + (count > 2 ? T[2] : 0) > kCUs) return best;
-  double least = 1e300;
+  double least = 1e300, macs = 0;
+  int longest_share = 1;
+  for (int i = 0; i < count; ++i) macs += double(d[i].M) * d[i].N * d[i].K;
   for (int s = 1; s <= 64 && s <= longest; ++s) {
     const int L = std::max((longest + s - 1) / s, 2);
     GroupPlan pl{};
@@ -3251,15 +3267,17 @@ inline GroupPlan group_plan(const mg_gemm_desc* d, int count, bool deterministic
       const int si = (kt[i] + L - 1) / L;
       pl.kt[i] = (kt[i] + si - 1) / si;
       pl.splits[i] = (kt[i] + pl.kt[i] - 1) / pl.kt[i];
-      pl.wgs[i] = static_cast<int>((T[i] * pl.splits[i] + 7) / 8 * 8);
-      wgs += T[i] * pl.splits[i];
+      pl.wgs[i] = static_cast<int>((T[i] * pl.splits[i] + 7) / 8 * 8);  // whole eighths: an XCD's range of each
+      wgs += pl.wgs[i];
       most = std::max(most, pl.kt[i]);
       if (pl.splits[i] > 1) part += double(pl.splits[i]) * d[i].M * d[i].N * 8.0;
     }
     if (wgs > kCUs) continue;
     const double cost = 1.25 * most + 8.0 + (part > 0 ? 4.0 + part / 7.4e6 : 0.0);
-    if (cost < least) least = cost, best = pl, best.ok = true;
+    if (cost < least) least = cost, best = pl, best.ok = true, longest_share = most;
   }
+  const double share = macs / (double(kCUs) * 256 * 256 * BK * longest_share);
+  if (longest_share >= 48 && share < (count == 2 ? 0.5 : 0.4)) best.ok = false;
   return best;
 }
 

@@ -205,6 +205,12 @@ struct DW {
 std::optional<std::vector<Tensor>> group(const Tensor& dy, const Tensor& w, const std::vector<DW>& dws, int64_t stream) {
   const int64_t n = dy.size(0), o = dy.size(1), k = extent(w, o, w.size(-1), "w").size(1);
   const Mat dm = mat(dy, "dy"), wm = mat(w, "w");
+  // One weight gradient beside dX needs 512 rows and 16 tiles with it: below, the launch saved is less
+  // than the partials cost (us, apart -> together: 279 rows, 512 x 1024, 18.2 -> 21.2; 25 rows, 1024 x
+  // 2048, accumulated, 18.5 -> 19.8; 1919 rows, 256 x 512, 23.6 -> 25.8; 1194 rows, 1024 x
+  // 2048, accumulated, 49 -> 36).
+  const auto tiles = [](int64_t r, int64_t c) { return ((r + 255) / 256) * ((c + 255) / 256); };
+  if (dws.size() == 1 && (n < 512 || tiles(n, k) + tiles(dws[0].m, dws[0].k) < 16)) return std::nullopt;
   const auto span = [](int64_t rows, int64_t ld) { return (rows + 512) * ld * 2 < (int64_t(1) << 31); };
   bool ok = span(n, dm.ld) && span(o, wm.ld) && (dws.size() == 1 || dws.size() == 2);
   mg_gemm_desc d[3] = {{dm.p, wm.p, nullptr, dm.ld, wm.ld, k, int(n), int(k), int(o), 0}};

@@ -440,8 +440,9 @@ size_t mg_gemm_wgrad_pair_workspace_bytes(int M0, int N0, int M1, int N1, int K,
  * (mg_gemm_group_workspace_bytes, 16-byte aligned) and one reduction in split
  * order, so results repeat bit for bit. mg_gemm_group_fits: 1 where the
  * products share a launch (d[0].K % 64 == 0, at most one 256 x 256 tile per CU
- * in all, no MG_GEMM_DETERMINISTIC); otherwise mg_gemm_group
- * fails and the caller runs them alone. N and the weight gradients' M are
+ * in all and on every XCD, no product so long that it holds up the others, no
+ * MG_GEMM_DETERMINISTIC); otherwise mg_gemm_group fails and the caller runs them
+ * alone. N and the weight gradients' M are
  * multiples of 8, lda and ldb too, ldc of 4; pointers 16-byte aligned; each
  * operand spans less than 2 GiB. */
 typedef struct mg_gemm_desc {

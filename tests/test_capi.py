@@ -229,3 +229,29 @@ def test_product_plans(L, ak, bk, bf16, hilo, M, N, K, splits):
     want = splits * M * N * 4 if splits > 1 else 0
     assert L.mg_gemm_workspace_bytes(*args, 4 if hilo else 0) == want
     assert L.mg_gemm_workspace_bytes(*args, (4 if hilo else 0) | 2) == 0
+
+
+# (rows, output width o and input width k of dX, weight gradients, whether they share a launch)
+@pytest.mark.parametrize("n,o,k,dws,fits", [
+    (2048, 6144, 1024, [(6144, 1024), (1024, 3072)], 1),   # the expansion-3 block of a 2048-row chunk
+    (1639, 3072, 1536, [(1536, 3072), (3072, 1536)], 1),   # 46% of the chip over the longest share
+    (838, 6144, 1536, [(6144, 1536), (1536, 3072)], 0),    # 19%: dX's 96 k-tiles hold up the rest
+    (1772, 5632, 1408, [(5632, 1408), (1408, 2816)], 0),   # 37%
+    (5758, 2816, 1408, [(2816, 1408)], 0),                 # 47%, two products
+    (2541, 4096, 2048, [(4096, 2048)], 1),                 # 61%
+    (4600, 2816, 1408, [(1408, 2816), (2816, 1408)], 1),
+    (4900, 2816, 1408, [(1408, 2816), (2816, 1408)], 0),   # 252 workgroups, 33 on seven of the XCDs
+])
+def test_group_plans(L, n, o, k, dws, fits):
+    """mg_gemm_group_fits on both sides of its lines: the chip's share in use and the CUs of an XCD."""
+    class Desc(ctypes.Structure):
+        _fields_ = [("A", ctypes.c_void_p), ("B", ctypes.c_void_p), ("C", ctypes.c_void_p), ("lda", ctypes.c_int64),
+                    ("ldb", ctypes.c_int64), ("ldc", ctypes.c_int64), ("M", ctypes.c_int), ("N", ctypes.c_int),
+                    ("K", ctypes.c_int), ("accumulate", ctypes.c_int)]
+
+    d = (Desc * (1 + len(dws)))()
+    d[0] = Desc(16, 16, 16, o, k, k, n, k, o, 0)
+    for i, (m, kk) in enumerate(dws):
+        d[i + 1] = Desc(16, 16, 16, m, kk, kk, m, kk, n, 0)
+    assert L.mg_gemm_group_fits(d, len(d), 0) == fits
+    assert L.mg_gemm_group_fits(d, len(d), 2) == 0
