@@ -214,3 +214,16 @@ def test_linked_libraries_are_readable_by_every_user(tmp_path):
     with pytest.raises(RuntimeError, match="linking f.so failed"):
         build._link(["g++", "-shared", str(tmp_path / "missing.c")], str(out), False)
     assert os.listdir(out.parent) == ["f.so"]
+
+
+@pytest.mark.parametrize("dtype,rows,native", [(torch.bfloat16, 777, True), (torch.bfloat16, 3800, True),
+                                               (torch.bfloat16, 3900, False), (torch.float32, 3900, True)])
+def test_long_bf16_prompts_stay_op_by_op(dtype, rows, native):
+    """The no-grad forward's native layers take bf16 prompts up to rows * dim^2 of 4e9 (above, torch's
+    products are faster) and fp32 ones of any length; never with gradients on."""
+    from gruboros_amd.mingru.minLM import minLM
+
+    model = minLM(num_tokens=16, dim=1024, depth=1, ff_mult=1, expansion=1.0).to(dtype)
+    with torch.no_grad():
+        assert model._infer_applies(dtype, rows) == native
+    assert not model._infer_applies(dtype, rows)
