@@ -323,6 +323,35 @@ def test_hilo_product_is_fp32_accurate(M, N, K, out_dtype):
     assert bool((buf[:, N:] == 3.0).all())  # the other half of the packed buffer is untouched
 
 
+@pytest.mark.parametrize("M,N,K,splits", [(4133, 1032, 1056, 1), (4100, 1160, 2080, 1), (2047, 1024, 3072, 4),
+                                           (2047, 1016, 4128, 4), (1279, 1280, 4128, 5)])
+def test_hilo_fp32_product_on_wide_tiles(M, N, K, splits):
+    """MG_GEMM_HILO with an fp32 C on 256 x 128 tiles, whole and split along K (129 steps of 32 over 4
+    and 5 splits are uneven), at ragged rows and columns: within 2e-5 of the fp64 product of the fp32
+    operands (norm-relative; ~7e-6 from the pairs' 2^-16 and the dropped lo lo term; 3e-3 were a lo limb
+    lost), padding untouched, repeated bit for bit. They sum the limb products per 32 k, so the result
+    is not the deterministic product's, bit for bit; the workspace holds the splits' partials."""
+    from gruboros_amd import _lib
+    from gruboros_amd.gemm import KCONTIG, gemm, split_hilo
+
+    gen = torch.Generator(device=DEV).manual_seed(M + N + K)
+    a = torch.randn(M, K, device=DEV, generator=gen)
+    b = torch.randn(N, K, device=DEV, generator=gen) * 0.02
+    ap, bp = split_hilo(a), split_hilo(b)
+    want = splits * M * N * 4 if splits > 1 else 0
+    assert _lib.lib().mg_gemm_workspace_bytes(0, 0, M, N, K, 0, _lib.MG_F32, 4) == want
+    buf = torch.full((M, N + 24), 3.0, device=DEV)
+    outs = []
+    for det in (False, False, True):
+        gemm(ap, KCONTIG, bp, KCONTIG, M, N, K, buf[:, :N], hilo=True, deterministic=det)
+        outs.append(buf[:, :N].clone())
+    ref = a.double() @ b.double().t()
+    for out in outs:
+        assert _rel(out, ref) <= 2e-5
+    assert torch.equal(outs[0], outs[1]) and not torch.equal(outs[0], outs[2])
+    assert bool((buf[:, N:] == 3.0).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(37, 64, 32), (300, 392, 192), (777, 1536, 768), (2047, 1032, 1024)])
 def test_hilo_product_rounds_as_asked(M, N, K):
     """MG_GEMM_HILO with a bf16 C rounds the fp32 hi/lo sum once: to nearest, or with

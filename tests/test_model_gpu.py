@@ -891,3 +891,43 @@ def test_prompt_runs_the_hooks_of_an_idle_dropout(where):
         after = model(ids)
     assert calls == [(2, 17, 64)] * 3
     assert torch.equal(before, after) and float(hooked.abs().max()) == 0.0  # norm of zeros
+
+
+@pytest.mark.parametrize("block", ["feed forward", "minGRU"])
+def test_blocks_over_2gib_run_in_row_blocks(block):
+    """Block passes whose operands span more than mg_gemm's 2 GiB buffer range (270,336 rows of 4096
+    bf16 columns: the FeedForward's hidden layer, to_hidden_and_gate's output and to_out's input) launch
+    their products in row blocks (csrc/host/native.cpp's row_step), weight gradients adding each block
+    to the last. Halves of the batch stay below the range: outputs and input gradients are theirs, weight
+    gradients their sum. Bounds: outputs are rounded once from the same sums (1e-3 allows flipped bf16
+    roundings), gradients differ by their stochastic rounding (5e-3 of a gradient each; 2e-2 allowed),
+    where a block of rows left out or added twice (3% of them) would show as 0.17."""
+    from gruboros_amd import blocks
+
+    B, T, D, W = 66, 4096, 64, 4096
+    assert B * T * W * 2 > 1 << 31
+    gen = torch.Generator(device=DEV).manual_seed(8)
+    rnd = lambda *s, std=1.0: torch.randn(*s, device=DEV, generator=gen) * std
+    x, dx, dout = rnd(B, T, D), rnd(B, T, D, std=1e-2), rnd(B, T, D, std=1e-2)
+    if block == "minGRU":
+        params = [torch.ones(D, device=DEV), rnd(W, D, std=D ** -0.5), rnd(D, W // 2, std=W ** -0.5)]
+        run = lambda x, w: blocks.MinGRUBlock.apply(x, None, w[0], w[1], None, w[2])[:2]
+    else:
+        dout = dout.to(torch.bfloat16)
+        params = [torch.ones(D, device=DEV), rnd(W, D, std=D ** -0.5), rnd(W, std=0.1), rnd(D, W, std=W ** -0.5), rnd(D, std=0.1)]
+        run = lambda x, w: blocks.FFBlock.apply(x, None, *w)
+
+    def passes(part):
+        xs, w = x[part].clone().requires_grad_(True), [p.clone().requires_grad_(True) for p in params]
+        outs = run(xs, w)
+        torch.autograd.backward(outs, [dx[part], dout[part]])
+        return [outs[1].detach(), xs.grad], [p.grad for p in w]
+
+    rows, weights = passes(slice(0, B))
+    first, second = passes(slice(0, B // 2)), passes(slice(B // 2, B))
+    for whole, a, b, tol in zip(rows, first[0], second[0], (1e-3, 2e-2)):
+        ref = torch.cat([a, b])
+        at = 261_632 // T  # the sample in which the second row block begins
+        assert _rel(whole, ref) < tol and _rel(whole[at:at + 1], ref[at:at + 1]) < tol
+    for whole, a, b in zip(weights, first[1], second[1]):
+        assert _rel(whole, a + b) < 2e-2
