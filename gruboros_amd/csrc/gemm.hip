@@ -2879,15 +2879,21 @@ inline HiloPlan hilo_plan(int M, int N, int K, bool whole) {
 // MN-contiguous B) and two two-stage workgroups of a CU 0.92 (1.0) together, so
 // the two-stage loop wins where a workgroup has many k-tiles, the four-stage one
 // where the fixed cost of a workgroup and the partials of twice the splits
-// weigh more. The lines between them are numbers of k-tiles per workgroup,
-// taken from 505 sizes of 16 to 16376 rows, N and K 256 to 8192, each timed on
-// every plan (us, small | deep | two stages):
+// weigh more, and where one workgroup per CU must hide memory's latency alone.
+// The lines between them are numbers of k-tiles per workgroup, taken from 505
+// sizes of 16 to 16376 rows, N and K 256 to 8192, each timed on every plan with
+// its operands in the caches, and 530 with the weights in memory, as a model
+// finds them (us in the caches, small | deep | two stages):
 //   2048 x 1024 x 1536   13.9 |  -   | 22.0     24 k-tiles, whole
 //    777 x 1024 x 3072   16.3 | 19.2 | 22.8     24
 //    827 x 1152 x 8192   39.0 | 43.1 | 28.4     64
 //   1200 x 3072 x 1152     -  | 17.0 | 25.1     18, whole
 //    777 x 2048 x 8192     -  | 43.3 | 38.5     64
 //   1896 x 1304 x 5832     -  | 60.4 | 52.9     92, whole
+// Unsplit products with weights in memory take 0.63 to 0.88 of the two-stage
+// time on four stages at any K from 448 on, K-contiguous ones from 256 on (0.95
+// to 1.08 in the caches up to 20 k-tiles: 0.4 us); weight gradients, whose operands were just written, gain
+// from 17 k-tiles on (0.94 to 0.99) and lose up to 10% below.
 // `ysplits` is the split count the launch uses (gridDim.y).
 struct Plan {
   bool big, deep, small;
@@ -2946,7 +2952,7 @@ inline Plan plan(int M, int N, int K, bool ak, bool bk, int c_dtype, int epilogu
     // tile's MFMAs, 64 values a thread on 128 x 128 tiles (777 x 1536 x 1024 23.3 -> 11.7 us; with
     // more than two tiles per CU and a long K the four-stage tiles: 1896 x 1304 x 5832 88 -> 68)
     pl.small = (nkt <= 24 && t64 <= 2 * kCUs) ||
-               (epilogue == MG_EPI_BIAS_GELU && t128 <= kCUs && (t64 <= 2 * kCUs || nkt <= 24));
+               (epilogue == MG_EPI_BIAS_GELU && t128 <= kCUs && (t64 <= 2 * kCUs || nkt <= 16));
     if (pl.small) {
       split(1);
       return pl;
@@ -2955,8 +2961,8 @@ inline Plan plan(int M, int N, int K, bool ak, bool bk, int c_dtype, int epilogu
       const int64_t n = std::min<int64_t>(2 * kCUs / t64, nkt / 6);
       // (an MN-contiguous B with rows that start inside a cache line costs its 64-column loads
       // two lines each: 224 x 2448 x 3384 24.3 against 21.0 us; a weight gradient's two splits
-      // lose from 29 k-tiles on, four from 49: 376 x 2072 x 4033 32.3 against 28.2)
-      const int most = ak ? (bk || N % 64 == 0 ? 32 : 16) : n >= 4 ? 40 : 28;
+      // lose from 29 k-tiles on, four from 33: 376 x 2072 x 4033 32.3 against 28.2)
+      const int most = ak ? (bk || N % 64 == 0 ? 24 : 16) : n >= 4 ? 32 : 28;
       const int kt = split(n);
       if (kt <= (uneven(t64) ? 16 : most)) {
         pl.small = true;
@@ -2967,11 +2973,12 @@ inline Plan plan(int M, int N, int K, bool ak, bool bk, int c_dtype, int epilogu
   if (tiles <= kCUs) {
     const int kt = split(fill(kCUs));
     const bool whole = pl.ysplits == 1;
-    if (may_split)  // (with 6 k-tiles or less the prologue's third stage is not made up for: 0.6 us)
-      pl.deep = kt >= 7 && kt <= (whole ? (ak && bk ? 40 : 32) : hilo ? (nkt <= 256 ? 20 : 0) : ak ? (bk ? 24 : 20) : 12) &&
-                (kt <= 12 || !uneven(tiles));
-    else  // the same loop on both sides but for the stages: a longer prologue against latency hidden
-      pl.deep = nkt >= (tiles > 128 ? 20 : tiles > 32 ? 25 : 48);
+    if (!may_split)
+      pl.deep = nkt >= (wgrad ? 17 : bk ? 4 : 7);
+    else if (whole)  // two stages would split: the partials' pass against the longer loop
+      pl.deep = kt >= (ak && bk ? 4 : 7) && kt <= (ak && bk ? 40 : 32);
+    else
+      pl.deep = kt >= 7 && kt <= (hilo ? (nkt <= 256 ? 20 : 0) : ak ? (bk ? 24 : 16) : 12) && (kt <= 12 || !uneven(tiles));
     if (pl.deep) return pl;
   }
   split(fill(2 * kCUs));
@@ -3429,7 +3436,8 @@ extern "C" int mg_gemm(int a_layout, const void* A, int64_t lda, int b_layout, c
   p.nkt_seg = (K + gemm::BK - 1) / gemm::BK;
   if (K == 0 && accumulate) return MG_OK;
   if (hilo && epilogue == MG_EPI_NONE && !accumulate && c_dtype == MG_F32 && !deterministic) {
-    const gemm::HiloPlan hp = gemm::hilo_plan(M, N, K, !workspace);
+    gemm::HiloPlan hp = gemm::hilo_plan(M, N, K, false);
+    if (hp.splits > 1 && !workspace) hp = gemm::hilo_plan(M, N, K, true);
     if (hp.ok) {
       const size_t need = hp.splits > 1 ? static_cast<size_t>(hp.splits) * M * N * sizeof(float) : 0;
       if (need && workspace_bytes < need)
@@ -3453,8 +3461,8 @@ extern "C" int mg_gemm(int a_layout, const void* A, int64_t lda, int b_layout, c
       return MG_OK;
     }
   }
-  // Without a workspace the product runs unsplit.
-  gemm::Plan pl = gemm::plan(M, N, K, ak, bk, c_dtype, epilogue, deterministic || !workspace, hilo);
+  gemm::Plan pl = gemm::plan(M, N, K, ak, bk, c_dtype, epilogue, deterministic, hilo);
+  if (pl.ysplits > 1 && !workspace) pl = gemm::plan(M, N, K, ak, bk, c_dtype, epilogue, true, hilo);  // unsplit
   if (pl.ysplits > 1) {
     const size_t need = gemm::ws_bytes(pl, M, N);
     if (workspace_bytes < need)

@@ -213,7 +213,7 @@ def test_product_refuses_cpu_tensors():
     (1, 1, 1, 0, 777, 2048, 8192, 4),    # 64 each in four stages: two
     (1, 1, 1, 0, 1896, 1304, 5832, 3),   # 92, whole, in four: two
     (1, 1, 1, 0, 819, 768, 8192, 12),    # 252 four-stage workgroups are not whole splits per XCD: two
-    (1, 0, 1, 0, 2048, 1024, 6144, 4),   # an MN-contiguous B: four stages to 20 k-tiles per split
+    (1, 0, 1, 0, 2048, 1024, 6144, 4),   # an MN-contiguous B: four stages to 16 k-tiles per split
     (1, 0, 1, 0, 988, 3072, 3072, 2),    # 48, whole
     (1, 0, 1, 0, 224, 2448, 3384, 6),    # rows of B that start inside a cache line: no 64 x 64 above 16
     (0, 0, 0, 0, 1440, 1200, 16376, 4),  # weight gradients: four stages to 12 k-tiles per split
