@@ -47,7 +47,8 @@ extern "C" {
 /* Library version (major*10000 + minor*100 + patch): 206 = 0.2.6, the ABI
  * declared in this file (0.2.1 to 0.2.5 add entry points to 0.2.0 and change
  * none; 0.2.6 changes no signature: mg_gemm also splits small bf16 products
- * along K, see mg_gemm). */
+ * along K, see mg_gemm, and mg_gemm_f32, mg_gemm_group, mg_gemm_hilo_cols and
+ * mg_scan_fwd_pair are additions under the same number). */
 int mg_version(void);
 
 /* Message of the last failed call on this thread ("" if none). */

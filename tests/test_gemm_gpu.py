@@ -747,7 +747,7 @@ def test_split_limbs_reconstructs_fp32_exactly():
 def test_f32_linear_matches_fp64(N, K, O, bias):
     """F32Linear (the fp32 path's nn.Linear, reference mingru/minGRU.py:45,71 and minLM.py:17-23,
     :138 in fp32) against float64 for the output and the x, W and bias gradients: all three
-    products on mg_gemm over three-limb bf16 splits, fp32-accurate (within 2e-6,
+    products on mg_gemm_f32 (three bf16 limbs), fp32-accurate (within 2e-6,
     norm-relative: an fp32 product's accumulation error at these K). N = 4092 and 37 put the
     weight gradient's reduction off a multiple of 8; (4096, 512, 1024) is cfg1's
     to_hidden_and_gate."""
